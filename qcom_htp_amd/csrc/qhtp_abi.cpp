@@ -69,8 +69,8 @@ qh_status qh_qmm_run_path(const qh_qmm_prepared *prep, uint32_t m, const void *a
   if (prep->shape.exact_only) {
     if (prep->shape.wfmt == QH_WEIGHT_I16)
       return fail(QH_STATUS_UNSUPPORTED, "qh_qmm_run: int16 weights have no float requantisation; use qh_qmm_run_contract");
-    // per-group weights: the exact integer GEMM for every M (path ignored)
-    return launch_qmm_exact(prep, static_cast<int>(m), act_dev, out_dev, 0, 0, 1, s);
+    // per-group weights: the tile kernel for every M (path ignored)
+    return launch_qmm_tile(prep, static_cast<int>(m), act_dev, out_dev, 0, 0, 1, s);
   }
   const bool gemv = path == 2 || (path == 0 && m <= 16 && gemv_fits(prep, static_cast<int>(m)));
   if (gemv) return launch_qmm_gemv(prep, static_cast<int>(m), act_dev, out_dev, s);
@@ -90,7 +90,7 @@ qh_status qh_qmm_accumulate(const qh_qmm_prepared *prep, uint32_t m, const void 
   if (reinterpret_cast<uintptr_t>(act_dev) % 16)
     return fail(QH_STATUS_INVALID_ARGUMENT, "qh_qmm_accumulate: activation must be 16-byte aligned");
   if (prep->shape.exact_only)
-    return launch_qmm_exact(prep, static_cast<int>(m), act_dev, acc_dev, 1, 0, 1, static_cast<hipStream_t>(stream));
+    return launch_qmm_tile(prep, static_cast<int>(m), act_dev, acc_dev, 1, 0, 1, static_cast<hipStream_t>(stream));
   return launch_qmm_accumulate(prep, static_cast<int>(m), act_dev, acc_dev, static_cast<hipStream_t>(stream));
 }
 
@@ -122,8 +122,8 @@ qh_status qh_qmm_run_contract(const qh_qmm_prepared *prep, uint32_t m, const voi
   uint32_t param = 1;
   const qh_status st = contract_param("qh_qmm_run_contract", contract, divisor, &param);
   if (st != QH_STATUS_OK) return st;
-  return launch_qmm_exact(prep, static_cast<int>(m), act_dev, out_dev, 2, static_cast<int>(contract),
-                          static_cast<int>(param), static_cast<hipStream_t>(stream));
+  return launch_qmm_tile(prep, static_cast<int>(m), act_dev, out_dev, 2, static_cast<int>(contract),
+                         static_cast<int>(param), static_cast<hipStream_t>(stream));
 }
 
 qh_status qh_qmm_run_chain(const qh_qmm_prepared *prep, uint32_t m, uint32_t chain, const void *act_dev,
@@ -196,7 +196,7 @@ qh_status qh_qmm_release(qh_qmm_prepared *prep) {
   void *ptrs[] = {D.tiles, D.gemv_tiles, D.gemv_lpbq, D.alpha, D.beta, D.corr,
                   D.margin, D.absb, D.bias_deq, D.s32, D.mant, D.colsum, D.gemv_margin_r1,
                   D.colsum_r, D.alpha_e, D.scale_exp, D.margin_exact, D.resid, D.bias_q,
-                  D.corr_int, D.mult, D.corr_rq, D.s32g, D.margin_lo, D.lpbq_nk, D.gemv_rec};
+                  D.corr_int, D.mult, D.thr, D.s32g, D.margin_lo, D.lpbq_nk, D.gemv_rec};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   (void)hipSetDevice(cur);

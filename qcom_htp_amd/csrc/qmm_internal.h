@@ -106,10 +106,13 @@ struct QmmDevice {
                     // scattered 16-byte pieces
   int32_t *bias_q;  // [Np] the descriptor's int32 bias (integer contracts)
   int64_t *corr_int; // [Np] activation-shift term of the exact integer dot product sum (a - zp) w_int
-  // Per-group weights (exact integer GEMM): multipliers of the code and residue planes per
-  // (plane, group, channel) [2][G][Np], the shift term of that sum, and the float32 group scales
-  int64_t *mult;
-  int64_t *corr_rq;
+  // Per-group weights (qmm_tile.hip): the group scales as int32 multiples of one unit per channel
+  // (16-bit acts: a second plane for 256 times the high byte's residue sum) [planes][G][Np], and per
+  // channel the largest |t - rint(t)| that certifies the rounding; alpha_e is output LSB per unit and
+  // beta includes the activation shift's term.  The float32 group scales serve the float64
+  // recomputation.
+  int32_t *mult;
+  double *thr;
   float *s32g;      // [N][G]
 };
 
@@ -125,9 +128,9 @@ struct QmmShape {
   int act_zp, out_zp;
   double act_scale, out_scale;
   int epi_clamp;      // GEMM epilogue must clamp t before rounding (|t| < 2^30 not proven)
-  // Exact integer GEMM (qmm_exact.hip): weight planes per 32 channels in the tile layout (1, or 2
-  // for 16-bit acts and the exact-only formats), the planes / multipliers / all-ones multiplier
-  // of the integer dot product, and the per-group scale groups.
+  // Weight planes per 32 channels in the tile layout (1, or 2 for 16-bit acts and the exact-only
+  // formats), the planes / multipliers / all-ones multiplier of the integer dot product, and the
+  // per-group scale groups.
   int layout_planes;
   int exact_only;     // per-group / int16 weights: no GEMM / GEMV state
   int int_planes;
@@ -136,22 +139,35 @@ struct QmmShape {
   int groups, group_shift;
 };
 
-// Arguments of the exact integer GEMM (qmm_exact.hip).
+// Arguments of the one-launch chains (qmm_exact.hip).
 struct ExactArgs {
   const uint8_t *act;
   void *out;
   const uint8_t *tiles;
   int KT, layout_planes;
-  int M, N, K, Np;
+  int M, N, K;
   int nplanes, ones;
   long long cm[2];
-  const int64_t *mult;
-  int G, gshift;
   const int64_t *corr;
-  const double *alpha_e, *beta, *margin_exact, *absb, *bias_deq;
+  int out_zp, out_qmax;
+  int contract, divisor;
+  const int32_t *bias_q;
+};
+
+// Arguments of the tile kernel (qmm_tile.hip).
+struct TileArgs {
+  const uint8_t *act;
+  void *out;
+  const uint8_t *tiles;
+  int KT, lp;  // 128-k tiles; weight planes per 32 channels of the tile layout
+  int M, N, K, Np, TM, TN;
+  const int64_t *corr;     // activation-shift term of the integer dot product
+  const int32_t *mult;     // per-group (QmmDevice)
+  const double *alpha, *beta, *thr, *bias_deq;
   const float *s32g;
+  int G, gshift;
   double sA, sO;
-  int act_zp, out_zp, out_qmax, out16;
+  int act_zp, out_zp, out_qmax, out16, vec_out;
   int contract, divisor;
   const int32_t *bias_q;
 };
@@ -184,8 +200,8 @@ bool gemv_fits(const qh_qmm_prepared *p, int m);  // the GEMV's LDS staging hold
 qh_status launch_qmm_accumulate(const qh_qmm_prepared *p, int m, const void *act, int64_t *acc,
                                 hipStream_t stream);
 // mode 0: requantised output (per-group weights), 1: int64 accumulators, 2: integer contract
-qh_status launch_qmm_exact(const qh_qmm_prepared *p, int m, const void *act, void *out, int mode, int contract,
-                           int divisor, hipStream_t stream);
+qh_status launch_qmm_tile(const qh_qmm_prepared *p, int m, const void *act, void *out, int mode, int contract,
+                          int divisor, hipStream_t stream);
 // Every step of an integer-contract chain in one launch, for K == N <= 256 (chain_fusable).
 bool chain_fusable(const qh_qmm_prepared *p);
 qh_status launch_qmm_chain(const qh_qmm_prepared *p, int m, int chain, const void *act, void *out, int contract,

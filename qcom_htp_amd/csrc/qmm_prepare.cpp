@@ -77,11 +77,12 @@ struct TileWriter {
   }
 };
 
-// Prepared state of the formats that run on the exact integer GEMM only (qmm_exact.hip):
+// Prepared state of the formats that run on the tile kernel only (qmm_tile.hip):
 //   * QH_WEIGHT_I4_GROUP: the oracle's weight fl32(q s_g) = 2^E_g (q M_g + r) (s_g = M_g 2^E_g);
 //     with E_min = min_g E_g and d_g = E_g - E_min the dot product is 2^E_min D exactly, where
 //     D = sum_g [M_g 2^d_g sum_{k in g} (a - zp) q + 2^d_g sum_{k in g} (a - zp) r].  Plane 0
-//     holds q, plane 1 holds r (|r| <= 64), with those multipliers per (group, channel).
+//     holds q, plane 1 holds r (|r| <= 64); the multipliers per (group, channel) are int32, in
+//     units of 2^(E_min + u) with the smallest u >= 0 that fits them all (rounded if u > 0).
 //   * QH_WEIGHT_I16: q16 = 256 hi + lo' + 128 (hi = q16 >> 8, lo' = (q16 & 255) - 128): planes hi
 //     (x 256) and lo' (x 1) plus 128 times the activation row sum (the all-ones plane).
 qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
@@ -119,14 +120,15 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
   sh.groups = G;
   sh.group_shift = gshift;
   const int Np = sh.Np, KT = sh.Kp / kBK;
-  const int64_t c = (a16 ? 32896 : 128) - d->act_zp;  // activation shift of the exact GEMM
+  const int64_t c = (a16 ? 32896 : 128) - d->act_zp;  // activation shift of the kernel
   const double amax = static_cast<double>(std::max(d->act_zp, (1 << d->act_bits) - 1 - d->act_zp));
 
   std::vector<uint8_t> tiles(static_cast<size_t>(sh.ncols_op) * sh.Kp, 0);
   TileWriter tw{tiles, KT};
-  std::vector<int64_t> corr_int(Np, 0), corr_rq(Np, 0), mult;
+  std::vector<int64_t> corr_int(Np, 0);
   std::vector<int32_t> biasv(Np, 0);
-  std::vector<double> alpha_e(Np, 0.0), beta(Np, 0.0), margin_exact(Np, 0.0), absb(Np, 1.0), bdeq(Np, 0.0);
+  std::vector<int32_t> mult;
+  std::vector<double> alpha_e(Np, 0.0), beta(Np, 0.0), thr(Np, 0.0), bdeq(Np, 0.0);
   std::vector<float> s32g;
   for (int n = 0; n < N; ++n) biasv[n] = d->bias_q ? d->bias_q[n] : 0;
   if (!group) {
@@ -150,10 +152,10 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
     sh.int_mult[0] = 1;
     sh.int_mult[1] = 0;
     sh.int_ones = 0;
-    mult.assign(static_cast<size_t>(2) * G * Np, 0);
+    mult.assign(static_cast<size_t>(a16 ? 2 : 1) * G * Np, 0);
     s32g.assign(static_cast<size_t>(N) * G, 1.0f);
     const double sA = d->act_scale, sO = d->out_scale;
-    std::vector<int64_t> Mg(G);
+    std::vector<int64_t> Mg(G), m0s(G), m1s(G);
     std::vector<int> Eg(G);
     std::vector<char> live(G);
     for (int n = 0; n < N; ++n) {
@@ -174,22 +176,24 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
       const int cq = (n / 32) * 64 + (n % 32);
       int64_t csq = 0;
       double sum_abs = 0.0;  // sum_k 2^d_g |q M_g + r|: bounds D and the oracle's float noise
+      double sum_r = 0.0;    // sum_k 2^d_g |r|: bounds the residue products the kernel leaves out
       double corr_d = 0.0;
       int64_t corr_acc = 0;
       for (int g = 0; g < G; ++g) {
         const int dg = live[g] ? Eg[g] - emin : 0;
         if (dg > 30) return fail(QH_STATUS_UNSUPPORTED, "channel %d: group scales span more than 2^30", n);
         const int64_t m0 = live[g] ? Mg[g] << dg : 0, m1 = live[g] ? int64_t{1} << dg : 0;
-        mult[(static_cast<size_t>(0) * G + g) * Np + n] = m0;
-        mult[(static_cast<size_t>(1) * G + g) * Np + n] = m1;
-        int64_t sq = 0, sr = 0;
+        m0s[g] = m0;
+        m1s[g] = m1;
+        int64_t sq = 0, sr = 0, aw = 0, ar = 0;  // aw = sum |W'| < 2^31 K: exact
         const float sg = s32g[static_cast<size_t>(n) * G + g];
+        const double inv_e = std::ldexp(1.0, -Eg[g]);  // a power of two: the product below is exact
         for (int k = g * gsz; k < (g + 1) * gsz; ++k) {
           const int q = d->weight_nk[static_cast<size_t>(n) * K + k];
           if (q < -127 || q > 127)
             return fail(QH_STATUS_INVALID_ARGUMENT, "weight code %d at (n=%d,k=%d) outside [-127,127]", q, n, k);
           const float wd = static_cast<float>(q) * sg;  // the oracle's float32 weight
-          const double wp = std::ldexp(static_cast<double>(wd), -Eg[g]);
+          const double wp = static_cast<double>(wd) * inv_e;
           const int64_t Wp = static_cast<int64_t>(wp);
           if (static_cast<double>(Wp) != wp) return fail(QH_STATUS_RUNTIME_ERROR, "internal: non-integer weight at n=%d", n);
           const int64_t r = Wp - static_cast<int64_t>(q) * Mg[g];
@@ -198,8 +202,11 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
           tw.put(cq + 32, k, static_cast<int>(r));
           sq += q;
           sr += r;
-          sum_abs += std::ldexp(std::fabs(static_cast<double>(Wp)), dg);
+          aw += std::llabs(Wp);
+          ar += std::llabs(r);
         }
+        sum_abs += std::ldexp(static_cast<double>(aw), dg);
+        sum_r += std::ldexp(static_cast<double>(ar), dg);
         csq += sq;
         corr_acc += m0 * sq + m1 * sr;
         corr_d += static_cast<double>(m0) * static_cast<double>(sq) + static_cast<double>(m1) * static_cast<double>(sr);
@@ -208,15 +215,42 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
       const double bound = amax * sum_abs + std::fabs(static_cast<double>(c) * corr_d);
       if (!(bound < 0x1p62))
         return fail(QH_STATUS_UNSUPPORTED, "channel %d: per-group exact sum exceeds int64 (group scales span too far)", n);
-      corr_rq[n] = c * corr_acc;
       corr_int[n] = c * csq;
       const double ae = std::ldexp(sA, emin) / sO;
-      alpha_e[n] = ae;
       bdeq[n] = d->bias_float ? static_cast<double>(d->bias_float[n]) : 0.0;
-      beta[n] = bdeq[n] / sO + d->out_zp;
-      absb[n] = 2.0 * std::fabs(beta[n]) + 2.0 * d->out_zp + 1.0;
-      // the oracle's float64 noise: K roundings of terms bounded by amax 2^E_min sum_abs / K
-      margin_exact[n] = (K + 8.0) * std::ldexp(1.0, -52) * amax * sum_abs * ae * kSafety;
+      const double shift = static_cast<double>(c * corr_acc) * ae;  // the activation shift, codes and residues
+      const double off = bdeq[n] / sO + d->out_zp;
+      beta[n] = off + shift;
+      // int32 multipliers: M_g 2^d_g (and 256 * 2^d_g for the residues) over 2^u, with every
+      // partial sum below 2^62
+      int u = 0;
+      for (int g = 0; g < G; ++g)
+        while ((m0s[g] >> u) >= (int64_t{1} << 31) - 1) ++u;
+      while (std::ldexp((a16 ? 33024.0 : 128.0) * (sum_abs + 2.0 * sum_r), -u) >= 0x1p61) ++u;
+      const double unit = std::ldexp(1.0, u), half = u > 0 ? 0.5 * unit : 0.0;  // rounding error of a multiplier
+      double rounded = 0.0;  // bound of what the rounded multipliers change, units of 2^E_min
+      for (int g = 0; g < G; ++g) {
+        mult[static_cast<size_t>(g) * Np + n] = static_cast<int32_t>(std::rint(static_cast<double>(m0s[g]) / unit));
+        if (a16) mult[(static_cast<size_t>(G) + g) * Np + n] = static_cast<int32_t>(std::rint(256.0 * static_cast<double>(m1s[g]) / unit));
+        double aq = 0.0, ar = 0.0;
+        for (int k = g * gsz; k < (g + 1) * gsz && u > 0; ++k) {
+          aq += std::abs(static_cast<int>(d->weight_nk[static_cast<size_t>(n) * K + k]));
+          ar += 127.0;
+        }
+        rounded += half * (a16 ? 33024.0 * aq + 128.0 * ar : 128.0 * aq);
+      }
+      alpha_e[n] = ae * unit;
+      // The kernel's t = alpha_e sum_g S_g mult_g + beta leaves out the residue products of the
+      // shifted activations (8 bits: |a - 128| <= 128; 16 bits: of the low byte, |lo'| <= 128), rounds
+      // the multipliers to their unit and makes a few float64 roundings; the oracle's own float64
+      // noise is K roundings of terms bounded by amax 2^E_min sum_abs / K.  rint(t) is certain while
+      // |t - rint(t)| stays below this threshold.
+      const double left_out = (128.0 * sum_r + rounded) * ae;
+      const double noise = (K + 8.0) * std::ldexp(1.0, -52) * amax * sum_abs * ae;
+      const double size = (a16 ? 33024.0 : 128.0) * (sum_abs + sum_r) * ae + std::fabs(shift) + 2.0 * std::fabs(off) +
+                          2.0 * d->out_zp + ((1 << d->out_bits) + 2.0);
+      const double own = 16.0 * std::ldexp(1.0, -52) * size + std::ldexp(1.0, -48) * (std::fabs(off) + (1 << d->out_bits));
+      thr[n] = 0.5 - (left_out + noise + own) * kSafety;
     }
   }
   auto *p = new qh_qmm_prepared();
@@ -232,12 +266,10 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
   if (st == QH_STATUS_OK) st = al.upload(&D.bias_q, biasv);
   if (st == QH_STATUS_OK) st = al.upload(&D.corr_int, corr_int);
   if (st == QH_STATUS_OK && group) st = al.upload(&D.mult, mult);
-  if (st == QH_STATUS_OK && group) st = al.upload(&D.corr_rq, corr_rq);
-  if (st == QH_STATUS_OK && group) st = al.upload(&D.s32g, s32g);
   if (st == QH_STATUS_OK && group) st = al.upload(&D.alpha_e, alpha_e);
+  if (st == QH_STATUS_OK && group) st = al.upload(&D.thr, thr);
+  if (st == QH_STATUS_OK && group) st = al.upload(&D.s32g, s32g);
   if (st == QH_STATUS_OK && group) st = al.upload(&D.beta, beta);
-  if (st == QH_STATUS_OK && group) st = al.upload(&D.margin_exact, margin_exact);
-  if (st == QH_STATUS_OK && group) st = al.upload(&D.absb, absb);
   if (st == QH_STATUS_OK && group) st = al.upload(&D.bias_deq, bdeq);
   if (st != QH_STATUS_OK) {
     al.release();

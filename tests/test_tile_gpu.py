@@ -1,0 +1,81 @@
+"""The small-tile kernel at the sizes where it can go wrong: edges of its row and column tiles, K
+tails of a 128-deep step, each number of K groups, group sizes over 64, group scales that span more
+than the int32 multipliers hold exactly, and output buffers that are not aligned to its stores.
+Bar: bit-exact."""
+
+import dataclasses
+
+import numpy as np
+import pytest
+
+from oracle import qmm as oq
+from qcom_htp_amd import cases as C
+
+pytestmark = pytest.mark.gpu
+
+# (M, K, N): one output block; row and column remainders with a K tail; 8 K groups with a tail; a
+# row past a tile at many columns; a grid of wide tiles
+SHAPES = [(1, 32, 32), (33, 160, 96), (64, 1056, 1088), (65, 2048, 352), (700, 288, 2080)]
+
+
+def unaligned(gpu, m, n, dtype):
+    """A contiguous [m, n] buffer that starts one element past an allocation."""
+    import torch
+
+    return torch.empty(m * n + 1, dtype=dtype, device=gpu)[1:].view(m, n)
+
+
+@pytest.mark.parametrize("mkn", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("bits", [(8, 8), (16, 8), (8, 16), (16, 16)], ids=lambda b: f"a{b[0]}w{b[1]}")
+def test_contracts_and_accumulators(gpu, mkn, bits):
+    import torch
+
+    from qcom_htp_amd import _lib
+    from qcom_htp_amd.qmm import QuantMatmul
+
+    (m, k, n), (ab, wb) = mkn, bits
+    rng = np.random.default_rng(m + k + n + ab)
+    x = rng.integers(0, 1 << ab, size=(m, k)).astype(np.uint16 if ab == 16 else np.uint8)
+    q = rng.integers(-32768 if wb == 16 else -127, 32768 if wb == 16 else 128, size=(n, k)).astype(np.int16)
+    bias = rng.integers(-(1 << 20), 1 << 20, size=n).astype(np.int32)
+    zp, out_zp = 3 << (ab - 3), 1 << (ab - 1)
+    op = QuantMatmul(q if wb == 16 else q.astype(np.int8), np.ones(n, np.float32), bias, act_bits=ab, out_bits=ab,
+                     act_scale=1.0, out_scale=1.0, act_zp=zp, out_zp=out_zp,
+                     weight_format=_lib.QH_WEIGHT_I16 if wb == 16 else _lib.QH_WEIGHT_I8, device=gpu)
+    act = torch.from_numpy(x).to(gpu)
+    want = oq.int_accumulator(x, q, zp)
+    np.testing.assert_array_equal(op.accumulate(act).cpu().numpy(), want)
+    spread = max(1, int(np.abs(want).max()) >> (ab - 1))
+    for name, d in (("clip_i32", 1), ("clip_i64", 1), ("div_rint", spread), ("div_rint", 2), ("floor256_div_rint", spread),
+                    ("round_div", spread)):
+        out = unaligned(gpu, m, n, op.out_dtype)
+        got = op.run_contract(act, name, d, out=out).cpu().numpy()
+        ref = oq.contract_output(want, name, d, bias, out_zp, ab)
+        assert np.array_equal(got, ref), f"{name}/{d}: {(got != ref).sum()} differ"
+    op.close()
+
+
+@pytest.mark.parametrize("span", [0, 10], ids=["near_scales", "wide_scales"])
+@pytest.mark.parametrize("mkng", [(1, 256, 32, 128), (33, 192, 96, 64), (64, 1280, 1088, 256), (65, 2048, 352, 1024),
+                                  (700, 320, 2080, 64)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("fam", C.PER_GROUP_FAMILIES)
+def test_per_group(gpu, fam, mkng, span):
+    import torch
+
+    from qcom_htp_amd.qmm import QuantMatmul
+
+    m, k, n, gsz = mkng
+    c = C.synthetic_case(fam, m, k, n, seed=m + k)
+    rng = np.random.default_rng(k + n)
+    s = rng.uniform(1e-3, 1e-2, size=(n, k // gsz)) * 2.0 ** rng.integers(-span, 1, size=(n, k // gsz))
+    scale = s.astype(np.float32)
+    deq = c.weight_q_nk.astype(np.float32) * np.repeat(scale, gsz, axis=1)
+    x = (c.activation_q.astype(np.float64) - c.family.act_zp) * c.act_scale
+    t = x @ deq.astype(np.float64).T + c.bias_float
+    out_scale = C.affine_scale_from_minmax(float(t.min()), float(t.max()), 0, c.family.out_qmax, c.family.out_zp)
+    c = dataclasses.replace(c, weight_scale=scale, weight_deq=deq, out_scale=out_scale)
+    want = np.clip(np.rint(t / out_scale + c.family.out_zp), 0, c.family.out_qmax)
+    op = QuantMatmul.from_case(c, device=gpu)
+    got = op(torch.from_numpy(c.activation_q).to(gpu), out=unaligned(gpu, m, n, op.out_dtype)).cpu().numpy()
+    op.close()
+    assert np.array_equal(got, want.astype(got.dtype)), f"{(got != want).sum()} of {got.size} differ"
