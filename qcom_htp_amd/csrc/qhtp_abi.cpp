@@ -70,10 +70,12 @@ qh_status qh_qmm_run_path(const qh_qmm_prepared *prep, uint32_t m, const void *a
     if (prep->shape.wfmt == QH_WEIGHT_I16)
       return fail(QH_STATUS_UNSUPPORTED, "qh_qmm_run: int16 weights have no float requantisation; use qh_qmm_run_contract");
     // per-group weights: the tile kernel for every M (path ignored)
-    return launch_qmm_tile(prep, static_cast<int>(m), act_dev, out_dev, 0, 0, 1, s);
+    return launch_qmm_tile(prep, static_cast<int>(m), act_dev, out_dev, kTileGroup, 0, 1, s);
   }
   const bool gemv = path == 2 || (path == 0 && m <= 16 && gemv_fits(prep, static_cast<int>(m)));
   if (gemv) return launch_qmm_gemv(prep, static_cast<int>(m), act_dev, out_dev, s);
+  if (path == 0 && tile_pays(prep, static_cast<int>(m)))
+    return launch_qmm_tile(prep, static_cast<int>(m), act_dev, out_dev, kTileRequant, 0, 1, s);
   return launch_qmm_gemm(prep, static_cast<int>(m), act_dev, out_dev, s);
 }
 
@@ -90,7 +92,7 @@ qh_status qh_qmm_accumulate(const qh_qmm_prepared *prep, uint32_t m, const void 
   if (reinterpret_cast<uintptr_t>(act_dev) % 16)
     return fail(QH_STATUS_INVALID_ARGUMENT, "qh_qmm_accumulate: activation must be 16-byte aligned");
   if (prep->shape.exact_only)
-    return launch_qmm_tile(prep, static_cast<int>(m), act_dev, acc_dev, 1, 0, 1, static_cast<hipStream_t>(stream));
+    return launch_qmm_tile(prep, static_cast<int>(m), act_dev, acc_dev, kTileAccumulate, 0, 1, static_cast<hipStream_t>(stream));
   return launch_qmm_accumulate(prep, static_cast<int>(m), act_dev, acc_dev, static_cast<hipStream_t>(stream));
 }
 
@@ -122,7 +124,7 @@ qh_status qh_qmm_run_contract(const qh_qmm_prepared *prep, uint32_t m, const voi
   uint32_t param = 1;
   const qh_status st = contract_param("qh_qmm_run_contract", contract, divisor, &param);
   if (st != QH_STATUS_OK) return st;
-  return launch_qmm_tile(prep, static_cast<int>(m), act_dev, out_dev, 2, static_cast<int>(contract),
+  return launch_qmm_tile(prep, static_cast<int>(m), act_dev, out_dev, kTileContract, static_cast<int>(contract),
                          static_cast<int>(param), static_cast<hipStream_t>(stream));
 }
 

@@ -164,6 +164,10 @@ struct TileArgs {
   const int64_t *corr;     // activation-shift term of the integer dot product
   const int32_t *mult;     // per-group (QmmDevice)
   const double *alpha, *beta, *thr, *bias_deq;
+  // per-channel requantisation (QmmDevice)
+  const double *margin, *margin_lo, *absb, *alpha_e, *margin_exact;
+  const int64_t *mant, *colsum, *colsum_r;
+  const int8_t *resid;
   const float *s32g;
   int G, gshift;
   double sA, sO;
@@ -199,7 +203,10 @@ qh_status launch_qmm_gemv_unit(const qh_qmm_prepared *p, int m, const void *act,
 bool gemv_fits(const qh_qmm_prepared *p, int m);  // the GEMV's LDS staging holds M x K
 qh_status launch_qmm_accumulate(const qh_qmm_prepared *p, int m, const void *act, int64_t *acc,
                                 hipStream_t stream);
-// mode 0: requantised output (per-group weights), 1: int64 accumulators, 2: integer contract
+// What the tile kernel makes of the sums: requantised outputs of per-group weights, int64
+// accumulators, an integer contract, or requantised outputs of per-channel / LPBQ weights.
+enum TileOutput : int { kTileGroup = 0, kTileAccumulate = 1, kTileContract = 2, kTileRequant = 3 };
+bool tile_pays(const qh_qmm_prepared *p, int m);  // per-channel / LPBQ weights: faster than the GEMM
 qh_status launch_qmm_tile(const qh_qmm_prepared *p, int m, const void *act, void *out, int mode, int contract,
                           int divisor, hipStream_t stream);
 // Every step of an integer-contract chain in one launch, for K == N <= 256 (chain_fusable).

@@ -1,6 +1,8 @@
 // Quantized matmul on small output tiles with K split over the waves of a workgroup, i8 MFMA
-// (v_mfma_i32_32x32x32_i8).  It serves the schemas whose dot product is not one int8 product
-// times one per-channel constant, and the exact integer dot products:
+// (v_mfma_i32_32x32x32_i8).  It serves the shapes whose 128 x 512 tiles (qmm_gemm.hip) would leave
+// most compute units idle, the schemas whose dot product is not one int8 product times one
+// per-channel constant, and the exact integer dot products:
+//   * per-channel and LPBQ weights, requantised, with few output tiles (launch_qmm_gemm's rule);
 //   * per-group (K64) scales (generate_qnn_matmul_python_cases.py:392-423), requantised;
 //   * the integer contracts (gen_quant_chain.py:963-996, HmxU8I4ToU8MatMulOp.cpp:210-233,
 //     HmxU16I4ToU16MatMulOp.cpp:514-568) of every prepared weight;
@@ -32,6 +34,10 @@
 // product and bound the low byte's.  An output closer to a rounding boundary than that bound and
 // the roundings is listed and recomputed as the oracle forms its dot product (float64 products of
 // fl64((a - zp) sA) and fl32(q s_g)).
+// Per-channel requantisation is the same with one group: 8-bit activations keep the code products
+// alone, 16-bit ones add the high byte's residue products (sum M S + 256 R in int64), and a listed
+// output first gets its missing residue sum exactly (a dot product over the residue plane or
+// column), then the float64 recomputation if it still lies within the oracle's own noise.
 
 #include <type_traits>
 
@@ -48,7 +54,7 @@ constexpr int kTlThreads = 512;
 constexpr int kTlWaves = kTlThreads / 64;
 constexpr int kTlStage = 64 * kBK;  // bytes of one group's activation tile: 64 operand rows x 128 k
 
-enum TileMode : int { kGroup = 0, kContract = 1, kAccumulate = 2 };
+enum TileMode : int { kGroup = 0, kContract = 1, kAccumulate = 2, kRequant = 3 };
 
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
   return __builtin_amdgcn_perm(hi, lo, sel);
@@ -81,7 +87,7 @@ __device__ __forceinline__ void store_out(const TileArgs &g, size_t idx, int v) 
     static_cast<uint8_t *>(g.out)[idx] = static_cast<uint8_t>(v);
 }
 
-// The oracle's float64 dot product for output (m, n) of a per-group weight, by one wave:
+// The oracle's float64 dot product for output (m, n), by one wave (per-channel weights: one group):
 // sum_k fl64((a_k - zp) sA) * fl32(q_k s_g), then + bias, / sO, + zp, rint, clip.
 template <bool A16>
 __device__ void emulate_one(const TileArgs &g, int m, int n, int lane) {
@@ -117,6 +123,51 @@ __device__ void emulate_one(const TileArgs &g, int m, int n, int lane) {
   }
 }
 
+// A listed output of a per-channel weight, by one wave: S is its sum from the tile (8-bit acts
+// sum (a - 128) w; 16-bit acts M sum (a - 32896) w + 256 sum hi' r).  The missing residue products
+// (8-bit: sum (a - 128) r over the residue plane; 16-bit: sum lo' r over the residue column) make
+// the dot product D exact in units of 2^E, and t = D alpha_e + beta rounds like the oracle unless it
+// lies within the oracle's own float64 noise of a boundary.
+template <bool A16>
+__device__ void complete_one(const TileArgs &g, long long S, int m, int n, int lane) {
+  const long long mant = g.mant[n], csum = g.colsum[n], csum_r = g.colsum_r[n];
+  const double alpha_e = g.alpha_e[n], beta = g.beta[n], margin = g.margin_exact[n], absb = g.absb[n];
+  int part = 0;  // |part| <= 128 * 64 * K / 64 per lane, 2^29 over the wave at K = 65536
+  for (int kc = lane; kc < g.K / 16; kc += 64) {
+    if (!A16) {
+      const uint4 a = reinterpret_cast<const uint4 *>(g.act + static_cast<size_t>(m) * g.K)[kc];
+      const uint4 r = reinterpret_cast<const uint4 *>(g.resid + static_cast<size_t>(n) * g.K)[kc];
+      part = __builtin_amdgcn_sdot4(static_cast<int>(a.x ^ 0x80808080u), static_cast<int>(r.x), part, false);
+      part = __builtin_amdgcn_sdot4(static_cast<int>(a.y ^ 0x80808080u), static_cast<int>(r.y), part, false);
+      part = __builtin_amdgcn_sdot4(static_cast<int>(a.z ^ 0x80808080u), static_cast<int>(r.z), part, false);
+      part = __builtin_amdgcn_sdot4(static_cast<int>(a.w ^ 0x80808080u), static_cast<int>(r.w), part, false);
+    } else {
+      const uint4 *ap = reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(g.act) + static_cast<size_t>(m) * g.K + kc * 16);
+      const uint4 a0 = ap[0], a1 = ap[1], r = load_w16(g, plane_col(1, n, g.lp), kc * 16);
+      part = __builtin_amdgcn_sdot4(static_cast<int>(perm(a0.y, a0.x, 0x06040200u) ^ 0x80808080u), static_cast<int>(r.x), part, false);
+      part = __builtin_amdgcn_sdot4(static_cast<int>(perm(a0.w, a0.z, 0x06040200u) ^ 0x80808080u), static_cast<int>(r.y), part, false);
+      part = __builtin_amdgcn_sdot4(static_cast<int>(perm(a1.y, a1.x, 0x06040200u) ^ 0x80808080u), static_cast<int>(r.z), part, false);
+      part = __builtin_amdgcn_sdot4(static_cast<int>(perm(a1.w, a1.z, 0x06040200u) ^ 0x80808080u), static_cast<int>(r.w), part, false);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+  // |D| < 2^63; partial terms may wrap, so the sum is formed modulo 2^64
+  const unsigned long long M64 = static_cast<unsigned long long>(mant);
+  const unsigned long long sw = M64 * static_cast<unsigned long long>(csum) + static_cast<unsigned long long>(csum_r);
+  const unsigned long long Du = (A16 ? 1ull : M64) * static_cast<unsigned long long>(S) +
+                                static_cast<unsigned long long>(static_cast<long long>(part)) +
+                                static_cast<unsigned long long>(static_cast<long long>((A16 ? 32896 : 128) - g.act_zp)) * sw;
+  const double u = static_cast<double>(static_cast<long long>(Du)) * alpha_e;
+  const double tv = u + beta, rd = rint(tv);
+  const double slack = margin + 0x1p-48 * (fabs(u) + fabs(tv) + absb);
+  if (!(fabs(tv - rd) <= 0.5 - slack)) {  // uniform: every lane holds the same sums
+    emulate_one<A16>(g, m, n, lane);
+  } else if (lane == 0) {
+    store_out(g, static_cast<size_t>(m) * g.N + n, static_cast<int>(fmin(fmax(rd, 0.0), static_cast<double>(g.out_qmax))));
+  }
+}
+
 // Compile-time shape of one instantiation.  A16: 16-bit activations.  NT: weight fragments per wave
 // and 32-k step.  PL2: those are the two planes of the same 32 channels (int16 bytes, or per-group
 // codes and residues); otherwise NT blocks of 32 channels.  KS: K groups of the workgroup.
@@ -126,20 +177,22 @@ struct TileCfg {
   static constexpr int kWavesN = kTlWaves / KS;           // waves of a group
   static constexpr int TC = kCols * kWavesN;              // channels of the tile
   static constexpr int RB = A16 ? 32 : 64;                // rows of the tile
-  static constexpr bool kW16 = PL2 && MODE != kGroup;     // int16 weights
+  static constexpr bool kRound = MODE == kGroup || MODE == kRequant;  // requantised, with a list
+  static constexpr bool kW16 = PL2 && !kRound;            // int16 weights
   // 16-bit activations: the low byte's residue products are left out (bounded instead)
-  static constexpr bool kSkipLoRes = A16 && PL2 && MODE == kGroup;
+  static constexpr bool kSkipLoRes = A16 && PL2 && kRound;
   // the sums in LDS: int64 where two digits or planes or the groups combine, else int32
   using Val = std::conditional_t<MODE == kGroup || A16 || kW16, long long, int>;
   static constexpr int kPlanes = MODE == kGroup ? (PL2 ? 2 : 1) : 0;  // group multipliers per channel
   static constexpr int kStages = 2 * KS * kTlStage;
   static constexpr int kSums = RB * TC * static_cast<int>(sizeof(Val));
-  static constexpr int kList = MODE == kGroup ? RB * TC * 2 : 0;  // every output fits: no overflow
+  static constexpr int kList = kRound ? RB * TC * 2 : 0;  // every output fits: no overflow
   static constexpr int kSmem = kStages > kSums + kList ? kStages : kSums + kList;
   static constexpr int kUnits = 512 / (64 * kWavesN);     // 16-byte activation chunks per thread per 128-k step
 };
 
-// MODE kGroup: requantised per-group output; kContract: integer contract; kAccumulate: int64.
+// MODE kGroup: requantised per-group output; kRequant: requantised per-channel output; kContract:
+// integer contract; kAccumulate: int64.
 template <bool A16, int NT, bool PL2, int MODE, int KS>
 __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs g) {
   using C = TileCfg<A16, NT, PL2, MODE, KS>;
@@ -147,8 +200,8 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
   constexpr int TC = C::TC, RB = C::RB, NW = C::kWavesN;
   __shared__ __attribute__((aligned(16))) uint8_t smem[C::kSmem];
   // per column: scale, offset and certified threshold (per-group), else the shift term and the bias
-  __shared__ double ctab[MODE == kGroup ? 3 * TC : 1];
-  __shared__ long long itab[MODE == kGroup ? 1 : 2 * TC];
+  __shared__ double ctab[C::kRound ? 3 * TC : 1];
+  __shared__ long long itab[C::kRound ? 1 : 2 * TC];
   __shared__ int rsum[C::kW16 ? 64 : 1];                // row sums of the shifted operand rows
   __shared__ int fix_cnt;
   const int t = threadIdx.x, lane = t & 63;
@@ -167,13 +220,20 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
   if (t == 0) fix_cnt = 0;
   if (C::kW16 && t < 64) rsum[t] = 0;
   // the epilogue's per-column constants are requested first, so that their latency is the loop's
-  double calpha = 0.0, cbeta = 0.0, cthr = 0.0;
-  long long ccorr = 0, cbias = 0;
+  double calpha = 0.0, cbeta = 0.0, cthr = 0.0, cmargin = 0.0, cabsb = 0.0;
+  long long ccorr = 0, cbias = 0, cmant = 0;
   if (t < TC) {
     if constexpr (MODE == kGroup) {
       calpha = g.alpha[n0 + t];
       cbeta = g.beta[n0 + t];
       cthr = g.thr[n0 + t];
+    } else if constexpr (MODE == kRequant) {
+      calpha = g.alpha[n0 + t];
+      cbeta = g.beta[n0 + t];
+      cmargin = g.margin[n0 + t] + (A16 ? g.margin_lo[n0 + t] : 0.0);
+      cabsb = g.absb[n0 + t];
+      ccorr = g.corr[n0 + t];
+      if (A16) cmant = g.mant[n0 + t];
     } else {
       ccorr = g.corr[n0 + t];
       if (MODE == kContract && g.bias_q) cbias = g.bias_q[n0 + t];
@@ -274,6 +334,7 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
 #pragma unroll
     for (int j = 0; j < (MODE == kGroup ? 16 : 1); ++j) dacc[i][j] = 0;
   int rs[2] = {0, 0};
+  const int wmant = A16 && MODE == kRequant ? static_cast<int>(g.mant[ncol]) : 0;  // 24 bits
 
   uint8_t *const stage0 = smem + kg * 2 * kTlStage;
   const int frow = lane & 31, fswz = swz8(frow);
@@ -335,6 +396,14 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
       ctab[t] = calpha;
       ctab[TC + t] = cbeta;
       ctab[2 * TC + t] = cthr;
+    } else if constexpr (MODE == kRequant) {
+      // the shift term folded into the offset; the threshold keeps the residue bound and the float
+      // slack for |t| <= qmax + 2 (16-bit acts: |sum (a - 32896) w| <= K 33024 127)
+      const double shift = static_cast<double>(ccorr) * calpha;
+      const double umax = A16 ? fabs(calpha * static_cast<double>(cmant)) * static_cast<double>(g.K) * (33024.0 * 127.0) : 0.0;
+      ctab[t] = calpha;
+      ctab[TC + t] = cbeta + shift;
+      ctab[2 * TC + t] = 0.5 - cmargin - 0x1p-48 * (cabsb + 2.0 * fabs(shift) + umax + static_cast<double>(g.out_qmax) + 2.0);
     } else {
       itab[t] = ccorr;
       itab[TC + t] = cbias;
@@ -364,6 +433,8 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
       if constexpr (MODE == kGroup) {
 #pragma unroll
         for (int i = 0; i < kGB; ++i) f(32 * i + r, c, dacc[i][j]);
+      } else if constexpr (A16 && MODE == kRequant) {
+        f(r, c, (256LL * acc[0][0][j] + acc[1][0][j]) * wmant + 256LL * acc[0][NT - 1][j]);
       } else if constexpr (A16 && C::kW16) {
         f(r, c, 65536LL * acc[0][0][j] + 256LL * (static_cast<long long>(acc[0][NT - 1][j]) + acc[1][0][j]) + acc[1][NT - 1][j]);
       } else if constexpr (A16) {
@@ -440,7 +511,7 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
       D += 128LL * (A16 ? 256LL * rsum[r] + rsum[32 + (r & 31)] : static_cast<long long>(rsum[r]));
     return D;
   };
-  if constexpr (MODE == kGroup) {
+  if constexpr (C::kRound) {
     // rint by adding 1.5 * 2^52 after a clamp to [-1, qmax + 1] (outside, both candidate roundings
     // clip to the same output)
     constexpr double kMagic = 6755399441055744.0;
@@ -499,14 +570,17 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
       default: run(std::integral_constant<int, QH_CONTRACT_U8_DRAIN>{}); break;
     }
   }
-  if constexpr (MODE == kGroup) {
+  if constexpr (C::kRound) {
     lds_barrier();
     const int cnt = fix_cnt;
     if (cnt == 0) return;
     __syncthreads();  // every provisional output is stored before any is rewritten
     for (int e = wave; e < cnt; e += kTlWaves) {
       const int v = __builtin_amdgcn_readfirstlane(static_cast<int>(list[e]));
-      emulate_one<A16>(g, m0 + v / TC, n0 + v % TC, lane);
+      if constexpr (MODE == kGroup)
+        emulate_one<A16>(g, m0 + v / TC, n0 + v % TC, lane);
+      else
+        complete_one<A16>(g, sums[v], m0 + v / TC, n0 + v % TC, lane);
     }
   }
 }
@@ -525,26 +599,38 @@ qh_status launch(TileArgs g, hipStream_t stream) {
   return QH_STATUS_OK;
 }
 
-// K groups of a workgroup.  Fewer groups make wider tiles, which read the activations less often and
-// add up fewer partial sums; more groups make more tiles and a shorter loop.  The widest tile that
-// still gives three quarters of the compute units a tile is the fastest: per-group W4A8 500 x 4096 x
-// 4096 (256 / 512 / 1024 tiles for 2 / 4 / 8 groups) 24.4 / 30.0 / 48.0 us; u8i8 contract 1024 x 2048
-// x 2048 (128 / 256 / 512) 14.4 / 11.0 / 16.7 us; per-group W4A16 100 x 1024 x 1024 (32 / 64 / 128)
-// 9.7 / 8.2 / 7.0 us.  Eight groups need eight 128-k steps to be worth their sums: int16 weights
-// 200 x 512 x 1024 take 6.1 us with 4 groups and 6.7 us with 8.
+// Tiles of a launch with ks K groups per workgroup (cols: channels per wave).
+long long tile_count(int m, int n, bool a16, int cols, int ks) {
+  const long long tm = (m + (a16 ? 31LL : 63LL)) / (a16 ? 32 : 64), tc = cols * (kTlWaves / ks);
+  return tm * ((n + tc - 1) / tc);
+}
+
+// K groups of a workgroup: as many as leave every tile a compute unit of its own.  More groups make
+// a shorter loop and less to requantise per tile, but one tile more than compute units is a second
+// round.  u8 x int4 500 x 4096 x 4096 (128 / 256 / 512 tiles for 2 / 4 / 8 groups): 24.2 / 18.8 / 27.9
+// us; 200 x 4096 x 4096 (64 / 128 / 256): 23.0 / 16.9 / 15.0; 1000 x 2048 x 4096 (256 / 512 / 1024):
+// 18.0 / 22.7 / 35.3; u16 x int4 500 x 4096 x 1024 (128 / 256 / 512): 22.8 / 20.2 / 28.1.  Eight
+// groups also need eight 128-k steps to be worth their sums: int16 weights 200 x 512 x 1024 take 6.1
+// us with 4 groups and 6.7 us with 8.
 template <bool A16, int NT, bool PL2, int MODE>
 qh_status pick_split(const TileArgs &g, hipStream_t stream) {
-  const long long tm = (g.M + (A16 ? 31 : 63)) / (A16 ? 32 : 64), enough = 3LL * device_cu_count() / 4;
-  auto tiles = [&](int ks) {
-    const int tc = (PL2 ? 32 : 32 * NT) * (kTlWaves / ks);
-    return tm * ((g.N + tc - 1) / tc);
-  };
-  if (tiles(2) >= enough) return launch<A16, NT, PL2, MODE, 2>(g, stream);
-  if (tiles(4) >= enough || g.KT < 8) return launch<A16, NT, PL2, MODE, 4>(g, stream);
-  return launch<A16, NT, PL2, MODE, 8>(g, stream);
+  const int cus = device_cu_count(), cols = PL2 ? 32 : 32 * NT;
+  if (g.KT >= 8 && tile_count(g.M, g.N, A16, cols, 8) <= cus) return launch<A16, NT, PL2, MODE, 8>(g, stream);
+  if (tile_count(g.M, g.N, A16, cols, 4) <= cus) return launch<A16, NT, PL2, MODE, 4>(g, stream);
+  return launch<A16, NT, PL2, MODE, 2>(g, stream);
 }
 
 }  // namespace
+
+// One round of the widest tiles covers the product: then its time is one tile's, below the GEMM's,
+// whose 128 x 512 tiles (64 x 256 outputs for 16-bit activations) are a quarter as many and deeper.
+// Past that the GEMM wins: u8 x int4 1000 x 2048 x 4096 (256 tiles) 18.0 against 28.3 us, 500 x 2048 x
+// 12000 (376) 31.1 against 29.7 us; u16 x int4 256 x 1024 x 4096 (256) 10.3 against 14.9 us, 500 x 1024
+// x 4096 (512) 19.3 against 16.7 us.
+bool tile_pays(const qh_qmm_prepared *p, int m) {
+  const bool a16 = p->shape.act_bits == 16;
+  return tile_count(m, p->shape.N, a16, a16 ? 32 : 64, 2) <= device_cu_count();
+}
 
 qh_status launch_qmm_tile(const qh_qmm_prepared *p, int m, const void *act, void *out, int mode, int contract,
                           int divisor, hipStream_t stream) {
@@ -581,9 +667,26 @@ qh_status launch_qmm_tile(const qh_qmm_prepared *p, int m, const void *act, void
   g.bias_deq = D.bias_deq;
   g.G = sh.groups;
   g.gshift = sh.group_shift;
+  if (mode == kTileRequant) {
+    g.alpha = D.alpha;
+    g.corr = D.corr;
+    g.margin = D.margin;
+    g.margin_lo = D.margin_lo;
+    g.absb = D.absb;
+    g.mant = D.mant;
+    g.colsum = D.colsum;
+    g.colsum_r = D.colsum_r;
+    g.alpha_e = D.alpha_e;
+    g.margin_exact = D.margin_exact;
+    g.resid = D.resid;
+    g.s32g = D.s32;  // one group
+    g.G = 1;
+    g.gshift = 30;
+  }
   const bool a16 = sh.act_bits == 16, w16 = sh.int_planes == 2;
-  if (mode == 0) return a16 ? pick_split<true, 2, true, kGroup>(g, stream) : pick_split<false, 1, false, kGroup>(g, stream);
-  if (mode == 1) {
+  if (mode == kTileRequant) return a16 ? pick_split<true, 2, true, kRequant>(g, stream) : pick_split<false, 2, false, kRequant>(g, stream);
+  if (mode == kTileGroup) return a16 ? pick_split<true, 2, true, kGroup>(g, stream) : pick_split<false, 1, false, kGroup>(g, stream);
+  if (mode == kTileAccumulate) {
     if (w16) return a16 ? pick_split<true, 2, true, kAccumulate>(g, stream) : pick_split<false, 2, true, kAccumulate>(g, stream);
     return a16 ? pick_split<true, 2, false, kAccumulate>(g, stream) : pick_split<false, 2, false, kAccumulate>(g, stream);
   }

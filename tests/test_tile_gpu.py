@@ -79,3 +79,34 @@ def test_per_group(gpu, fam, mkng, span):
     got = op(torch.from_numpy(c.activation_q).to(gpu), out=unaligned(gpu, m, n, op.out_dtype)).cpu().numpy()
     op.close()
     assert np.array_equal(got, want.astype(got.dtype)), f"{(got != want).sum()} of {got.size} differ"
+
+
+@pytest.mark.parametrize("tie", [False, True], ids=["random", "ties"])
+@pytest.mark.parametrize("mkn", [(17, 32, 32), (33, 160, 96), (65, 1184, 1088), (130, 4096, 480), (700, 288, 2080)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("fam", C.GATED_FAMILIES)
+def test_requantised_few_tiles(gpu, fam, mkn, tie):
+    """Per-channel and LPBQ weights on the automatic path; with ties, power-of-two scales put odd
+    dot products of the first rows exactly on half-integers (the float64 recomputation)."""
+    import torch
+
+    from qcom_htp_amd.qmm import QuantMatmul
+
+    m, k, n = mkn
+    c = C.synthetic_case(fam, m, k, n, seed=m + k, lpbq_block=32)
+    if tie:
+        rng = np.random.default_rng(n)
+        zp, x = c.family.act_zp, c.activation_q.copy()
+        for r in range(min(m, 40)):
+            x[r] = zp
+            pos = rng.choice(k, size=5, replace=False)
+            x[r, pos] = zp + rng.integers(-3, 4, size=5)
+        sA, s = 2.0 ** -7, 2.0 ** -8
+        c = dataclasses.replace(c, activation_q=x, act_scale=sA, weight_scale=np.full(n, s, np.float32), out_scale=2.0 * sA * s,
+                                weight_deq=c.weight_int_nk.astype(np.float32) * np.float32(s),
+                                bias_q=rng.integers(-8, 8, size=n).astype(np.int32))
+    op = QuantMatmul.from_case(c, device=gpu)
+    got = op(torch.from_numpy(c.activation_q).to(gpu), out=unaligned(gpu, m, n, op.out_dtype)).cpu().numpy()
+    op.close()
+    want = oq.expected_output_case(c)
+    assert np.array_equal(got, want), f"{(got != want).sum()} of {got.size} differ"
