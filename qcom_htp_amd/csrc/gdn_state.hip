@@ -28,6 +28,17 @@
 // fp32 accumulation; products with the exact q, k take two terms); QH_GDN_BF16 uses the hi
 // parts only.  Norms, decays and the prefix sum are fp32.
 
+//
+// Few sequences (gdn_state_cols_kernel): the chunks of a sequence follow one another, so the launch
+// lasts as long as one sequence however few there are, and what counts is a chunk's latency.  A lone
+// wave issues one vector instruction every 5 ns or so whatever it is, so that latency is the
+// instructions of one wave: the work of a chunk is spread over 16 waves and, since v_new, o and S act
+// on value columns independently, over 128 / (16 CT) workgroups of CT column tiles each.  A column
+// tile's waves share its S by key blocks; S, v_new and the state update's operand go through LDS as
+// the records that the next products read as they are.  The next chunk's rows go into LDS behind the
+// state update (q and W are free after the products, k has two buffers), and their global loads are
+// issued a whole chunk ahead.
+
 #include <type_traits>
 
 #include "bf16_split.h"
@@ -153,6 +164,67 @@ __device__ __forceinline__ Half4 bf16x4_tr(const uint16_t *p) {
   const uint2 v = __builtin_bit_cast(uint2, r);
   return exact4(v.x, v.y);
 }
+// 16 values of a W row into LDS: hi | lo words with SPLIT (a bf16 W is exact: the hi part only), else
+// bf16 (a float32 W rounded).
+template <bool SPLIT, bool WU_F32, class LW>
+__device__ __forceinline__ void stage_w(LW *dst, const uint4 (&w)[WU_F32 ? 4 : 2]) {
+  if constexpr (SPLIT) {
+    if constexpr (WU_F32) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        *reinterpret_cast<uint4 *>(dst + 4 * x) =
+            make_uint4(hilo<SPLIT>(__uint_as_float(w[x].x)), hilo<SPLIT>(__uint_as_float(w[x].y)),
+                       hilo<SPLIT>(__uint_as_float(w[x].z)), hilo<SPLIT>(__uint_as_float(w[x].w)));
+    } else {
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const uint32_t w4[4] = {w[x].x, w[x].y, w[x].z, w[x].w};
+        *reinterpret_cast<uint4 *>(dst + 8 * x) = make_uint4(w4[0] & 0xFFFFu, w4[0] >> 16, w4[1] & 0xFFFFu, w4[1] >> 16);
+        *reinterpret_cast<uint4 *>(dst + 8 * x + 4) = make_uint4(w4[2] & 0xFFFFu, w4[2] >> 16, w4[3] & 0xFFFFu, w4[3] >> 16);
+      }
+    }
+  } else {
+    if constexpr (WU_F32) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const uint4 lo = w[2 * x], hi = w[2 * x + 1];
+        *reinterpret_cast<uint4 *>(dst + 8 * x) =
+            make_uint4(pack_bf16(__uint_as_float(lo.x), __uint_as_float(lo.y)), pack_bf16(__uint_as_float(lo.z), __uint_as_float(lo.w)),
+                       pack_bf16(__uint_as_float(hi.x), __uint_as_float(hi.y)), pack_bf16(__uint_as_float(hi.z), __uint_as_float(hi.w)));
+      }
+    } else {
+      *reinterpret_cast<uint4 *>(dst) = w[0];
+      *reinterpret_cast<uint4 *>(dst + 8) = w[1];
+    }
+  }
+}
+
+// One 16 x 16 result tile of o: `at` is the element offset of the lane's column in row 4 qd of the
+// tile, tok the elements per token, qq the lane's place in its quad.
+template <bool OUT_F32>
+__device__ __forceinline__ void store_o(void *o, uint32_t at, uint32_t tok, int qq, const v4f &acc) {
+  if constexpr (OUT_F32) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) static_cast<float *>(o)[at + static_cast<uint32_t>(e) * tok] = acc[e];
+  } else {
+    // the quad's 4 rows x 4 adjacent columns, transposed with DPP quad broadcasts so that lane
+    // q of the quad stores row 4 qd + q, the quad's 4 columns, in one 8-byte store
+    const uint32_t P0 = pack_bf16(acc[0], acc[1]), P1 = pack_bf16(acc[2], acc[3]);
+    const uint32_t a0 = __builtin_amdgcn_mov_dpp(P0, 0x00, 0xF, 0xF, false);
+    const uint32_t a1 = __builtin_amdgcn_mov_dpp(P0, 0x55, 0xF, 0xF, false);
+    const uint32_t a2 = __builtin_amdgcn_mov_dpp(P0, 0xAA, 0xF, 0xF, false);
+    const uint32_t a3 = __builtin_amdgcn_mov_dpp(P0, 0xFF, 0xF, 0xF, false);
+    const uint32_t b0 = __builtin_amdgcn_mov_dpp(P1, 0x00, 0xF, 0xF, false);
+    const uint32_t b1 = __builtin_amdgcn_mov_dpp(P1, 0x55, 0xF, 0xF, false);
+    const uint32_t b2 = __builtin_amdgcn_mov_dpp(P1, 0xAA, 0xF, 0xF, false);
+    const uint32_t b3 = __builtin_amdgcn_mov_dpp(P1, 0xFF, 0xF, 0xF, false);
+    const uint32_t sel = (qq & 1) ? 0x07060302u : 0x05040100u;
+    const uint2 w = qq < 2 ? make_uint2(__builtin_amdgcn_perm(a1, a0, sel), __builtin_amdgcn_perm(a3, a2, sel))
+                           : make_uint2(__builtin_amdgcn_perm(b1, b0, sel), __builtin_amdgcn_perm(b3, b2, sel));
+    *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(o) + (at - static_cast<uint32_t>(qq) + static_cast<uint32_t>(qq) * tok)) = w;
+  }
+}
+
 template <bool SPLIT, bool WU_F32, bool OUT_F32>
 __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
   constexpr int RP = 8 * 64 / kThreads;  // row segments (16 columns of one token) per thread in L
@@ -211,37 +283,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
       for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
       ss = sum8(ss);
       if (seg == 0) invk[row] = 1.0f / sqrtf(ss + 1e-6f);
-      if constexpr (SPLIT) {
-        if constexpr (WU_F32) {
-#pragma unroll
-          for (int x = 0; x < 4; ++x)
-            *reinterpret_cast<uint4 *>(&Wl[row][16 * seg + 4 * x]) =
-                make_uint4(hilo<SPLIT>(__uint_as_float(in.w[rp][x].x)), hilo<SPLIT>(__uint_as_float(in.w[rp][x].y)),
-                           hilo<SPLIT>(__uint_as_float(in.w[rp][x].z)), hilo<SPLIT>(__uint_as_float(in.w[rp][x].w)));
-        } else {  // bf16 W is exact: the hi part only
-#pragma unroll
-          for (int x = 0; x < 2; ++x) {
-            const uint32_t w4[4] = {in.w[rp][x].x, in.w[rp][x].y, in.w[rp][x].z, in.w[rp][x].w};
-            *reinterpret_cast<uint4 *>(&Wl[row][16 * seg + 8 * x]) =
-                make_uint4(w4[0] & 0xFFFFu, w4[0] >> 16, w4[1] & 0xFFFFu, w4[1] >> 16);
-            *reinterpret_cast<uint4 *>(&Wl[row][16 * seg + 8 * x + 4]) =
-                make_uint4(w4[2] & 0xFFFFu, w4[2] >> 16, w4[3] & 0xFFFFu, w4[3] >> 16);
-          }
-        }
-      } else {  // bf16 LDS: W rounded to bf16 (a float32 W) or as given
-        if constexpr (WU_F32) {
-#pragma unroll
-          for (int x = 0; x < 2; ++x) {
-            const uint4 lo = in.w[rp][2 * x], hi = in.w[rp][2 * x + 1];
-            *reinterpret_cast<uint4 *>(&Wl[row][16 * seg + 8 * x]) =
-                make_uint4(pack_bf16(__uint_as_float(lo.x), __uint_as_float(lo.y)), pack_bf16(__uint_as_float(lo.z), __uint_as_float(lo.w)),
-                           pack_bf16(__uint_as_float(hi.x), __uint_as_float(hi.y)), pack_bf16(__uint_as_float(hi.z), __uint_as_float(hi.w)));
-          }
-        } else {
-          *reinterpret_cast<uint4 *>(&Wl[row][16 * seg]) = in.w[rp][0];
-          *reinterpret_cast<uint4 *>(&Wl[row][16 * seg + 8]) = in.w[rp][1];
-        }
-      }
+      stage_w<SPLIT, WU_F32>(&Wl[row][16 * seg], in.w[rp]);
     }
     {
       if (wave == 0) {
@@ -346,29 +388,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
         }
         acc = mma<SPLIT>(p0, p1, vB[2 * p], two ? vB[2 * p + 1] : kZero4, acc);
       }
-      if constexpr (OUT_F32) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          static_cast<float *>(a.o)[of.tile + static_cast<uint32_t>(n * kC + 16 * i + e) * of.tok] = acc[e];
-      } else {
-        // the quad's 4 rows x 4 adjacent columns, transposed with DPP quad broadcasts so that lane
-        // q of the quad stores row 4 qd + q, the quad's 4 columns, in one 8-byte store
-        const int qq = r16 & 3;
-        const uint32_t P0 = pack_bf16(acc[0], acc[1]), P1 = pack_bf16(acc[2], acc[3]);
-        const uint32_t a0 = __builtin_amdgcn_mov_dpp(P0, 0x00, 0xF, 0xF, false);
-        const uint32_t a1 = __builtin_amdgcn_mov_dpp(P0, 0x55, 0xF, 0xF, false);
-        const uint32_t a2 = __builtin_amdgcn_mov_dpp(P0, 0xAA, 0xF, 0xF, false);
-        const uint32_t a3 = __builtin_amdgcn_mov_dpp(P0, 0xFF, 0xF, 0xF, false);
-        const uint32_t b0 = __builtin_amdgcn_mov_dpp(P1, 0x00, 0xF, 0xF, false);
-        const uint32_t b1 = __builtin_amdgcn_mov_dpp(P1, 0x55, 0xF, 0xF, false);
-        const uint32_t b2 = __builtin_amdgcn_mov_dpp(P1, 0xAA, 0xF, 0xF, false);
-        const uint32_t b3 = __builtin_amdgcn_mov_dpp(P1, 0xFF, 0xF, 0xF, false);
-        const uint32_t sel = (qq & 1) ? 0x07060302u : 0x05040100u;
-        const uint2 w = qq < 2 ? make_uint2(__builtin_amdgcn_perm(a1, a0, sel), __builtin_amdgcn_perm(a3, a2, sel))
-                               : make_uint2(__builtin_amdgcn_perm(b1, b0, sel), __builtin_amdgcn_perm(b3, b2, sel));
-        const uint32_t oi = of.tile - static_cast<uint32_t>(qq) + static_cast<uint32_t>(n * kC + 16 * i + qq) * of.tok;
-        *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(a.o) + oi) = w;
-      }
+      store_o<OUT_F32>(a.o, of.tile + static_cast<uint32_t>(n * kC + 16 * i) * of.tok, of.tok, r16 & 3, acc);
     }
 
     // ---- S: S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new) -------------------------------
@@ -418,9 +438,260 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
   }
 }
 
+// One sequence's value columns 16 CT s .. 16 CT s + 16 CT - 1.  Waves: column tile wave / WPC; its WPC
+// waves own 8 / WPC key blocks of S each.  With WPC = 8 there are two waves per token tile, one for
+// W S (and v_new), the other for q S (and o); with WPC = 4 one wave does both.  The sums are formed in
+// the order of gdn_state_kernel, so the results are the same bit for bit.
+constexpr int kColThreads = 1024;
+template <bool SPLIT, bool WU_F32, bool OUT_F32, int CT>
+__global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a) {
+  constexpr int WPC = 16 / CT, KB = 8 / WPC;
+  constexpr bool kRoles = WPC == 8;        // W S and q S on different waves
+  constexpr bool kWlo = SPLIT && WU_F32;   // a bf16 W has no lo part
+  constexpr int kPr = kC + 8;              // P row stride, bf16 (36 words: 8-byte reads conflict-free)
+  using Rec = std::conditional_t<SPLIT, uint4, uint2>;  // 4 values as an operand: hi pairs (, lo pairs)
+  __shared__ __attribute__((aligned(16))) uint16_t Ql[kC][kQs];
+  __shared__ __attribute__((aligned(16))) uint16_t Kl[2][kC][kQs];
+  __shared__ __attribute__((aligned(16))) uint16_t Wh[kC][kQs], Wo[kWlo ? kC : 1][kQs];
+  __shared__ __attribute__((aligned(16))) uint16_t Ph[kC][kPr], Po[SPLIT ? kC : 1][kPr];
+  __shared__ Rec Sr[CT][8][64], Vr[CT][4][64], Dr[CT][4][64];  // S, v_new, (e^{g_last - g} / |k|) v_new
+  __shared__ float invq[2][kC], invk[2][kC], gl[2][kC], egl[2][kC], decl[2][kC], eglast[2];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int r16 = lane & 15, qd = lane >> 4;
+  // the slices of a sequence on one XCD (block indexes of one residue mod 8): they read the same q, k, W
+  constexpr int kSlices = kD / (16 * CT);
+  const int k8 = blockIdx.x >> 3, slice = k8 % kSlices, seq = (blockIdx.x & 7) + 8 * (k8 / kSlices);
+  if (seq >= a.B * a.H) return;  // uniform: before any barrier
+  const int b = seq / a.H, h = seq % a.H;
+  const int ct = wave / WPC, wc = wave % WPC;
+  const int ti = wc & 3;                           // the wave's token tile
+  const bool do_w = !kRoles || wc < 4, do_q = !kRoles || wc >= 4;
+  const int gcol = 16 * (CT * slice + ct) + r16;   // value column
+  auto put = [](Rec &r, const Half4 &x) __attribute__((always_inline)) {
+    if constexpr (SPLIT) r = make_uint4(x.h01, x.h23, x.l01, x.l23);
+    else r = make_uint2(x.h01, x.h23);
+  };
+  auto get = [](const Rec &r) __attribute__((always_inline)) {
+    if constexpr (SPLIT) return Half4{r.x, r.y, r.z, r.w};
+    else return exact4(r.x, r.y);
+  };
+
+  v4f S[KB];  // key blocks KB wc .. : rows 16 kb + 4 qd + e, column gcol
+  const size_t sbase = static_cast<size_t>(seq) * kD * kD;
+#pragma unroll
+  for (int i = 0; i < KB; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      S[i][e] = a.s_in ? a.s_in[sbase + static_cast<size_t>(16 * (KB * wc + i) + 4 * qd + e) * kD + gcol] : 0.0f;
+    put(Sr[ct][KB * wc + i][lane], split4<SPLIT>(S[i]));
+  }
+  // element offsets of chunk 0 (a chunk adds 64 H D).  Waves 0..7 stage q, 8..15 k: 16 columns of a row
+  // per thread; every wave W: 8 columns of a row per thread.
+  const uint32_t tok = static_cast<uint32_t>(a.H) * kD;
+  const uint32_t head = (static_cast<uint32_t>(b) * a.T * a.H + h) * kD;
+  const bool is_q = wave < 8;
+  const int row = (t & 511) >> 3, seg = t & 7, wrow = t >> 4, wseg = t & 15;
+  const uint16_t *const qk = is_q ? a.q : a.k;
+  const uint32_t of_row = head + row * tok + 16 * seg, of_w = head + wrow * tok + 8 * wseg;
+  const uint32_t of_tile = head + (16 * ti + 4 * qd) * tok + gcol;
+  const uint32_t of_g = static_cast<uint32_t>(b) * a.T * a.H + lane * a.H + h;
+
+  uint4 in[2], iw[WU_F32 ? 2 : 1];
+  float iu[4], igc;
+  auto load = [&](int n) __attribute__((always_inline)) {
+    const uint32_t c0 = static_cast<uint32_t>(n) * kC * tok;
+    const uint4 *p = reinterpret_cast<const uint4 *>(qk + of_row + c0);
+    in[0] = p[0];
+    in[1] = p[1];
+    const uint4 *wp = WU_F32 ? reinterpret_cast<const uint4 *>(static_cast<const float *>(a.w) + of_w + c0)
+                             : reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.w) + of_w + c0);
+    iw[0] = wp[0];
+    if (WU_F32) iw[WU_F32 ? 1 : 0] = wp[1];
+    igc = a.g[of_g + static_cast<uint32_t>(n) * kC * static_cast<uint32_t>(a.H)];
+  };
+  auto load_u = [&](int n) __attribute__((always_inline)) {
+    const uint32_t c0 = static_cast<uint32_t>(n) * kC * tok;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t ui = of_tile + c0 + static_cast<uint32_t>(e) * tok;
+      iu[e] = WU_F32 ? static_cast<const float *>(a.u)[ui] : bf16f(static_cast<const uint16_t *>(a.u)[ui]);
+    }
+  };
+  // a chunk's rows into LDS (buffer bf of the double-buffered arrays), with the norms and decays
+  auto stage = [&](int bf) __attribute__((always_inline)) {
+    uint16_t *const d = is_q ? &Ql[row][16 * seg] : &Kl[bf][row][16 * seg];
+    *reinterpret_cast<uint4 *>(d) = in[0];
+    *reinterpret_cast<uint4 *>(d + 8) = in[1];
+    float f[16];
+    unbf16x8(in[0], f);
+    unbf16x8(in[1], f + 8);
+    float ss = 0.0f;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
+    ss = sum8(ss);
+    if (seg == 0) {
+      const float r = 1.0f / sqrtf(ss + 1e-6f);
+      if (is_q)
+        invq[bf][row] = r * (1.0f / 11.313708498984761f);  // then 1/sqrt(128)
+      else
+        invk[bf][row] = r;
+    }
+    if constexpr (WU_F32) {
+      const Half4 x = split4<SPLIT>(__uint_as_float(iw[0].x), __uint_as_float(iw[0].y), __uint_as_float(iw[0].z), __uint_as_float(iw[0].w));
+      const uint4 w1 = iw[WU_F32 ? 1 : 0];
+      const Half4 y = split4<SPLIT>(__uint_as_float(w1.x), __uint_as_float(w1.y), __uint_as_float(w1.z), __uint_as_float(w1.w));
+      *reinterpret_cast<uint4 *>(&Wh[wrow][8 * wseg]) = make_uint4(x.h01, x.h23, y.h01, y.h23);
+      if constexpr (kWlo) *reinterpret_cast<uint4 *>(&Wo[wrow][8 * wseg]) = make_uint4(x.l01, x.l23, y.l01, y.l23);
+    } else {
+      *reinterpret_cast<uint4 *>(&Wh[wrow][8 * wseg]) = iw[0];
+    }
+    if (wave == 0) {  // (its token tile has no o to form)
+      const float g = scan64(igc);
+      const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), 63));
+      gl[bf][lane] = g;
+      egl[bf][lane] = expf(g);
+      decl[bf][lane] = expf(glast - g);
+      if (lane == 0) eglast[bf] = expf(glast);
+    }
+  };
+  load(0);
+  load_u(0);
+  stage(0);
+  load(min(1, a.nchunks - 1));
+  lds_barrier();
+
+  auto chunk = [&](const int n) __attribute__((always_inline)) {
+    const int bf = n & 1;
+    // ---- products: W S and q^ S of the wave's token tile, v_new; P tiles -------------------------
+    Half4 sB[8];
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb) sB[kb] = get(Sr[ct][kb][lane]);
+    v4f oacc = {0.f, 0.f, 0.f, 0.f};
+    if (do_w) {  // wave-uniform
+      v4f ws = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int c = 32 * p + 4 * qd;
+        Half4 w0 = bf16x4(&Wh[16 * ti + r16][c]), w1 = bf16x4(&Wh[16 * ti + r16][c + 16]);
+        if constexpr (kWlo) {
+          const Half4 l0 = bf16x4(&Wo[16 * ti + r16][c]), l1 = bf16x4(&Wo[16 * ti + r16][c + 16]);
+          w0.l01 = l0.h01; w0.l23 = l0.h23; w1.l01 = l1.h01; w1.l23 = l1.h23;
+        }
+        ws = WU_F32 ? mma<SPLIT>(w0, w1, sB[2 * p], sB[2 * p + 1], ws) : mma_exact_a<SPLIT>(w0, w1, sB[2 * p], sB[2 * p + 1], ws);
+      }
+      v4f vn, d;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int rw = 16 * ti + 4 * qd + e;
+        vn[e] = iu[e] - ws[e];
+        d[e] = vn[e] * (decl[bf][rw] * invk[bf][rw]);
+      }
+      put(Vr[ct][ti][lane], split4<SPLIT>(vn));
+      put(Dr[ct][ti][lane], split4<SPLIT>(d));
+    }
+    if (do_q) {
+      v4f qs = {0.f, 0.f, 0.f, 0.f};
+      const uint16_t *qrow = Ql[16 * ti + r16];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int c = 32 * p + 4 * qd;
+        qs = mma_exact_a<SPLIT>(bf16x4(qrow + c), bf16x4(qrow + c + 16), sB[2 * p], sB[2 * p + 1], qs);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int rw = 16 * ti + 4 * qd + e;
+        oacc[e] = qs[e] * (invq[bf][rw] * egl[bf][rw]);
+      }
+    }
+    load_u(min(n + 1, a.nchunks - 1));
+    if (15 - wave < 10) {  // wave-uniform: one P tile on each of 10 waves
+      int pi, pj;
+      p_tile(15 - wave, pi, pj);
+      v4f acc = {0.f, 0.f, 0.f, 0.f};
+      const uint16_t *qrow = Ql[16 * pi + r16];
+      const uint16_t *krow = Kl[bf][16 * pj + r16];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int c = 32 * p + 4 * qd;
+        acc = mma<false>(bf16x4(qrow + c), bf16x4(qrow + c + 16), bf16x4(krow + c), bf16x4(krow + c + 16), acc);
+      }
+      const int col = 16 * pj + r16;
+      const float kf = invk[bf][col];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int rw = 16 * pi + 4 * qd + e;
+        const float pv = col <= rw ? acc[e] * (invq[bf][rw] * kf) * expf(gl[bf][rw] - gl[bf][col]) : 0.0f;
+        const uint32_t w = hilo<SPLIT>(pv);
+        Ph[rw][col] = static_cast<uint16_t>(w);
+        if constexpr (SPLIT) Po[rw][col] = static_cast<uint16_t>(w >> 16);
+      }
+    }
+    lds_barrier();
+
+    // ---- S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new), the wave's key blocks --------------
+    const float el = eglast[bf];
+    const int te = r16 >> 2, ka = r16 & 3;
+#pragma unroll
+    for (int i = 0; i < KB; ++i) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[i][e] *= el;
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int c = 32 * p + 4 * qd;
+      const Half4 d0 = get(Dr[ct][2 * p][lane]), d1 = get(Dr[ct][2 * p + 1][lane]);
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        const int kc = 16 * (KB * wc + i) + 4 * ka;
+        S[i] = mma_exact_a<SPLIT>(bf16x4_tr(&Kl[bf][c + te][kc]), bf16x4_tr(&Kl[bf][c + 16 + te][kc]), d0, d1, S[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < KB; ++i) put(Sr[ct][KB * wc + i][lane], split4<SPLIT>(S[i]));
+    // ---- o = e^g q^ S + P v_new ------------------------------------------------------------------
+    if (do_q) {
+      v4f acc = oacc;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        if (p > ti / 2) continue;  // wave-uniform
+        const bool two = 2 * p + 1 <= ti;
+        const int c = 32 * p + 4 * qd;
+        Half4 p0 = bf16x4(&Ph[16 * ti + r16][c]), p1 = kZero4;
+        if (two) p1 = bf16x4(&Ph[16 * ti + r16][c + 16]);
+        if constexpr (SPLIT) {
+          const Half4 l0 = bf16x4(&Po[16 * ti + r16][c]);
+          p0.l01 = l0.h01; p0.l23 = l0.h23;
+          if (two) {
+            const Half4 l1 = bf16x4(&Po[16 * ti + r16][c + 16]);
+            p1.l01 = l1.h01; p1.l23 = l1.h23;
+          }
+        }
+        acc = mma<SPLIT>(p0, p1, get(Vr[ct][2 * p][lane]), two ? get(Vr[ct][2 * p + 1][lane]) : kZero4, acc);
+      }
+      store_o<OUT_F32>(a.o, of_tile + static_cast<uint32_t>(n * kC) * tok, tok, r16 & 3, acc);
+    }
+    // ---- the next chunk's rows (the last chunk stages itself again, unused) -------------------------
+    stage(bf ^ 1);
+    load(min(n + 2, a.nchunks - 1));
+    lds_barrier();
+  };
+  for (int n = 0; n < a.nchunks; ++n) chunk(n);
+
+#pragma unroll
+  for (int i = 0; i < KB; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a.s_out[sbase + static_cast<size_t>(16 * (KB * wc + i) + 4 * qd + e) * kD + gcol] = S[i][e];
+  }
+}
+
 template <bool SPLIT, bool WU_F32, bool OUT_F32>
 qh_status launch3(const StateArgs &a, hipStream_t stream) {
-  hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32>), dim3(a.B * a.H), dim3(kThreads), 0, stream, a);
+  const int seqs = a.B * a.H, cus = device_cu_count(), per8 = (seqs + 7) / 8 * 8;
+  if (per8 * 4 <= cus)
+    hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, 2>), dim3(per8 * 4), dim3(kColThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32>), dim3(seqs), dim3(kThreads), 0, stream, a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return hip_fail(err, "gdn_state_kernel launch");
   return QH_STATUS_OK;

@@ -287,3 +287,28 @@ def test_prefill_on_a_side_stream_matches_current_stream(gpu):
     _ = torch.empty((1 << 20,), device=gpu).fill_(1.0)  # reuse pressure on the current stream
     torch.cuda.synchronize()
     assert torch.equal(o0, o1) and torch.equal(s0, s1)
+
+
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("wu", ["f32", "bf16"], ids=["wu_f32", "wu_bf16"])
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp32", "bf16"])
+def test_few_sequences_equal_many(gpu, precision, wu, out):
+    """The column-sliced kernels of few sequences (8, 4 and 2 workgroups per sequence) form every sum
+    in the order of the one-workgroup kernel: the same sequences give the same bits alone, in groups
+    and in a launch of all of them."""
+    import torch
+
+    from qcom_htp_amd.gdn import gdn_chunk_state, gdn_chunk_uw
+
+    B, T, H = 1, 192, 160
+    qb, kb, vb, beta, gc = seq_inputs(B, T, H, seed=77)
+    q, k, v, bt, g = (to_dev(x, gpu) for x in (qb, kb, vb, beta, gc))
+    s0 = torch.randn((B, H, 128, 128), generator=torch.Generator(device=gpu).manual_seed(3), device=gpu)
+    w, u = gdn_chunk_uw(k, v, g, bt, 64, decay_w=True, out_dtype=torch.float32 if wu == "f32" else torch.bfloat16)
+    run = lambda sl: gdn_chunk_state(*(x[:, :, sl].contiguous() for x in (q, k, g, w, u)), s0[:, sl].contiguous(), precision,
+                                     torch.float32 if out == "f32" else torch.bfloat16)
+    o_all, s_all = run(slice(0, H))
+    for lo, n in ((0, 1), (1, 9), (10, 33), (43, 64), (90, 65)):
+        o, s = run(slice(lo, lo + n))
+        assert torch.equal(o, o_all[:, :, lo:lo + n]), f"{n} sequences: o differs"
+        assert torch.equal(s, s_all[:, lo:lo + n]), f"{n} sequences: S differs"
