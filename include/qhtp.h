@@ -294,12 +294,15 @@ qh_status qh_gdn_solve_u16(const uint16_t *A_dev, uint16_t *T_dev, uint32_t head
  * k_dev, v_dev: bf16 bit patterns [batch][tokens][heads][head_dim]; g_dev (gc) and beta_dev:
  * float32 [batch][tokens][heads]; w_dev, u_dev: [batch][tokens][heads][head_dim], bf16 bit
  * patterns, or float32 with QH_GDN_OUT_F32.  head_dim == 128, chunk in {64, 128, 256},
- * tokens % chunk == 0.  bf16 MFMA with fp32 accumulation (tolerance: the bf16 bound, 1.05e-2
+ * tokens % chunk == 0 unless QH_GDN_RAGGED.  bf16 MFMA with fp32 accumulation (tolerance: the bf16 bound, 1.05e-2
  * relative Frobenius against float64).  Buffers must be 16-byte aligned. */
 enum {
   QH_GDN_W_DECAY = 1u, /* W = T (beta * K^ * e^g) (the reference kernel's form)           */
   QH_GDN_OUT_F32 = 2u, /* W and U (qh_gdn_chunk_state: o) as float32 instead of bf16      */
   QH_GDN_WU_F32 = 4u,  /* qh_gdn_chunk_state: w_dev and u_dev hold float32, not bf16      */
+  QH_GDN_RAGGED = 8u,  /* chunk 64: tokens need not be a multiple of it; the last chunk's  */
+                       /* missing tokens count as zeros (q, k, v, beta, gc) and are not    */
+                       /* read or written                                                  */
 };
 qh_status qh_gdn_chunk_uw(const uint16_t *k_dev, const uint16_t *v_dev, const float *g_dev, const float *beta_dev,
                           void *w_dev, void *u_dev, uint32_t batch, uint32_t tokens, uint32_t heads,
@@ -327,8 +330,8 @@ qh_status qh_gdn_chunk_uw_ex(const uint16_t *k_dev, const uint16_t *v_dev, const
  * [batch][tokens][heads]; w_dev, u_dev: [batch][tokens][heads][128] bf16 bit patterns, or float32
  * with QH_GDN_WU_F32; o_dev: the same layout, bf16, or float32 with QH_GDN_OUT_F32;
  * s_in_dev, s_out_dev: float32 [batch][heads][128][128] (s_out_dev must not alias s_in_dev).
- * head_dim == 128, chunk == 64, tokens % 64 == 0 (zero-pad: zero q, k, v, beta and gc tokens
- * leave o and S unchanged).  precision: QH_GDN_FP32 (bf16 hi/lo split products, fp32
+ * head_dim == 128, chunk == 64, tokens % 64 == 0 unless QH_GDN_RAGGED (zero q, k, v, beta and gc
+ * tokens leave o and S unchanged).  precision: QH_GDN_FP32 (bf16 hi/lo split products, fp32
  * accumulation) or QH_GDN_BF16.  Buffers must be 16-byte aligned. */
 qh_status qh_gdn_chunk_state(const uint16_t *q_dev, const uint16_t *k_dev, const float *g_dev, const void *w_dev,
                              const void *u_dev, const float *s_in_dev, float *s_out_dev, void *o_dev, uint32_t batch,

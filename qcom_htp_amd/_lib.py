@@ -58,6 +58,7 @@ QH_GDN_OP_MODEL = 2
 QH_GDN_W_DECAY = 1
 QH_GDN_OUT_F32 = 2
 QH_GDN_WU_F32 = 4
+QH_GDN_RAGGED = 8
 
 # Every symbol include/qhtp.h declares (checked by the CPU test-suite).
 EXPORTED = (

@@ -99,7 +99,10 @@ __device__ __forceinline__ size_t tok_index(const ChunkArgs &a, int b, int tok, 
 template <int NB>
 constexpr int chunk_threads() { return NB >= 8 ? 512 : 256; }
 
-template <int NB, bool OUT_F32>
+// RAGGED: T need not be a multiple of C.  Rows past T repeat row T - 1 with beta = gc = 0, so their
+// rows of A and their scaled right-hand sides are zero and they touch no row before them (A and T are
+// lower triangular); they are not stored.
+template <int NB, bool OUT_F32, bool RAGGED>
 __device__ __forceinline__ void chunk_items(const ChunkArgs &a, const int nitems, uint8_t *smat, uint16_t *ablk,
                                             float *adiag, float *gs, float *bs, float *rn, float *wsc, float *wsum) {
   constexpr int C = NB * 16;
@@ -153,14 +156,17 @@ __device__ __forceinline__ void chunk_items(const ChunkArgs &a, const int nitems
 #pragma unroll
     for (int p = 0; p < kRowPasses; ++p) {
       const int row = p * (kChunkThreads / 8) + (t >> 3), part = t & 7;
-      const uint4 *src = reinterpret_cast<const uint4 *>(a.k + tok_index(a, it.b, it.c * C + row, it.h) * kD + part * 16);
+      const int tok = RAGGED ? min(it.c * C + row, a.T - 1) : it.c * C + row;
+      const uint4 *src = reinterpret_cast<const uint4 *>(a.k + tok_index(a, it.b, tok, it.h) * kD + part * 16);
       kr[p][0] = src[0];
       kr[p][1] = src[1];
     }
     {  // every lane loads (rows clamped), so that the count of outstanding loads is uniform
-      const size_t ix = tok_index(a, it.b, it.c * C + (t < C ? t : C - 1), it.h);
+      const int tok = it.c * C + (t < C ? t : C - 1);
+      const size_t ix = tok_index(a, it.b, RAGGED ? min(tok, a.T - 1) : tok, it.h);
       gpre = a.g[ix];
       bpre = a.beta[ix];
+      if (RAGGED && tok >= a.T) gpre = bpre = 0.0f;
     }
   };
 
@@ -239,14 +245,20 @@ __device__ __forceinline__ void chunk_items(const ChunkArgs &a, const int nitems
     // does not precompute (and keep live) the offsets of every row.
     uint32_t ld_off = rm_base;
     v4u rring[NB][kWords];
-    auto rhs_load = [&](v4u (&r)[kWords]) __attribute__((always_inline)) {
+    const int last = a.T - 1 - tok0;  // RAGGED: the last row of the chunk that exists
+    auto rhs_load = [&](v4u (&r)[kWords], int I) __attribute__((always_inline)) {
+      uint32_t off = ld_off;
+      if (RAGGED) {  // (rm_base is the lane's row lane / 4)
+        const int row = 16 * I + (lane >> 2);
+        off = rm_base + static_cast<uint32_t>(min(row, last) - (lane >> 2)) * tsb;
+      }
 #pragma unroll
-      for (int w = 0; w < kWords; ++w) r[w] = *(gptr<const v4u>)(rsrc + (ld_off + 16 * w));
+      for (int w = 0; w < kWords; ++w) r[w] = *(gptr<const v4u>)(rsrc + (off + 16 * w));
       ld_off += 16 * tsb;
       asm volatile("" : "+v"(ld_off));
     };
 #pragma unroll
-    for (int I = 0; I < kEarly; ++I) rhs_load(rring[I]);
+    for (int I = 0; I < kEarly; ++I) rhs_load(rring[I], I);
 
     // ---- 2. A = -beta_i (K^ K^T)_ij e^{g_i - g_j}, lower blocks -----------------------------
     // Wave w < NB/2 takes the block rows I0 = w and I1 = NB-1-w (NB+1 blocks, balanced): the
@@ -313,7 +325,7 @@ __device__ __forceinline__ void chunk_items(const ChunkArgs &a, const int nitems
     lds_barrier();
 
 #pragma unroll
-    for (int J = kEarly; J < NB; ++J) rhs_load(rring[J]);  // the A-build's registers are free now
+    for (int J = kEarly; J < NB; ++J) rhs_load(rring[J], J);  // the A-build's registers are free now
     it += gridDim.x;
     const Item nxt = item_of(it);
     if (kKeyRow == 0) prefetch(nxt);
@@ -444,6 +456,7 @@ __device__ __forceinline__ void chunk_items(const ChunkArgs &a, const int nitems
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           const uint32_t o = st_off + s * tstride;
+          if (RAGGED && 16 * I + 4 * q + s > last) continue;
           if constexpr (kTiles == 2)
             *(gptr<v2f>)(of + o) = v2f{xt[0][s], xt[1][s]};
           else
@@ -465,9 +478,11 @@ __device__ __forceinline__ void chunk_items(const ChunkArgs &a, const int nitems
           else
             *reinterpret_cast<uint2 *>(stg_mf + s * kStageRow) = make_uint2(wv[0], wv[1]);
         }
+        if (!RAGGED || 16 * I + (lane >> 2) <= last) {
 #pragma unroll
-        for (int w = 0; w < kWords; ++w)
-          *(gptr<v4u>)(oh + (st_off + 16 * w)) = *reinterpret_cast<const v4u *>(stg_rm + 16 * w);
+          for (int w = 0; w < kWords; ++w)
+            *(gptr<v4u>)(oh + (st_off + 16 * w)) = *reinterpret_cast<const v4u *>(stg_rm + 16 * w);
+        }
         st_off += 16 * tsb;
       }
       asm volatile("" : "+v"(st_off));
@@ -478,7 +493,7 @@ __device__ __forceinline__ void chunk_items(const ChunkArgs &a, const int nitems
   }
 }
 
-template <int NB, bool OUT_F32>
+template <int NB, bool OUT_F32, bool RAGGED>
 __global__ __launch_bounds__(chunk_threads<NB>(), 1) void gdn_chunk_kernel(const ChunkArgs a, const int nitems) {
   constexpr int C = NB * 16;
   constexpr int kLowBlocks = NB * (NB - 1) / 2;
@@ -486,10 +501,10 @@ __global__ __launch_bounds__(chunk_threads<NB>(), 1) void gdn_chunk_kernel(const
   __shared__ __attribute__((aligned(16))) uint16_t ablk[(kLowBlocks > 0 ? kLowBlocks : 1) * 256];  // A_IJ, I > J
   __shared__ __attribute__((aligned(16))) float adiag[NB * kDiagStride];     // A_II, then T_II
   __shared__ float gs[C], bsw[2 * C], rn[C], wsum[8];  // bsw: beta, then W's row scales
-  chunk_items<NB, OUT_F32>(a, nitems, smat, ablk, adiag, gs, bsw, rn, bsw + C, wsum);
+  chunk_items<NB, OUT_F32, RAGGED>(a, nitems, smat, ablk, adiag, gs, bsw, rn, bsw + C, wsum);
 }
 
-template <int NB, bool OUT_F32>
+template <int NB, bool OUT_F32, bool RAGGED>
 qh_status launch_nb(const ChunkArgs &a, int max_wg, hipStream_t stream) {
   const long long items = static_cast<long long>(a.B) * a.nchunks * a.H;  // (batch, chunk, head)
   if (items > 0x7FFFFFFFLL) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_uw: too many chunks");
@@ -503,7 +518,7 @@ qh_status launch_nb(const ChunkArgs &a, int max_wg, hipStream_t stream) {
   int grid_slots = dev >= 0 && dev < kMaxDevices ? slots[dev].load(std::memory_order_relaxed) : 0;
   if (grid_slots == 0) {
     int per_cu = 0, cus = 0;
-    err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gdn_chunk_kernel<NB, OUT_F32>, chunk_threads<NB>(), 0);
+    err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gdn_chunk_kernel<NB, OUT_F32, RAGGED>, chunk_threads<NB>(), 0);
     if (err != hipSuccess) return hip_fail(err, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
     err = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (err != hipSuccess) return hip_fail(err, "hipDeviceGetAttribute");
@@ -512,7 +527,7 @@ qh_status launch_nb(const ChunkArgs &a, int max_wg, hipStream_t stream) {
   }
   if (max_wg > 0 && max_wg < grid_slots) grid_slots = max_wg;  // caller's cap on the persistent grid
   const long long grid = grid_slots < items ? grid_slots : items;
-  hipLaunchKernelGGL((gdn_chunk_kernel<NB, OUT_F32>), dim3(static_cast<unsigned>(grid)), dim3(chunk_threads<NB>()), 0,
+  hipLaunchKernelGGL((gdn_chunk_kernel<NB, OUT_F32, RAGGED>), dim3(static_cast<unsigned>(grid)), dim3(chunk_threads<NB>()), 0,
                      stream, a, static_cast<int>(items));
   err = hipGetLastError();
   if (err != hipSuccess) return hip_fail(err, "gdn_chunk_kernel launch");
@@ -521,7 +536,10 @@ qh_status launch_nb(const ChunkArgs &a, int max_wg, hipStream_t stream) {
 
 template <int NB>
 qh_status launch_nb(const ChunkArgs &a, int max_wg, hipStream_t stream) {
-  return a.out_f32 ? launch_nb<NB, true>(a, max_wg, stream) : launch_nb<NB, false>(a, max_wg, stream);
+  if constexpr (NB == 4) {  // (the boundary takes ragged lengths for C = 64 only)
+    if (a.T % a.C) return a.out_f32 ? launch_nb<NB, true, true>(a, max_wg, stream) : launch_nb<NB, false, true>(a, max_wg, stream);
+  }
+  return a.out_f32 ? launch_nb<NB, true, false>(a, max_wg, stream) : launch_nb<NB, false, false>(a, max_wg, stream);
 }
 
 }  // namespace
@@ -539,7 +557,7 @@ qh_status launch_gdn_chunk_uw(const uint16_t *k, const uint16_t *v, const float 
   a.T = T;
   a.H = H;
   a.C = C;
-  a.nchunks = T / C;
+  a.nchunks = (T + C - 1) / C;
   a.decay_w = (flags & QH_GDN_W_DECAY) != 0;
   a.out_f32 = (flags & QH_GDN_OUT_F32) != 0;
   switch (C) {

@@ -98,12 +98,21 @@ __device__ __forceinline__ Offsets offsets(const StateArgs &a, int b, int h, int
           static_cast<uint32_t>(b) * a.T * a.H + lane * a.H + h, tok};
 }
 
-template <bool WU_F32, int RP>
-__device__ __forceinline__ void load_chunk(const StateArgs &a, const Offsets &of, int n, ChunkIn<WU_F32, RP> &in) {
+// RAGGED: T need not be a multiple of the chunk.  Rows past T repeat row T - 1 with gc = 0 and a zero
+// decay factor in the state update; P is lower triangular, so they touch no row before them, and
+// they are not stored.
+// Rows by which the row `row` of chunk n is moved back to exist (0 unless RAGGED).
+template <bool RAGGED>
+__device__ __forceinline__ uint32_t past_end(const StateArgs &a, int n, int row) {
+  return RAGGED ? static_cast<uint32_t>(max(n * kC + row - (a.T - 1), 0)) : 0u;
+}
+
+template <bool WU_F32, int RP, bool RAGGED>
+__device__ __forceinline__ void load_chunk(const StateArgs &a, const Offsets &of, int n, int row, int lane, ChunkIn<WU_F32, RP> &in) {
   const uint32_t c0 = static_cast<uint32_t>(n) * kC * of.tok;
 #pragma unroll
   for (int r = 0; r < RP; ++r) {
-    const uint32_t ri = of.row + c0 + static_cast<uint32_t>(32 * r) * of.tok;
+    const uint32_t ri = of.row + c0 + static_cast<uint32_t>(32 * r) * of.tok - past_end<RAGGED>(a, n, row + 32 * r) * of.tok;
     const uint4 *qp = reinterpret_cast<const uint4 *>(a.q + ri);
     const uint4 *kp = reinterpret_cast<const uint4 *>(a.k + ri);
     in.q[r][0] = qp[0];
@@ -125,11 +134,13 @@ __device__ __forceinline__ void load_chunk(const StateArgs &a, const Offsets &of
   for (int i = 0; i < 4; ++i) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const uint32_t ui = ti + static_cast<uint32_t>(16 * i + e) * of.tok;
+      const uint32_t ui = ti + static_cast<uint32_t>(16 * i + e) * of.tok - past_end<RAGGED>(a, n, 16 * i + 4 * (lane >> 4) + e) * of.tok;
       in.u[i][e] = WU_F32 ? static_cast<const float *>(a.u)[ui] : bf16f(static_cast<const uint16_t *>(a.u)[ui]);
     }
   }
-  in.gc = a.g[of.g + static_cast<uint32_t>(n) * kC * static_cast<uint32_t>(a.H)];
+  const uint32_t back = past_end<RAGGED>(a, n, lane);
+  in.gc = a.g[of.g + (static_cast<uint32_t>(n) * kC - back) * static_cast<uint32_t>(a.H)];
+  if (RAGGED && back) in.gc = 0.0f;
 }
 
 // 8 bf16 values of a uint4 as floats.
@@ -200,12 +211,14 @@ __device__ __forceinline__ void stage_w(LW *dst, const uint4 (&w)[WU_F32 ? 4 : 2
 }
 
 // One 16 x 16 result tile of o: `at` is the element offset of the lane's column in row 4 qd of the
-// tile, tok the elements per token, qq the lane's place in its quad.
-template <bool OUT_F32>
-__device__ __forceinline__ void store_o(void *o, uint32_t at, uint32_t tok, int qq, const v4f &acc) {
+// tile, tok the elements per token, qq the lane's place in its quad; rows: how many of the lane's 4
+// rows exist (RAGGED).
+template <bool OUT_F32, bool RAGGED>
+__device__ __forceinline__ void store_o(void *o, uint32_t at, uint32_t tok, int qq, const v4f &acc, int rows) {
   if constexpr (OUT_F32) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) static_cast<float *>(o)[at + static_cast<uint32_t>(e) * tok] = acc[e];
+    for (int e = 0; e < 4; ++e)
+      if (!RAGGED || e < rows) static_cast<float *>(o)[at + static_cast<uint32_t>(e) * tok] = acc[e];
   } else {
     // the quad's 4 rows x 4 adjacent columns, transposed with DPP quad broadcasts so that lane
     // q of the quad stores row 4 qd + q, the quad's 4 columns, in one 8-byte store
@@ -221,11 +234,12 @@ __device__ __forceinline__ void store_o(void *o, uint32_t at, uint32_t tok, int 
     const uint32_t sel = (qq & 1) ? 0x07060302u : 0x05040100u;
     const uint2 w = qq < 2 ? make_uint2(__builtin_amdgcn_perm(a1, a0, sel), __builtin_amdgcn_perm(a3, a2, sel))
                            : make_uint2(__builtin_amdgcn_perm(b1, b0, sel), __builtin_amdgcn_perm(b3, b2, sel));
-    *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(o) + (at - static_cast<uint32_t>(qq) + static_cast<uint32_t>(qq) * tok)) = w;
+    if (!RAGGED || qq < rows)
+      *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(o) + (at - static_cast<uint32_t>(qq) + static_cast<uint32_t>(qq) * tok)) = w;
   }
 }
 
-template <bool SPLIT, bool WU_F32, bool OUT_F32>
+template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
   constexpr int RP = 8 * 64 / kThreads;  // row segments (16 columns of one token) per thread in L
   // q, k rows as given (bf16, exact MFMA operands) with their l2norm factors; W and the lower
@@ -257,7 +271,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
 
   const Offsets of = offsets(a, b, h, t, wave, lane);
   ChunkIn<WU_F32, RP> in;
-  load_chunk<WU_F32, RP>(a, of, 0, in);
+  load_chunk<WU_F32, RP, RAGGED>(a, of, 0, t >> 3, lane, in);
 
   auto chunk = [&](const int n) __attribute__((always_inline)) {
     // ---- L: q, k, W into LDS; norms; g, e^g, e^{g_last - g} ------------------------------------
@@ -291,7 +305,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
         const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), 63));
         gl[lane] = g;
         egl[lane] = expf(g);
-        decl[lane] = expf(glast - g);
+        decl[lane] = RAGGED && n * kC + lane >= a.T ? 0.0f : expf(glast - g);
         if (lane == 0) eglast = expf(glast);
       }
     }
@@ -305,7 +319,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
     // Unconditional (the last chunk reloads itself, unused): behind a branch the compiler would
     // lose count of the loads in flight and make the next chunk wait for every memory operation,
     // this chunk's o stores included, instead of just these loads.
-    load_chunk<WU_F32, RP>(a, of, min(n + 1, a.nchunks - 1), in);
+    load_chunk<WU_F32, RP, RAGGED>(a, of, min(n + 1, a.nchunks - 1), t >> 3, lane, in);
 
     // ---- M: W S, q^ S, v_new; P tiles ----------------------------------------------------------
     Half4 sB[8];
@@ -388,7 +402,8 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
         }
         acc = mma<SPLIT>(p0, p1, vB[2 * p], two ? vB[2 * p + 1] : kZero4, acc);
       }
-      store_o<OUT_F32>(a.o, of.tile + static_cast<uint32_t>(n * kC + 16 * i) * of.tok, of.tok, r16 & 3, acc);
+      store_o<OUT_F32, RAGGED>(a.o, of.tile + static_cast<uint32_t>(n * kC + 16 * i) * of.tok, of.tok, r16 & 3, acc,
+                               a.T - (n * kC + 16 * i + 4 * qd));
     }
 
     // ---- S: S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new) -------------------------------
@@ -443,7 +458,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
 // W S (and v_new), the other for q S (and o); with WPC = 4 one wave does both.  The sums are formed in
 // the order of gdn_state_kernel, so the results are the same bit for bit.
 constexpr int kColThreads = 1024;
-template <bool SPLIT, bool WU_F32, bool OUT_F32, int CT>
+template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED, int CT>
 __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a) {
   constexpr int WPC = 16 / CT, KB = 8 / WPC;
   constexpr bool kRoles = WPC == 8;        // W S and q S on different waves
@@ -501,25 +516,29 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
   float iu[4], igc;
   auto load = [&](int n) __attribute__((always_inline)) {
     const uint32_t c0 = static_cast<uint32_t>(n) * kC * tok;
-    const uint4 *p = reinterpret_cast<const uint4 *>(qk + of_row + c0);
+    const uint4 *p = reinterpret_cast<const uint4 *>(qk + (of_row + c0 - past_end<RAGGED>(a, n, row) * tok));
     in[0] = p[0];
     in[1] = p[1];
-    const uint4 *wp = WU_F32 ? reinterpret_cast<const uint4 *>(static_cast<const float *>(a.w) + of_w + c0)
-                             : reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.w) + of_w + c0);
+    const uint32_t wi = of_w + c0 - past_end<RAGGED>(a, n, wrow) * tok;
+    const uint4 *wp = WU_F32 ? reinterpret_cast<const uint4 *>(static_cast<const float *>(a.w) + wi)
+                             : reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.w) + wi);
     iw[0] = wp[0];
     if (WU_F32) iw[WU_F32 ? 1 : 0] = wp[1];
-    igc = a.g[of_g + static_cast<uint32_t>(n) * kC * static_cast<uint32_t>(a.H)];
+    const uint32_t back = past_end<RAGGED>(a, n, lane);
+    igc = a.g[of_g + (static_cast<uint32_t>(n) * kC - back) * static_cast<uint32_t>(a.H)];
+    if (RAGGED && back) igc = 0.0f;
   };
   auto load_u = [&](int n) __attribute__((always_inline)) {
     const uint32_t c0 = static_cast<uint32_t>(n) * kC * tok;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const uint32_t ui = of_tile + c0 + static_cast<uint32_t>(e) * tok;
+      const uint32_t ui = of_tile + c0 + static_cast<uint32_t>(e) * tok - past_end<RAGGED>(a, n, 16 * ti + 4 * qd + e) * tok;
       iu[e] = WU_F32 ? static_cast<const float *>(a.u)[ui] : bf16f(static_cast<const uint16_t *>(a.u)[ui]);
     }
   };
-  // a chunk's rows into LDS (buffer bf of the double-buffered arrays), with the norms and decays
-  auto stage = [&](int bf) __attribute__((always_inline)) {
+  // chunk n's rows into LDS (buffer n & 1 of the double-buffered arrays), with the norms and decays
+  auto stage = [&](int n) __attribute__((always_inline)) {
+    const int bf = n & 1;
     uint16_t *const d = is_q ? &Ql[row][16 * seg] : &Kl[bf][row][16 * seg];
     *reinterpret_cast<uint4 *>(d) = in[0];
     *reinterpret_cast<uint4 *>(d + 8) = in[1];
@@ -551,7 +570,7 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
       const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), 63));
       gl[bf][lane] = g;
       egl[bf][lane] = expf(g);
-      decl[bf][lane] = expf(glast - g);
+      decl[bf][lane] = RAGGED && n * kC + lane >= a.T ? 0.0f : expf(glast - g);
       if (lane == 0) eglast[bf] = expf(glast);
     }
   };
@@ -669,10 +688,10 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
         }
         acc = mma<SPLIT>(p0, p1, get(Vr[ct][2 * p][lane]), two ? get(Vr[ct][2 * p + 1][lane]) : kZero4, acc);
       }
-      store_o<OUT_F32>(a.o, of_tile + static_cast<uint32_t>(n * kC) * tok, tok, r16 & 3, acc);
+      store_o<OUT_F32, RAGGED>(a.o, of_tile + static_cast<uint32_t>(n * kC) * tok, tok, r16 & 3, acc, a.T - (n * kC + 16 * ti + 4 * qd));
     }
     // ---- the next chunk's rows (the last chunk stages itself again, unused) -------------------------
-    stage(bf ^ 1);
+    stage(n + 1);
     load(min(n + 2, a.nchunks - 1));
     lds_barrier();
   };
@@ -685,16 +704,21 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
   }
 }
 
-template <bool SPLIT, bool WU_F32, bool OUT_F32>
-qh_status launch3(const StateArgs &a, hipStream_t stream) {
+template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED>
+qh_status launch4(const StateArgs &a, hipStream_t stream) {
   const int seqs = a.B * a.H, cus = device_cu_count(), per8 = (seqs + 7) / 8 * 8;
   if (per8 * 4 <= cus)
-    hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, 2>), dim3(per8 * 4), dim3(kColThreads), 0, stream, a);
+    hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, 2>), dim3(per8 * 4), dim3(kColThreads), 0, stream, a);
   else
-    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32>), dim3(seqs), dim3(kThreads), 0, stream, a);
+    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32, RAGGED>), dim3(seqs), dim3(kThreads), 0, stream, a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return hip_fail(err, "gdn_state_kernel launch");
   return QH_STATUS_OK;
+}
+
+template <bool SPLIT, bool WU_F32, bool OUT_F32>
+qh_status launch3(const StateArgs &a, hipStream_t stream) {
+  return a.T % kC ? launch4<SPLIT, WU_F32, OUT_F32, true>(a, stream) : launch4<SPLIT, WU_F32, OUT_F32, false>(a, stream);
 }
 
 template <bool SPLIT>
@@ -708,7 +732,7 @@ qh_status launch2(const StateArgs &a, bool wu_f32, bool out_f32, hipStream_t str
 qh_status launch_gdn_chunk_state(const uint16_t *q, const uint16_t *k, const float *g, const void *w, const void *u,
                                  const float *s_in, float *s_out, void *o, int B, int T, int H, int precision,
                                  bool wu_f32, bool out_f32, hipStream_t stream) {
-  StateArgs a{q, k, g, w, u, s_in, s_out, o, B, T, H, T / kC};
+  StateArgs a{q, k, g, w, u, s_in, s_out, o, B, T, H, (T + kC - 1) / kC};
   return precision == QH_GDN_BF16 ? launch2<false>(a, wu_f32, out_f32, stream)
                                   : launch2<true>(a, wu_f32, out_f32, stream);
 }

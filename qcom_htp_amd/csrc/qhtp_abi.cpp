@@ -262,12 +262,14 @@ qh_status qh_gdn_chunk_uw_ex(const uint16_t *k_dev, const uint16_t *v_dev, const
   if (head_dim != 128) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_uw: head_dim=%u (need 128)", head_dim);
   if (chunk != 64 && chunk != 128 && chunk != 256)
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_uw: chunk=%u (need 64, 128 or 256)", chunk);
-  if (batch == 0 || heads == 0 || tokens == 0 || tokens % chunk)
+  const bool ragged = (flags & QH_GDN_RAGGED) != 0;
+  if (ragged && chunk != 64) return fail(QH_STATUS_UNSUPPORTED, "qh_gdn_chunk_uw: QH_GDN_RAGGED needs chunk 64 (got %u)", chunk);
+  if (batch == 0 || heads == 0 || tokens == 0 || (!ragged && tokens % chunk))
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_uw: batch=%u tokens=%u heads=%u (tokens %% chunk == 0)",
                 batch, tokens, heads);
   if (static_cast<uint64_t>(batch) * tokens * heads > (1ull << 31) / 128)
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_uw: batch * tokens * heads too large");
-  if (flags & ~static_cast<uint32_t>(QH_GDN_W_DECAY | QH_GDN_OUT_F32))
+  if (flags & ~static_cast<uint32_t>(QH_GDN_W_DECAY | QH_GDN_OUT_F32 | QH_GDN_RAGGED))
     return fail(QH_STATUS_UNSUPPORTED, "qh_gdn_chunk_uw: unknown flags 0x%x", flags);
   const uintptr_t al = reinterpret_cast<uintptr_t>(k_dev) | reinterpret_cast<uintptr_t>(v_dev) |
                        reinterpret_cast<uintptr_t>(w_dev) | reinterpret_cast<uintptr_t>(u_dev);
@@ -296,13 +298,13 @@ qh_status qh_gdn_chunk_state(const uint16_t *q_dev, const uint16_t *k_dev, const
     return fail(QH_STATUS_INVALID_ARGUMENT, "qh_gdn_chunk_state: NULL buffer");
   if (head_dim != 128) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_state: head_dim=%u (need 128)", head_dim);
   if (chunk != 64) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_state: chunk=%u (need 64)", chunk);
-  if (batch == 0 || heads == 0 || tokens == 0 || tokens % 64)
+  if (batch == 0 || heads == 0 || tokens == 0 || (!(flags & QH_GDN_RAGGED) && tokens % 64))
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_state: batch=%u tokens=%u heads=%u (tokens %% 64 == 0)",
                 batch, tokens, heads);
   if (static_cast<uint64_t>(batch) * tokens * heads > (1ull << 31) / 128 ||
       static_cast<uint64_t>(batch) * heads > (1u << 24))
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_state: batch * tokens * heads too large");
-  if (flags & ~static_cast<uint32_t>(QH_GDN_OUT_F32 | QH_GDN_WU_F32))
+  if (flags & ~static_cast<uint32_t>(QH_GDN_OUT_F32 | QH_GDN_WU_F32 | QH_GDN_RAGGED))
     return fail(QH_STATUS_UNSUPPORTED, "qh_gdn_chunk_state: unknown flags 0x%x", flags);
   if (precision > QH_GDN_BF16) return fail(QH_STATUS_UNSUPPORTED, "qh_gdn_chunk_state: unknown precision %u", precision);
   if (s_in_dev != nullptr && s_in_dev == s_out_dev)

@@ -90,6 +90,10 @@ def gdn_chunk_uw(k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, beta: torch.
     float32 [B, T, H]: U = T (beta v), W = T (beta l2norm(k)) [times e^g when decay_w], with
     T = (I - A)^-1 of each chunk of ``chunk`` tokens.  ``max_workgroups`` caps the persistent
     grid (0: every workgroup the device holds at once)."""
+    return _chunk_uw(k, v, g, beta, chunk, decay_w, out_dtype, stream, max_workgroups, 0)
+
+
+def _chunk_uw(k, v, g, beta, chunk, decay_w, out_dtype, stream, max_workgroups, more_flags):
     for name, x, dt in (("k", k, torch.bfloat16), ("v", v, torch.bfloat16), ("g", g, torch.float32),
                         ("beta", beta, torch.float32)):
         if x.device.type != "cuda" or x.dtype != dt or not x.is_contiguous():
@@ -103,7 +107,7 @@ def gdn_chunk_uw(k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, beta: torch.
     with _on(stream):
         w = torch.empty((B, T, H, D), dtype=out_dtype, device=k.device)
         u = torch.empty_like(w)
-    flags = (W_DECAY if decay_w else 0) | (_lib.QH_GDN_OUT_F32 if out_dtype == torch.float32 else 0)
+    flags = more_flags | (W_DECAY if decay_w else 0) | (_lib.QH_GDN_OUT_F32 if out_dtype == torch.float32 else 0)
     st = _lib.lib().qh_gdn_chunk_uw_ex(k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), w.data_ptr(),
                                        u.data_ptr(), B, T, H, D, chunk, flags, int(max_workgroups), _stream(stream))
     _lib.check(st, "qh_gdn_chunk_uw")
@@ -120,6 +124,10 @@ def gdn_chunk_state(q: torch.Tensor, k: torch.Tensor, g: torch.Tensor, w: torch.
     tokens from q, k bf16 [B, T, H, 128], the per-token log decays g float32 [B, T, H] and the
     stage-A outputs w, u [B, T, H, 128] (bf16 or float32; ``gdn_chunk_uw(..., 64, decay_w=True)``),
     starting from ``initial_state`` (float32 [B, H, 128, 128]; None = zero)."""
+    return _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, 0)
+
+
+def _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, more_flags):
     for name, x in (("q", q), ("k", k)):
         if x.device.type != "cuda" or x.dtype != torch.bfloat16 or not x.is_contiguous():
             raise TypeError(f"{name} must be a contiguous bfloat16 CUDA tensor")
@@ -143,7 +151,7 @@ def gdn_chunk_state(q: torch.Tensor, k: torch.Tensor, g: torch.Tensor, w: torch.
     with _on(stream):
         o = torch.empty((B, T, H, D), dtype=out_dtype, device=q.device)
         s_out = torch.empty((B, H, D, D), dtype=torch.float32, device=q.device)
-    flags = (_lib.QH_GDN_WU_F32 if w.dtype == torch.float32 else 0) | (
+    flags = more_flags | (_lib.QH_GDN_WU_F32 if w.dtype == torch.float32 else 0) | (
         _lib.QH_GDN_OUT_F32 if out_dtype == torch.float32 else 0)
     st = _lib.lib().qh_gdn_chunk_state(q.data_ptr(), k.data_ptr(), g.data_ptr(), w.data_ptr(), u.data_ptr(),
                                        0 if initial_state is None else initial_state.data_ptr(), s_out.data_ptr(),
@@ -157,20 +165,19 @@ def gdn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tens
                 out_dtype: torch.dtype = torch.bfloat16, stream: Optional[torch.cuda.Stream] = None):
     """The chunked gated-delta-rule prefill, the reference's ``gdn_kernel``
     (scripts/gdn_ref_kernel.py:104-131): q, k, v bf16 [B, T, H, 128], g (per-token log decay) and
-    beta float32 [B, T, H] -> (o [B, T, H, 128], S [B, H, 128, 128] float32).  T is zero-padded
-    to whole chunks of 64, which leaves o and S unchanged.  Stage A runs with float32 W, U for
-    ``FP32`` and bf16 for ``BF16``."""
+    beta float32 [B, T, H] -> (o [B, T, H, 128], S [B, H, 128, 128] float32).  The missing tokens
+    of a last partial chunk of 64 count as zeros, which leaves o and S unchanged.  Stage A runs
+    with float32 W, U for ``FP32`` and bf16 for ``BF16``."""
     B, T, H, D = q.shape
     _same_device(q.device, k=k, v=v, g=g, beta=beta, initial_state=initial_state)
-    # the padded inputs and the stage-A outputs are temporaries: allocated (and padded) on the
-    # launch stream, so they stay reserved until the kernels queued there have read them
+    ragged = _lib.QH_GDN_RAGGED if T % STATE_CHUNK else 0
+    wu_dtype = torch.float32 if precision == FP32 else torch.bfloat16
+    # w and u (and the copies below) are temporaries: allocated on the launch stream, so they stay
+    # reserved until the kernels queued there have read them
     with _on(stream):
-        pad = (-T) % STATE_CHUNK
-        if pad:
-            F = torch.nn.functional
-            q, k, v = (F.pad(x, (0, 0, 0, 0, 0, pad)).contiguous() for x in (q, k, v))
-            g, beta = (F.pad(x, (0, 0, 0, pad)).contiguous() for x in (g, beta))
-        wu_dtype = torch.float32 if precision == FP32 else torch.bfloat16
-        w, u = gdn_chunk_uw(k, v, g, beta, STATE_CHUNK, decay_w=True, out_dtype=wu_dtype, stream=stream)
-        o, s = gdn_chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream)
-        return (o[:, :T].contiguous() if pad else o), s
+        if ragged:
+            # a partial last chunk takes inputs of any strides and alignment; whole chunks are checked
+            g, beta = g.contiguous(), beta.contiguous()
+            q, k, v = (x if x.data_ptr() % 16 == 0 else x.clone() for x in (q.contiguous(), k.contiguous(), v.contiguous()))
+        w, u = _chunk_uw(k, v, g, beta, STATE_CHUNK, True, wu_dtype, stream, 0, ragged)
+        return _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, ragged)

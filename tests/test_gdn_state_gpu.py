@@ -312,3 +312,41 @@ def test_few_sequences_equal_many(gpu, precision, wu, out):
         o, s = run(slice(lo, lo + n))
         assert torch.equal(o, o_all[:, :, lo:lo + n]), f"{n} sequences: o differs"
         assert torch.equal(s, s_all[:, lo:lo + n]), f"{n} sequences: S differs"
+
+
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("H", [3, 70], ids=["few_sequences", "many_sequences"])
+@pytest.mark.parametrize("T", [1, 16, 63, 65, 100, 177])
+def test_ragged_prefill_equals_zero_padded(gpu, T, H, precision, out):
+    """A last partial chunk gives the bits of the same tokens padded with zeros to whole chunks."""
+    import torch
+
+    from qcom_htp_amd.gdn import gdn_prefill
+
+    B = 2
+    qb, kb, vb, beta, gc = seq_inputs(B, T, H, seed=T + H)
+    q, k, v, bt, g = (to_dev(x, gpu) for x in (qb, kb, vb, beta, gc))
+    s0 = torch.randn((B, H, 128, 128), generator=torch.Generator(device=gpu).manual_seed(3), device=gpu)
+    odt = torch.float32 if out == "f32" else torch.bfloat16
+    pad = -T % 64
+    P = torch.nn.functional.pad
+    qp, kp, vp = (P(x, (0, 0, 0, 0, 0, pad)) for x in (q, k, v))
+    o_ref, s_ref = gdn_prefill(qp, kp, vp, P(g, (0, 0, 0, pad)), P(bt, (0, 0, 0, pad)), s0, precision, odt)
+    o, s = gdn_prefill(q, k, v, g, bt, s0, precision, odt)
+    assert torch.equal(o, o_ref[:, :T]) and torch.equal(s, s_ref)
+
+
+def test_ragged_prefill_takes_strided_and_unaligned_inputs(gpu):
+    import torch
+
+    from qcom_htp_amd.gdn import gdn_prefill
+
+    B, T, H = 1, 70, 2
+    q, k, v, bt, g = (to_dev(x, gpu) for x in seq_inputs(B, T, H, seed=5))
+    want = gdn_prefill(q, k, v, g, bt)
+    odd = torch.empty(k.numel() + 1, dtype=k.dtype, device=gpu)[1:].view(k.shape)  # 2-byte aligned
+    odd.copy_(k)
+    strided = torch.stack((v, v), dim=-1)[..., 0]
+    got = gdn_prefill(q, odd, strided, torch.stack((g, g), dim=-1)[..., 0], bt)
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
