@@ -16,7 +16,12 @@
 // once, as ready operand records.
 // Work split: G = 2 workgroups (8 waves) per head for NB > 8, one otherwise.  Strips k and
 // NB - 1 - k share a SIMD (waves w and w + 4), so the longest strip (k = 0) has its SIMD's matrix
-// core nearly to itself.  The G workgroups of a head get block indexes of one residue mod 8,
+// core nearly to itself.  The kernel is compiled for at most M = 1, 2, 4, 8 or 16 diagonal blocks: a
+// head of up to 4 blocks is one wave per strip with the LDS and registers of that size, so that a
+// compute unit holds several heads (up to 10 of C = 64) and their latencies overlap, where the
+// 16-block workgroup (512 threads, 157 KB of LDS) has the unit to itself.  With the 16-block kernel
+// for every C against this: u16 C = 64 x 2048 heads 43.3 -> 15.1 us, C = 16 x 8192 101 -> 8.4, C = 128 x
+// 1024 35.1 -> 22.5; 8 heads of C = 64 6.2 -> 5.3.  The G workgroups of a head get block indexes of one residue mod 8,
 // which places them on one XCD and one L2.
 // The products run on v_mfma_f32_16x16x32_bf16: a 32-deep k step takes rows 4q .. 4q+3 of two
 // 16-row blocks, the k order in which the MFMA result layout (lane: rows 4q .. 4q+3 of one
@@ -38,7 +43,9 @@ using namespace bf16s;
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 
-constexpr int kRdThreads = 512;
+// Threads of a workgroup for heads of at most M blocks.
+template <int M>
+constexpr int fs_threads() { return M <= 4 ? 64 * M : 512; }
 constexpr int kAtRow = 20;  // staged diagonal block A^T: row stride (16-byte aligned rows) ..
 constexpr int kAtBlk = 336;  // .. and block stride (= 16 mod 64 banks: the 4 blocks of a wave differ)
 
@@ -91,8 +98,6 @@ __device__ __forceinline__ void stage_at(float *dstage, int bb, int i, int k4, c
   d[3 * kAtRow] = v.w;
 }
 
-constexpr int kFsMaxNB = 16;
-constexpr int kFsLowBlocks = kFsMaxNB * (kFsMaxNB - 1) / 2;  // strictly lower 16 x 16 blocks
 constexpr int kFsTd = 16;  // Td row stride, words
 
 // Word column of column c in row r of a 16 x 16 LDS block: the 4-word quarters of row r are
@@ -102,8 +107,11 @@ constexpr int kFsTd = 16;  // Td row stride, words
 __device__ __forceinline__ int fs_col(int r, int c) { return ((((c >> 2) ^ (r >> 2)) & 3) << 2) | (c & 3); }
 
 // Strip of wave `wave` in workgroup `part`: pair k = 4 part + wave % 4, strip k for waves 0..3 and
-// NB - 1 - k for waves 4..7 (none when that would repeat strip k or lie past NB).
+// NB - 1 - k for waves 4..7 (none when that would repeat strip k or lie past NB).  At most 4 blocks:
+// strip `wave`.
+template <int M>
 __device__ __forceinline__ int fs_strip(int NB, int part, int wave) {
+  if constexpr (M <= 4) return wave < NB ? wave : -1;
   const int k = 4 * part + (wave & 3);
   const int j = wave < 4 ? k : NB - 1 - k;
   return (j < NB && (wave < 4 || j > k)) ? j : -1;
@@ -191,7 +199,7 @@ __device__ __forceinline__ void store_tile_rows(const GdnArgs &g, __amdgpu_buffe
 
 // One wave's strip j (after level 0, with Al, Td and the fp32 T_bb in dstage staged): T_jj, then
 // the strip's steps, each tile stored as it is computed.
-template <bool U16, bool SPLIT>
+template <bool U16, bool SPLIT, int M>
 __device__ __forceinline__ void fs_strip_solve(const GdnArgs &g, size_t hbase, const uint32_t (*Al)[16][16],
                                                const uint32_t (*Td)[16][kFsTd], const float *dstage, int NB, int j,
                                                int lane) {
@@ -199,10 +207,10 @@ __device__ __forceinline__ void fs_strip_solve(const GdnArgs &g, size_t hbase, c
   // Blocks are indexed relative to the strip (u = c - j, v = b - j), so every step's loops have
   // compile-time bounds: a step is one basic block whose LDS reads all issue before its products
   // (guards per block pair made each pair wait for its own reads).
-  Half4 xs[kFsMaxNB];  // X_{j+u} as B operands (rows 4q .. 4q + 3 of column r16)
+  Half4 xs[M];  // X_{j+u} as B operands (rows 4q .. 4q + 3 of column r16)
   // The stored values of every step stay allocated until the strip ends: when a later step's LDS
   // reads reused a store's data registers, the compiler made them wait for the whole store.
-  float wk[kFsMaxNB][4];
+  float wk[M][4];
   // T of this head as a buffer (C x C elements) and this lane's offset in a stored tile: row
   // 4q + p, columns 4a .. 4a + 3 (lane 16 q + 4 a + p)
   const size_t esz = U16 ? 2 : 4;
@@ -221,7 +229,7 @@ __device__ __forceinline__ void fs_strip_solve(const GdnArgs &g, size_t hbase, c
   // A step's operands (the operand records of its A blocks and its T_bb) are read during the step
   // before: the reads of a step issued at its start left one LDS round trip per few products on
   // the strip's critical path.  Reads for a step past the last one fetch block 0 (never used).
-  uint4 rc[kFsMaxNB];
+  uint4 rc[M];
   uint4 tc;
   {
     const bool any = steps > 0;
@@ -229,13 +237,13 @@ __device__ __forceinline__ void fs_strip_solve(const GdnArgs &g, size_t hbase, c
     tc = *reinterpret_cast<const uint4 *>(&Td[any ? j + 1 : 0][r16][qs]);
   }
 #pragma unroll
-  for (int v = 1; v < kFsMaxNB; ++v) {
+  for (int v = 1; v < M; ++v) {
     if (v > steps) continue;  // uniform (a break would stop the unrolling)
     const int b = j + v;
     const bool more = v < steps;
     const int nbase = more ? (b + 1) * b / 2 + j : 0;  // the next step's row of A blocks
     const int nstep = more ? 1 : 0;
-    uint4 rn[kFsMaxNB];
+    uint4 rn[M];
     // Y = sum_{u < v} A_{b, j+u} X_{j+u} over pairs (u, u + 1); products go to kAcc accumulators
     // in turn (with SPLIT one per product kind), so consecutive products do not wait for each other
     constexpr int kAcc = SPLIT ? 3 : 2;
@@ -279,19 +287,21 @@ __device__ __forceinline__ void fs_strip_solve(const GdnArgs &g, size_t hbase, c
     for (int u = 0; u <= v; ++u) rc[u] = rn[u];
   }
 #pragma unroll
-  for (int v = 0; v < kFsMaxNB; ++v)
+  for (int v = 0; v < M; ++v)
     if (v <= steps) asm volatile("" ::"v"(wk[v][0]), "v"(wk[v][1]), "v"(wk[v][2]), "v"(wk[v][3]));
 }
 
-template <bool U16, bool SPLIT>
-__global__ __launch_bounds__(kRdThreads) void gdn_fs_kernel(GdnArgs g) {
+template <bool U16, bool SPLIT, int M>
+__global__ __launch_bounds__(fs_threads<M>()) void gdn_fs_kernel(GdnArgs g) {
+  constexpr int NT = fs_threads<M>(), kWaves = NT / 64;
+  constexpr int kLow = M * (M - 1) / 2;  // strictly lower 16 x 16 blocks
   // A's strictly lower blocks (b, c), block index b (b - 1) / 2 + c.  Row r16 of a block is 16
   // words: per 4-column quarter, the operand record of the lane that reads it (bf16 hi parts of
   // the 4 values as two pairs, then the lo parts), so an A operand is one 16-byte read with no
   // unpacking, and a block's reads are one contiguous KiB
-  __shared__ __attribute__((aligned(16))) uint32_t Al[kFsLowBlocks][16][16];
-  __shared__ __attribute__((aligned(16))) uint32_t Td[kFsMaxNB][16][kFsTd];  // T_bb, hi | lo
-  __shared__ __attribute__((aligned(16))) float dstage[kFsMaxNB * kAtBlk];   // A_bb^T for level 0
+  __shared__ __attribute__((aligned(16))) uint32_t Al[kLow > 0 ? kLow : 1][16][16];
+  __shared__ __attribute__((aligned(16))) uint32_t Td[M][16][kFsTd];  // T_bb, hi | lo
+  __shared__ __attribute__((aligned(16))) float dstage[M * kAtBlk];   // A_bb^T for level 0
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // scalar: strip choices branch on it
   const int k8 = blockIdx.x >> 3;
@@ -301,26 +311,26 @@ __global__ __launch_bounds__(kRdThreads) void gdn_fs_kernel(GdnArgs g) {
   const int C = g.C, NB = C / 16;
 
   // ---- A reads: the diagonal blocks (level 0) first, then the strictly lower blocks -------------
-  float4 dv[2];
+  constexpr int kDiagLoads = (M + kWaves - 1) / kWaves;
+  float4 dv[kDiagLoads];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {  // block wave + 8 u, row (t / 4) % 16, quarter t % 4
-    const int bb = wave + 8 * u, i = (lane >> 2) & 15, k4 = lane & 3;
+  for (int u = 0; u < kDiagLoads; ++u) {  // block wave + kWaves u, row (t / 4) % 16, quarter t % 4
+    const int bb = wave + kWaves * u, i = (lane >> 2) & 15, k4 = lane & 3;
     dv[u] = load_a4_or0<U16>(g, hbase, 16 * bb + i, 16 * bb + 4 * k4, bb < NB);
   }
   __builtin_amdgcn_sched_barrier(0);  // level 0's reads first: its wait then covers only them
-  // lower block slot s = t + 512 u (u < 15): block s / 64 in row-major (b, c) order, row
-  // (s / 4) % 16, quarter s % 4
-  constexpr int kLowLoads = kFsLowBlocks * 64 / kRdThreads;
-  static_assert(kFsLowBlocks * 64 % kRdThreads == 0, "whole lower-block loads per thread");
+  // lower block slot s = t + NT u: block s / 64 in row-major (b, c) order, row (s / 4) % 16,
+  // quarter s % 4
+  constexpr int kLowLoads = (kLow * 64 + NT - 1) / NT;
   const int nlow = NB * (NB - 1) / 2;
-  float4 lv[kLowLoads];
+  float4 lv[kLowLoads > 0 ? kLowLoads : 1];
 #pragma unroll
   for (int u = 0; u < kLowLoads; ++u) {
-    const int s = t + kRdThreads * u, blk = s >> 6;
+    const int s = t + NT * u, blk = s >> 6;
     // block index -> (b, c): b is the largest with b (b - 1) / 2 <= blk
     int b = 1;
 #pragma unroll
-    for (int bb = 2; bb < kFsMaxNB; ++bb) b = (bb * (bb - 1) / 2 <= blk) ? bb : b;
+    for (int bb = 2; bb < M; ++bb) b = (bb * (bb - 1) / 2 <= blk) ? bb : b;
     const int c = blk - b * (b - 1) / 2;
     lv[u] = load_a4_or0<U16>(g, hbase, 16 * b + ((s >> 2) & 15), 16 * c + 4 * (s & 3), blk < nlow);
   }
@@ -328,15 +338,15 @@ __global__ __launch_bounds__(kRdThreads) void gdn_fs_kernel(GdnArgs g) {
 
   // ---- level 0 --------------------------------------------------------------------------------
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int bb = wave + 8 * u, i = (lane >> 2) & 15, k4 = lane & 3;
+  for (int u = 0; u < kDiagLoads; ++u) {
+    const int bb = wave + kWaves * u, i = (lane >> 2) & 15, k4 = lane & 3;
     if (bb < NB) stage_at(dstage, bb, i, k4, dv[u]);
   }
   lds_barrier();
   fs_level0<SPLIT>(Td, dstage, NB, t);
 #pragma unroll
   for (int u = 0; u < kLowLoads; ++u) {
-    const int s = t + kRdThreads * u, blk = s >> 6;
+    const int s = t + NT * u, blk = s >> 6;
     if (blk < nlow) {
       // the operand record of lane (row, quarter): hi pairs then lo pairs, read as one Half4
       const Half4 h = split4<SPLIT>(lv[u]);
@@ -347,12 +357,14 @@ __global__ __launch_bounds__(kRdThreads) void gdn_fs_kernel(GdnArgs g) {
   lds_barrier();
 
   // ---- the wave's strip ---------------------------------------------------------------------------
-  const int j = __builtin_amdgcn_readfirstlane(fs_strip(NB, part, wave));
-  if (j >= 0) fs_strip_solve<U16, SPLIT>(g, hbase, Al, Td, dstage, NB, j, lane);
-  // Zeros above the diagonal blocks, after the strips and by waves 4..7 (the shorter strips):
-  // issued before the strips they held the longest strip back by about a microsecond
-  if (wave >= 4) {
-    for (int row = part + (wave - 4) * g.groups; row < C; row += 4 * g.groups) {
+  const int j = __builtin_amdgcn_readfirstlane(fs_strip<M>(NB, part, wave));
+  if (j >= 0) fs_strip_solve<U16, SPLIT, M>(g, hbase, Al, Td, dstage, NB, j, lane);
+  // Zeros above the diagonal blocks, after the strips and by waves 4..7 (the shorter strips; every
+  // wave of a small head): issued before the strips they held the longest strip back by about a
+  // microsecond
+  constexpr int kZ0 = M <= 4 ? 0 : 4;
+  if (wave >= kZ0) {
+    for (int row = part + (wave - kZ0) * g.groups; row < C; row += (kWaves - kZ0) * g.groups) {
       const int c = 4 * lane;
       if (c < C && c >= 16 * (row / 16) + 16) {
         const size_t idx = hbase + static_cast<size_t>(row) * C + c;
@@ -376,7 +388,18 @@ template <bool U16, bool SPLIT>
 qh_status launch_fs(const GdnArgs &g, int heads, hipStream_t stream) {
   const long long blocks = static_cast<long long>((heads + 7) / 8) * 8 * g.groups;
   if (blocks > 0x7FFFFFFFLL) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "gdn: %d heads exceed one launch", heads);
-  hipLaunchKernelGGL((gdn_fs_kernel<U16, SPLIT>), dim3(static_cast<unsigned>(blocks)), dim3(kRdThreads), 0, stream, g);
+  const dim3 grid(static_cast<unsigned>(blocks));
+  const int nb = g.C / 16;
+  if (nb <= 1)
+    hipLaunchKernelGGL((gdn_fs_kernel<U16, SPLIT, 1>), grid, dim3(fs_threads<1>()), 0, stream, g);
+  else if (nb <= 2)
+    hipLaunchKernelGGL((gdn_fs_kernel<U16, SPLIT, 2>), grid, dim3(fs_threads<2>()), 0, stream, g);
+  else if (nb <= 4)
+    hipLaunchKernelGGL((gdn_fs_kernel<U16, SPLIT, 4>), grid, dim3(fs_threads<4>()), 0, stream, g);
+  else if (nb <= 8)
+    hipLaunchKernelGGL((gdn_fs_kernel<U16, SPLIT, 8>), grid, dim3(fs_threads<8>()), 0, stream, g);
+  else
+    hipLaunchKernelGGL((gdn_fs_kernel<U16, SPLIT, 16>), grid, dim3(fs_threads<16>()), 0, stream, g);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return hip_fail(err, "gdn_fs_kernel launch");
   return QH_STATUS_OK;

@@ -36,9 +36,9 @@ BF16_FLOP_PER_CU_CYCLE = 2.5e15 / (256 * 2.4e9)
 _ANCHORS = [
     ("  // ---- A reads", 0),
     ("  fs_level0<SPLIT>(Td, dstage, NB, t);\n", 1),
-    ("#pragma unroll\n  for (int u = 0; u < kLowLoads; ++u) {\n    const int s = t + kRdThreads * u, blk = s >> 6;\n    if (blk < nlow) {", 2),
+    ("#pragma unroll\n  for (int u = 0; u < kLowLoads; ++u) {\n    const int s = t + NT * u, blk = s >> 6;\n    if (blk < nlow) {", 2),
     ("  // ---- the wave's strip", 3),
-    ("#pragma unroll\n  for (int v = 0; v < kFsMaxNB; ++v)\n    if (v <= steps) asm volatile", 4),
+    ("#pragma unroll\n  for (int v = 0; v < M; ++v)\n    if (v <= steps) asm volatile", 4),
 ]
 
 
@@ -56,7 +56,7 @@ def stamped_source() -> str:
         if src.count(anchor) != 1:
             raise RuntimeError(f"gdn_solve.hip changed: anchor not found once: {anchor!r}")
         src = src.replace(anchor, f"  STAMP({k});\n" + anchor, 1)
-    call = "  if (j >= 0) fs_strip_solve<U16, SPLIT>(g, hbase, Al, Td, dstage, NB, j, lane);\n"
+    call = "  if (j >= 0) fs_strip_solve<U16, SPLIT, M>(g, hbase, Al, Td, dstage, NB, j, lane);\n"
     if src.count(call) != 1:
         raise RuntimeError("gdn_solve.hip changed: strip call not found")
     src = src.replace(call, call + "  STAMP(5);\n"
@@ -68,8 +68,8 @@ extern "C" int stamps_set(unsigned long long *stamps) {
 extern "C" int stamps_solve(const void *A, void *T, int heads, int C, int split, void *stream) {
   qh::GdnArgs g{A, T, C, C / 16 > 8 ? 2 : 1, heads, 0, 0, 1.0f, 1.0f, 1.0f};
   const dim3 grid((heads + 7) / 8 * 8 * g.groups);
-  if (split) hipLaunchKernelGGL((qh::gdn_fs_kernel<false, true>), grid, dim3(512), 0, (hipStream_t)stream, g);
-  else hipLaunchKernelGGL((qh::gdn_fs_kernel<false, false>), grid, dim3(512), 0, (hipStream_t)stream, g);
+  if (split) hipLaunchKernelGGL((qh::gdn_fs_kernel<false, true, 16>), grid, dim3(512), 0, (hipStream_t)stream, g);
+  else hipLaunchKernelGGL((qh::gdn_fs_kernel<false, false, 16>), grid, dim3(512), 0, (hipStream_t)stream, g);
   return (int)hipGetLastError();
 }
 """

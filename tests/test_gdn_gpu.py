@@ -221,3 +221,30 @@ def test_gdn_op_model_rejects_large_chunks(gpu):
     st = _lib.lib().qh_gdn_solve_u16(A.data_ptr(), A.data_ptr(), 1, 128, 32768, 32768, 1e-4, 1e-4, 2,
                                     int(torch.cuda.current_stream().cuda_stream))
     assert st == _lib.QH_STATUS_SHAPE_UNSUPPORTED
+
+
+@pytest.mark.parametrize("heads", [1, 9, 40])
+@pytest.mark.parametrize("C", [16, 32, 48, 64, 80, 128, 144])
+def test_every_block_count_bound(gpu, C, heads):
+    """The solve is compiled for at most 1, 2, 4, 8 and 16 diagonal blocks: each bound and the first
+    size past it, float32 and u16 codes, head counts that do not fill the last round."""
+    import torch
+
+    from qcom_htp_amd.gdn import GdnSolve, gdn_solve
+
+    k, beta, gc = og.config4_inputs(heads=heads, C=C, seed=C + heads)
+    A = og.build_A(k, beta, gc).astype(np.float32)
+    dev = torch.from_numpy(A).to(gpu)
+    want = og.inverse_fp64(A.astype(np.float64))
+    for precision, tol in ((0, 1e-4), (1, 1.05e-2)):
+        T = gdn_solve(dev, precision=precision).cpu().numpy()
+        assert og.oc(T, want) <= tol
+        assert not np.triu(T, 1).any()
+    sA, sT = np.float32(np.abs(A).max() / 32767.0 + 1e-12), np.float32(2.0 / 32767.0)
+    codes = np.clip(np.rint(A / sA) + 32768, 0, 65535).astype(np.uint16)
+    got = GdnSolve(torch.from_numpy(codes.view(np.int16)).to(gpu).view(torch.uint16), 32768, float(sA), 32768, float(sT))
+    got = got.cpu().view(torch.int16).numpy().view(np.uint16).astype(np.int64)
+    Td = (got - 32768) * float(sT)
+    ref = og.inverse_fp64((codes.astype(np.int64) - 32768) * float(sA))
+    assert np.abs(np.clip(Td - ref, -1, 1)).max() <= 0.51 * float(sT) + 1e-4 * np.abs(ref).max()
+    assert (got[np.broadcast_to(np.triu(np.ones((C, C), bool), 1), got.shape)] == 32768).all()
