@@ -21,6 +21,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from .qmm import _stream_ptr as _stream
 
 FP32 = _lib.QH_GDN_FP32
 BF16 = _lib.QH_GDN_BF16
@@ -30,11 +31,6 @@ W_DECAY = _lib.QH_GDN_W_DECAY
 
 __all__ = ["gdn_solve", "gdn_chunk_uw", "gdn_chunk_state", "gdn_prefill", "GdnSolve", "FP32", "BF16", "OP_MODEL",
            "W_DECAY"]
-
-
-def _stream(stream):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
 
 
 def _on(stream):

@@ -60,9 +60,19 @@ def graph_contract(gc: GraphCase) -> tuple:
     return "div_rint", qmax
 
 
+# The current stream's handle without a Stream object, which takes 2.9 of a call's 9.7 us of host time
+# against 0.2 us.  (A call's tensors are on the GPU, so the runtime is initialised.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream_ptr(stream: Optional[torch.cuda.Stream]) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    """The hipStream_t of ``stream``, or of the current device's current stream."""
+    if stream is not None:
+        return int(stream.cuda_stream)
+    if _raw_stream is None or _raw_device is None:
+        return int(torch.cuda.current_stream().cuda_stream)
+    return _raw_stream(_raw_device())
 
 
 def _overlaps(a: Optional[torch.Tensor], b: Optional[torch.Tensor]) -> bool:
@@ -227,7 +237,7 @@ class QuantMatmul:
                  stream: Optional[torch.cuda.Stream] = None) -> torch.Tensor:
         m = self._check_act(act)
         if out is None:
-            out = torch.empty((m, self.n), dtype=self.out_dtype, device=act.device)
+            out = act.new_empty((m, self.n), dtype=self.out_dtype)
         else:
             self._check_out(out, m, act.device, "output")
             if _overlaps(act, out):
@@ -251,7 +261,7 @@ class QuantMatmul:
         m = self._check_act(act)
         cid = CONTRACTS[contract] if isinstance(contract, str) else int(contract)
         if out is None:
-            out = torch.empty((m, self.n), dtype=self.out_dtype, device=act.device)
+            out = act.new_empty((m, self.n), dtype=self.out_dtype)
         else:
             self._check_out(out, m, act.device, "output")
             if _overlaps(act, out):
@@ -272,7 +282,7 @@ class QuantMatmul:
         if int(chain) < 1:
             raise ValueError(f"chain must be >= 1, got {chain}")
         if out is None:
-            out = torch.empty((m, self.n), dtype=self.out_dtype, device=act.device)
+            out = act.new_empty((m, self.n), dtype=self.out_dtype)
         else:
             self._check_out(out, m, act.device, "output")
         if scratch is None and chain > 1:
