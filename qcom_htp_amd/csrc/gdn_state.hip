@@ -13,17 +13,20 @@
 // which is also the layout the MFMA reads as a B operand over pairs of key blocks (pair layout,
 // bf16_split.h), so W S and q S take S straight from the accumulators.  q and k stay the bf16
 // values they arrive as (exact MFMA operands); their l2norm factors scale the products' rows and
-// columns instead.  Per chunk:
-//   L. q, k rows and W (bf16 hi | lo words) into LDS; the row norms (8-lane DPP
-//      sums); g's prefix sum (64-lane DPP scan), e^g and e^{g_last - g} by one wave;
+// columns instead.  Per chunk, between two barriers each:
 //   M. each wave: W S and q S for its 16 value columns (4 token tiles), v_new = U - W S with U
 //      from registers, o's first term e^g q^ S; the 10 lower 16 x 16 tiles of q k^T over the
 //      waves, scaled by the norms and decays, into LDS as P;
-//   O. o = e^g q^ S + P v_new for the wave's columns (causal tiles only), stored;
-//   S. S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new), k^T read from the k rows by LDS
-//      transpose reads.
-// The next chunk's q, k, W, U and gc are read into registers during M, so their latency
-// overlaps this chunk's products; the workgroup issues them before its stores of o.
+//   N. S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new), k^T read from the k rows by LDS
+//      transpose reads; o = e^g q^ S + P v_new for the wave's columns (causal tiles only), stored;
+//      then the next chunk's rows into LDS: W and q, which are free after M, and k into the other
+//      of two buffers, with the row norms (8-lane DPP sums), g's prefix sum (64-lane DPP scan),
+//      e^g and e^{g_last - g} (one wave).  Their global loads were issued a whole chunk before.
+// W, q and P lie in LDS in operand order (kpos): each half of a 32-deep product step's A operand is
+// one 16-byte read, with nothing to repack.  The kernel is bound by what its two waves per SIMD
+// issue and wait for; with W and P as hi | lo words (two reads and eight byte permutes an operand)
+// and a staging phase of its own between two more barriers it took 523 / 398 us (fp32 / bf16), now 505 / 387
+// (B = 8, T = 4096, H = 32; the bytes it moves take 365 / 257 us at the 5.2 TB/s of a large copy).
 // Precision: QH_GDN_FP32 carries W, S, P and v_new as bf16 hi/lo splits (hi*hi + hi*lo + lo*hi,
 // fp32 accumulation; products with the exact q, k take two terms); QH_GDN_BF16 uses the hi
 // parts only.  Norms, decays and the prefix sum are fp32.
@@ -54,8 +57,8 @@ constexpr int kC = 64;          // chunk (tokens)
 constexpr int kD = 128;         // head dimension
 constexpr int kThreads = 512;   // 8 waves
 constexpr int kQs = kD + 8;     // LDS row stride of the q / k stores, bf16 (16-byte aligned rows)
-constexpr int kRs = kD + 4;     // LDS row stride of the W store, words
-constexpr int kPs = kC + 4;     // LDS row stride of P, words
+constexpr int kWs = kD + 16;    // LDS row stride of operand-ordered W and q, bf16 (72 words: 16-byte reads conflict-free)
+constexpr int kPs = kC + 16;    // LDS row stride of operand-ordered P, bf16 (40 words)
 
 struct StateArgs {
   const uint16_t *q, *k;  // bf16 [B][T][H][D]
@@ -71,33 +74,6 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 
 __device__ __forceinline__ float bf16f(uint32_t h) { return __uint_as_float(h << 16); }
 
-// One chunk's inputs as read from global memory, per thread: the row segment (token t / 8,
-// columns 16 (t % 8) ..) of q, k and W, this wave's U tiles (MFMA result layout) and one gc
-// value per lane (every wave reads the same 64; wave 0 uses them).
-template <bool WU_F32, int RP>
-struct ChunkIn {
-  uint4 q[RP][2], k[RP][2];
-  uint4 w[RP][WU_F32 ? 4 : 2];
-  float u[4][4];
-  float gc;
-};
-
-// Per-lane element offsets of chunk 0 (a chunk adds 64 H D): the thread's first row segment
-// (token t / 8, or t / 8 + 32 r for its r-th), its wave's U / o tile elements (token 4 qd + e of
-// tile i is + (16 i + e) H D) and lane's gc.
-struct Offsets {
-  uint32_t row, tile, g;
-  uint32_t tok;  // H D: one token
-};
-
-__device__ __forceinline__ Offsets offsets(const StateArgs &a, int b, int h, int t, int wave, int lane) {
-  const int row = t >> 3, seg = t & 7, r16 = lane & 15, qd = lane >> 4;
-  const uint32_t tok = static_cast<uint32_t>(a.H) * kD;
-  const uint32_t seq = (static_cast<uint32_t>(b) * a.T * a.H + h) * kD;  // token 0 of the sequence
-  return {seq + row * tok + 16 * seg, seq + 4 * qd * tok + 16 * wave + r16,
-          static_cast<uint32_t>(b) * a.T * a.H + lane * a.H + h, tok};
-}
-
 // RAGGED: T need not be a multiple of the chunk.  Rows past T repeat row T - 1 with gc = 0 and a zero
 // decay factor in the state update; P is lower triangular, so they touch no row before them, and
 // they are not stored.
@@ -107,41 +83,9 @@ __device__ __forceinline__ uint32_t past_end(const StateArgs &a, int n, int row)
   return RAGGED ? static_cast<uint32_t>(max(n * kC + row - (a.T - 1), 0)) : 0u;
 }
 
-template <bool WU_F32, int RP, bool RAGGED>
-__device__ __forceinline__ void load_chunk(const StateArgs &a, const Offsets &of, int n, int row, int lane, ChunkIn<WU_F32, RP> &in) {
-  const uint32_t c0 = static_cast<uint32_t>(n) * kC * of.tok;
-#pragma unroll
-  for (int r = 0; r < RP; ++r) {
-    const uint32_t ri = of.row + c0 + static_cast<uint32_t>(32 * r) * of.tok - past_end<RAGGED>(a, n, row + 32 * r) * of.tok;
-    const uint4 *qp = reinterpret_cast<const uint4 *>(a.q + ri);
-    const uint4 *kp = reinterpret_cast<const uint4 *>(a.k + ri);
-    in.q[r][0] = qp[0];
-    in.q[r][1] = qp[1];
-    in.k[r][0] = kp[0];
-    in.k[r][1] = kp[1];
-    if constexpr (WU_F32) {
-      const uint4 *wp = reinterpret_cast<const uint4 *>(static_cast<const float *>(a.w) + ri);
-#pragma unroll
-      for (int x = 0; x < 4; ++x) in.w[r][x] = wp[x];
-    } else {
-      const uint4 *wp = reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.w) + ri);
-      in.w[r][0] = wp[0];
-      in.w[r][1] = wp[1];
-    }
-  }
-  const uint32_t ti = of.tile + c0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t ui = ti + static_cast<uint32_t>(16 * i + e) * of.tok - past_end<RAGGED>(a, n, 16 * i + 4 * (lane >> 4) + e) * of.tok;
-      in.u[i][e] = WU_F32 ? static_cast<const float *>(a.u)[ui] : bf16f(static_cast<const uint16_t *>(a.u)[ui]);
-    }
-  }
-  const uint32_t back = past_end<RAGGED>(a, n, lane);
-  in.gc = a.g[of.g + (static_cast<uint32_t>(n) * kC - back) * static_cast<uint32_t>(a.H)];
-  if (RAGGED && back) in.gc = 0.0f;
-}
+// Position of column c of a row in operand order: within 32 columns, the 4 that a lane quarter takes of
+// the first 16 and the 4 it takes of the last 16 lie side by side (8 k of one lane, 16 bytes).
+__device__ __forceinline__ constexpr int kpos(int c) { return (c & ~31) + 8 * ((c >> 2) & 3) + 4 * ((c >> 4) & 1) + (c & 3); }
 
 // 8 bf16 values of a uint4 as floats.
 __device__ __forceinline__ void unbf16x8(const uint4 v, float *f) {
@@ -175,40 +119,11 @@ __device__ __forceinline__ Half4 bf16x4_tr(const uint16_t *p) {
   const uint2 v = __builtin_bit_cast(uint2, r);
   return exact4(v.x, v.y);
 }
-// 16 values of a W row into LDS: hi | lo words with SPLIT (a bf16 W is exact: the hi part only), else
-// bf16 (a float32 W rounded).
-template <bool SPLIT, bool WU_F32, class LW>
-__device__ __forceinline__ void stage_w(LW *dst, const uint4 (&w)[WU_F32 ? 4 : 2]) {
-  if constexpr (SPLIT) {
-    if constexpr (WU_F32) {
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-        *reinterpret_cast<uint4 *>(dst + 4 * x) =
-            make_uint4(hilo<SPLIT>(__uint_as_float(w[x].x)), hilo<SPLIT>(__uint_as_float(w[x].y)),
-                       hilo<SPLIT>(__uint_as_float(w[x].z)), hilo<SPLIT>(__uint_as_float(w[x].w)));
-    } else {
-#pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        const uint32_t w4[4] = {w[x].x, w[x].y, w[x].z, w[x].w};
-        *reinterpret_cast<uint4 *>(dst + 8 * x) = make_uint4(w4[0] & 0xFFFFu, w4[0] >> 16, w4[1] & 0xFFFFu, w4[1] >> 16);
-        *reinterpret_cast<uint4 *>(dst + 8 * x + 4) = make_uint4(w4[2] & 0xFFFFu, w4[2] >> 16, w4[3] & 0xFFFFu, w4[3] >> 16);
-      }
-    }
-  } else {
-    if constexpr (WU_F32) {
-#pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        const uint4 lo = w[2 * x], hi = w[2 * x + 1];
-        *reinterpret_cast<uint4 *>(dst + 8 * x) =
-            make_uint4(pack_bf16(__uint_as_float(lo.x), __uint_as_float(lo.y)), pack_bf16(__uint_as_float(lo.z), __uint_as_float(lo.w)),
-                       pack_bf16(__uint_as_float(hi.x), __uint_as_float(hi.y)), pack_bf16(__uint_as_float(hi.z), __uint_as_float(hi.w)));
-      }
-    } else {
-      *reinterpret_cast<uint4 *>(dst) = w[0];
-      *reinterpret_cast<uint4 *>(dst + 8) = w[1];
-    }
-  }
+__device__ __forceinline__ v4f mfma(const v8bf a, const v8bf b, const v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+// A operand half of one 32-deep step in operand order.
+__device__ __forceinline__ v8bf op8(const uint16_t *p) { return __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4 *>(p)); }
 
 // One 16 x 16 result tile of o: `at` is the element offset of the lane's column in row 4 qd of the
 // tile, tok the elements per token, qq the lane's place in its quad; rows: how many of the lane's 4
@@ -241,19 +156,16 @@ __device__ __forceinline__ void store_o(void *o, uint32_t at, uint32_t tok, int 
 
 template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
-  constexpr int RP = 8 * 64 / kThreads;  // row segments (16 columns of one token) per thread in L
+  constexpr bool kWlo = SPLIT && WU_F32;  // a bf16 W has no lo part
   // q, k rows as given (bf16, exact MFMA operands) with their l2norm factors; W and the lower
-  // tiles of P as hi | lo words with SPLIT, as bf16 (hi) without; g, e^g, e^{g_last - g}
-  using LW = std::conditional_t<SPLIT, uint32_t, uint16_t>;
-  constexpr int kWs = SPLIT ? kRs : kQs;     // W row stride, elements
-  constexpr int kPs2 = SPLIT ? kPs : kC + 8;  // P row stride, elements (bf16: 36 words, 8-byte reads conflict-free)
-  __shared__ __attribute__((aligned(16))) uint16_t Ql[kC][kQs];
-  __shared__ __attribute__((aligned(16))) uint16_t Kl[kC][kQs];
-  __shared__ __attribute__((aligned(16))) LW Wl[kC][kWs];
-  __shared__ __attribute__((aligned(16))) LW Pl[kC][kPs2];
-  __shared__ float invq[kC], invk[kC];  // 1 / |q| / sqrt(D), 1 / |k| (eps 1e-6 inside the root)
-  __shared__ float gl[kC], egl[kC], decl[kC];
-  __shared__ float eglast;
+  // tiles of P as bf16 hi parts (and lo parts with SPLIT); g, e^g, e^{g_last - g}
+  __shared__ __attribute__((aligned(16))) uint16_t Ql[kC][kWs];
+  __shared__ __attribute__((aligned(16))) uint16_t Kl[2][kC][kQs];
+  __shared__ __attribute__((aligned(16))) uint16_t Wh[kC][kWs], Wo[kWlo ? kC : 1][kWs];
+  __shared__ __attribute__((aligned(16))) uint16_t Ph[kC][kPs], Po[SPLIT ? kC : 1][kPs];
+  // 1 / |q| / sqrt(D), 1 / |k| (eps 1e-6 inside the root); g, e^g, e^{g_last - g}
+  __shared__ __attribute__((aligned(16))) float invq[2][kC], invk[2][kC], gl[2][kC], egl[2][kC], decl[2][kC];
+  __shared__ float eglast[2];
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int r16 = lane & 15, qd = lane >> 4;
@@ -269,156 +181,194 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
       S[kb][e] = a.s_in ? a.s_in[sbase + static_cast<size_t>(16 * kb + 4 * qd + e) * kD + 16 * wave + r16] : 0.0f;
   }
 
-  const Offsets of = offsets(a, b, h, t, wave, lane);
-  ChunkIn<WU_F32, RP> in;
-  load_chunk<WU_F32, RP, RAGGED>(a, of, 0, t >> 3, lane, in);
+  // Element offsets of chunk 0 (a chunk adds 64 H D).  A thread stages 16 columns of one row: of q and
+  // k columns 16 seg .., of W the 8 columns 32 (seg / 2) + 8 (seg % 2) .. and the 8 that are 16 further
+  // on, which are adjacent in operand order.
+  const uint32_t tok = static_cast<uint32_t>(a.H) * kD;
+  const uint32_t head = (static_cast<uint32_t>(b) * a.T * a.H + h) * kD;
+  const int row = t >> 3, seg = t & 7, wcol = 32 * (seg >> 1) + 8 * (seg & 1);
+  const uint32_t of_row = head + row * tok + 16 * seg, of_w = head + row * tok + wcol;
+  const uint32_t of_tile = head + 4 * qd * tok + 16 * wave + r16;
+  const uint32_t of_g = static_cast<uint32_t>(b) * a.T * a.H + lane * a.H + h;
 
-  auto chunk = [&](const int n) __attribute__((always_inline)) {
-    // ---- L: q, k, W into LDS; norms; g, e^g, e^{g_last - g} ------------------------------------
+  uint4 iq[2], ik[2], iw[2][WU_F32 ? 2 : 1];
+  float iu[4][4], igc;
+  auto load = [&](int n) __attribute__((always_inline)) {
+    const uint32_t c0 = static_cast<uint32_t>(n) * kC * tok, back = past_end<RAGGED>(a, n, row) * tok;
+    const uint4 *qp = reinterpret_cast<const uint4 *>(a.q + (of_row + c0 - back));
+    const uint4 *kp = reinterpret_cast<const uint4 *>(a.k + (of_row + c0 - back));
+    iq[0] = qp[0];
+    iq[1] = qp[1];
+    ik[0] = kp[0];
+    ik[1] = kp[1];
 #pragma unroll
-    for (int rp = 0; rp < RP; ++rp) {
-      const int row = (t >> 3) + 32 * rp, seg = t & 7;
-      *reinterpret_cast<uint4 *>(&Ql[row][16 * seg]) = in.q[rp][0];
-      *reinterpret_cast<uint4 *>(&Ql[row][16 * seg + 8]) = in.q[rp][1];
-      *reinterpret_cast<uint4 *>(&Kl[row][16 * seg]) = in.k[rp][0];
-      *reinterpret_cast<uint4 *>(&Kl[row][16 * seg + 8]) = in.k[rp][1];
-      float f[16];
-      unbf16x8(in.q[rp][0], f);
-      unbf16x8(in.q[rp][1], f + 8);
-      float ss = 0.0f;
-#pragma unroll
-      for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
-      ss = sum8(ss);
-      if (seg == 0) invq[row] = (1.0f / sqrtf(ss + 1e-6f)) * (1.0f / 11.313708498984761f);  // then 1/sqrt(128)
-      unbf16x8(in.k[rp][0], f);
-      unbf16x8(in.k[rp][1], f + 8);
-      ss = 0.0f;
-#pragma unroll
-      for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
-      ss = sum8(ss);
-      if (seg == 0) invk[row] = 1.0f / sqrtf(ss + 1e-6f);
-      stage_w<SPLIT, WU_F32>(&Wl[row][16 * seg], in.w[rp]);
+    for (int x = 0; x < 2; ++x) {
+      const uint32_t wi = of_w + c0 - back + 16 * x;
+      const uint4 *wp = WU_F32 ? reinterpret_cast<const uint4 *>(static_cast<const float *>(a.w) + wi)
+                               : reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.w) + wi);
+      iw[x][0] = wp[0];
+      if constexpr (WU_F32) iw[x][1] = wp[1];
     }
-    {
-      if (wave == 0) {
-        const float g = scan64(in.gc);
-        const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), 63));
-        gl[lane] = g;
-        egl[lane] = expf(g);
-        decl[lane] = RAGGED && n * kC + lane >= a.T ? 0.0f : expf(glast - g);
-        if (lane == 0) eglast = expf(glast);
-      }
-    }
-    float u[4][4];
+    const uint32_t gb = past_end<RAGGED>(a, n, lane);
+    igc = a.g[of_g + (static_cast<uint32_t>(n) * kC - gb) * static_cast<uint32_t>(a.H)];
+    if (RAGGED && gb) igc = 0.0f;
+  };
+  auto load_u = [&](int n) __attribute__((always_inline)) {
+    const uint32_t ti = of_tile + static_cast<uint32_t>(n) * kC * tok;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) u[i][e] = in.u[i][e];
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t ui = ti + static_cast<uint32_t>(16 * i + e) * tok - past_end<RAGGED>(a, n, 16 * i + 4 * qd + e) * tok;
+        iu[i][e] = WU_F32 ? static_cast<const float *>(a.u)[ui] : bf16f(static_cast<const uint16_t *>(a.u)[ui]);
+      }
     }
-    lds_barrier();
-    // Unconditional (the last chunk reloads itself, unused): behind a branch the compiler would
-    // lose count of the loads in flight and make the next chunk wait for every memory operation,
-    // this chunk's o stores included, instead of just these loads.
-    load_chunk<WU_F32, RP, RAGGED>(a, of, min(n + 1, a.nchunks - 1), t >> 3, lane, in);
-
-    // ---- M: W S, q^ S, v_new; P tiles ----------------------------------------------------------
-    Half4 sB[8];
+  };
+  // chunk n's rows into LDS (buffer n & 1 of the double-buffered arrays), with the norms and decays
+  auto stage = [&](int n) __attribute__((always_inline)) {
+    const int bf = n & 1;
+    uint16_t *const qd4 = &Ql[row][32 * (seg >> 1) + 4 * (seg & 1)];  // kpos(16 seg); 4 columns on: + 8
+    *reinterpret_cast<uint2 *>(qd4) = make_uint2(iq[0].x, iq[0].y);
+    *reinterpret_cast<uint2 *>(qd4 + 8) = make_uint2(iq[0].z, iq[0].w);
+    *reinterpret_cast<uint2 *>(qd4 + 16) = make_uint2(iq[1].x, iq[1].y);
+    *reinterpret_cast<uint2 *>(qd4 + 24) = make_uint2(iq[1].z, iq[1].w);
+    *reinterpret_cast<uint4 *>(&Kl[bf][row][16 * seg]) = ik[0];
+    *reinterpret_cast<uint4 *>(&Kl[bf][row][16 * seg + 8]) = ik[1];
+    float f[16];
+    unbf16x8(iq[0], f);
+    unbf16x8(iq[1], f + 8);
+    float ss = 0.0f;
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb) sB[kb] = split4<SPLIT>(S[kb]);
+    for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
+    ss = sum8(ss);
+    if (seg == 0) invq[bf][row] = (1.0f / sqrtf(ss + 1e-6f)) * (1.0f / 11.313708498984761f);  // then 1/sqrt(128)
+    unbf16x8(ik[0], f);
+    unbf16x8(ik[1], f + 8);
+    ss = 0.0f;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
+    ss = sum8(ss);
+    if (seg == 0) invk[bf][row] = 1.0f / sqrtf(ss + 1e-6f);
+    // W: two lane quarters' 8 values, 4 of each 16-column block
+    uint16_t *const wd = &Wh[row][kpos(wcol)];
+    if constexpr (WU_F32) {
+      Half4 x[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          x[i][j] = split4<SPLIT>(__uint_as_float(iw[i][j].x), __uint_as_float(iw[i][j].y), __uint_as_float(iw[i][j].z),
+                                  __uint_as_float(iw[i][j].w));
+      }
+      *reinterpret_cast<uint4 *>(wd) = make_uint4(x[0][0].h01, x[0][0].h23, x[1][0].h01, x[1][0].h23);
+      *reinterpret_cast<uint4 *>(wd + 8) = make_uint4(x[0][1].h01, x[0][1].h23, x[1][1].h01, x[1][1].h23);
+      if constexpr (kWlo) {
+        uint16_t *const wl = &Wo[row][kpos(wcol)];
+        *reinterpret_cast<uint4 *>(wl) = make_uint4(x[0][0].l01, x[0][0].l23, x[1][0].l01, x[1][0].l23);
+        *reinterpret_cast<uint4 *>(wl + 8) = make_uint4(x[0][1].l01, x[0][1].l23, x[1][1].l01, x[1][1].l23);
+      }
+    } else {
+      *reinterpret_cast<uint4 *>(wd) = make_uint4(iw[0][0].x, iw[0][0].y, iw[1][0].x, iw[1][0].y);
+      *reinterpret_cast<uint4 *>(wd + 8) = make_uint4(iw[0][0].z, iw[0][0].w, iw[1][0].z, iw[1][0].w);
+    }
+    if (wave == 0) {
+      const float g = scan64(igc);
+      const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), 63));
+      gl[bf][lane] = g;
+      egl[bf][lane] = expf(g);
+      decl[bf][lane] = RAGGED && n * kC + lane >= a.T ? 0.0f : expf(glast - g);
+      if (lane == 0) eglast[bf] = expf(glast);
+    }
+  };
+
+  load(0);
+  load_u(0);
+  // the upper tiles of P that a 32-deep step reads beside a diagonal one stay zero
+  for (int x = t; x < kC * kPs / 2; x += kThreads) {
+    reinterpret_cast<uint32_t *>(Ph)[x] = 0u;
+    if constexpr (SPLIT) reinterpret_cast<uint32_t *>(Po)[x] = 0u;
+  }
+  stage(0);
+  load(min(1, a.nchunks - 1));
+  lds_barrier();
+
+  auto chunk = [&](const int n) __attribute__((always_inline)) {
+    const int bf = n & 1;
+    // ---- M: W S, q^ S, v_new; P tiles ----------------------------------------------------------
+    v8bf sh[4], sl[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const Half4 s0 = split4<SPLIT>(S[2 * p]), s1 = split4<SPLIT>(S[2 * p + 1]);
+      sh[p] = op_hi(s0, s1);
+      sl[p] = op_lo(s0, s1);
+    }
     v4f ws[4], qs[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) ws[i] = qs[i] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int p = 0; p < 4; ++p) {  // key blocks 2p, 2p + 1: 8 independent accumulations
-      const int c = 32 * p + 4 * qd;
+      const int c = 32 * p + 8 * qd;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const LW *wrow = Wl[16 * i + r16];
-        const uint16_t *qrow = Ql[16 * i + r16];
-        Half4 w0, w1;
+        const v8bf w = op8(&Wh[16 * i + r16][c]), q = op8(&Ql[16 * i + r16][c]);
+        ws[i] = mfma(w, sh[p], ws[i]);
+        qs[i] = mfma(q, sh[p], qs[i]);
         if constexpr (SPLIT) {
-          w0 = unpack4(*reinterpret_cast<const uint4 *>(wrow + c));
-          w1 = unpack4(*reinterpret_cast<const uint4 *>(wrow + c + 16));
-        } else {
-          w0 = bf16x4(wrow + c);
-          w1 = bf16x4(wrow + c + 16);
+          ws[i] = mfma(w, sl[p], ws[i]);
+          qs[i] = mfma(q, sl[p], qs[i]);
         }
-        ws[i] = WU_F32 ? mma<SPLIT>(w0, w1, sB[2 * p], sB[2 * p + 1], ws[i])
-                       : mma_exact_a<SPLIT>(w0, w1, sB[2 * p], sB[2 * p + 1], ws[i]);
-        qs[i] = mma_exact_a<SPLIT>(bf16x4(qrow + c), bf16x4(qrow + c + 16), sB[2 * p], sB[2 * p + 1], qs[i]);
+        if constexpr (kWlo) ws[i] = mfma(op8(&Wo[16 * i + r16][c]), sh[p], ws[i]);
       }
     }
     v4f vnew[4], oacc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+      const v4f iq4 = *reinterpret_cast<const v4f *>(&invq[bf][16 * i + 4 * qd]);
+      const v4f eg4 = *reinterpret_cast<const v4f *>(&egl[bf][16 * i + 4 * qd]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int row = 16 * i + 4 * qd + e;
-        vnew[i][e] = u[i][e] - ws[i][e];
-        oacc[i][e] = qs[i][e] * (invq[row] * egl[row]);
+        vnew[i][e] = iu[i][e] - ws[i][e];
+        oacc[i][e] = qs[i][e] * (iq4[e] * eg4[e]);
       }
     }
-    for (int idx = wave; idx < 10; idx += kThreads / 64) {  // wave-uniform
+    load_u(min(n + 1, a.nchunks - 1));
+    for (int idx = kThreads / 64 - 1 - wave; idx < 10; idx += kThreads / 64) {  // wave-uniform
       int ti, tj;
       p_tile(idx, ti, tj);
       v4f acc = {0.f, 0.f, 0.f, 0.f};
-      const uint16_t *qrow = Ql[16 * ti + r16];
-      const uint16_t *krow = Kl[16 * tj + r16];
+      const uint16_t *krow = Kl[bf][16 * tj + r16];
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         const int c = 32 * p + 4 * qd;
-        acc = mma<false>(bf16x4(qrow + c), bf16x4(qrow + c + 16), bf16x4(krow + c), bf16x4(krow + c + 16), acc);
+        acc = mfma(op8(&Ql[16 * ti + r16][32 * p + 8 * qd]), op_hi(bf16x4(krow + c), bf16x4(krow + c + 16)), acc);
       }
       const int col = 16 * tj + r16;
-      const float kf = invk[col];
+      const float kf = invk[bf][col], gc = gl[bf][col];
+      const v4f iq4 = *reinterpret_cast<const v4f *>(&invq[bf][16 * ti + 4 * qd]);
+      const v4f gr4 = *reinterpret_cast<const v4f *>(&gl[bf][16 * ti + 4 * qd]);
+      const int pc = kpos(col);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int row = 16 * ti + 4 * qd + e;
-        const float pv = col <= row ? acc[e] * (invq[row] * kf) * expf(gl[row] - gl[col]) : 0.0f;
-        Pl[row][col] = static_cast<LW>(hilo<SPLIT>(pv));
+        const int rw = 16 * ti + 4 * qd + e;
+        const uint32_t pv = hilo<SPLIT>(col <= rw ? acc[e] * (iq4[e] * kf) * expf(gr4[e] - gc) : 0.0f);
+        Ph[rw][pc] = static_cast<uint16_t>(pv);
+        if constexpr (SPLIT) Po[rw][pc] = static_cast<uint16_t>(pv >> 16);
       }
     }
     lds_barrier();
 
-    // ---- O: o = e^g q^ S + P v_new (causal pairs of token tiles) -------------------------------
-    Half4 vB[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) vB[j] = split4<SPLIT>(vnew[j]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v4f acc = oacc[i];
-      const LW *prow = Pl[16 * i + r16];
-#pragma unroll
-      for (int p = 0; p <= i / 2; ++p) {
-        const bool two = 2 * p + 1 <= i;
-        const int c = 32 * p + 4 * qd;
-        Half4 p0, p1 = kZero4;
-        if constexpr (SPLIT) {
-          p0 = unpack4(*reinterpret_cast<const uint4 *>(prow + c));
-          if (two) p1 = unpack4(*reinterpret_cast<const uint4 *>(prow + c + 16));
-        } else {
-          p0 = bf16x4(prow + c);
-          if (two) p1 = bf16x4(prow + c + 16);
-        }
-        acc = mma<SPLIT>(p0, p1, vB[2 * p], two ? vB[2 * p + 1] : kZero4, acc);
-      }
-      store_o<OUT_F32, RAGGED>(a.o, of.tile + static_cast<uint32_t>(n * kC + 16 * i) * of.tok, of.tok, r16 & 3, acc,
-                               a.T - (n * kC + 16 * i + 4 * qd));
-    }
-
-    // ---- S: S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new) -------------------------------
+    // ---- N: S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new) --------------------------------
     Half4 dB[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      const v4f de4 = *reinterpret_cast<const v4f *>(&decl[bf][16 * j + 4 * qd]);
+      const v4f ik4 = *reinterpret_cast<const v4f *>(&invk[bf][16 * j + 4 * qd]);
       v4f d;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = 16 * j + 4 * qd + e;
-        d[e] = vnew[j][e] * (decl[row] * invk[row]);
-      }
+      for (int e = 0; e < 4; ++e) d[e] = vnew[j][e] * (de4[e] * ik4[e]);
       dB[j] = split4<SPLIT>(d);
     }
-    const float el = eglast;
+    const float el = eglast[bf];
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb) {
 #pragma unroll
@@ -433,15 +383,40 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
       const int c = 32 * p + 4 * qd;
 #pragma unroll
       for (int kb = 0; kb < 8; ++kb) {
-        S[kb] = mma_exact_a<SPLIT>(bf16x4_tr(&Kl[c + te][16 * kb + 4 * ka]), bf16x4_tr(&Kl[c + 16 + te][16 * kb + 4 * ka]),
+        S[kb] = mma_exact_a<SPLIT>(bf16x4_tr(&Kl[bf][c + te][16 * kb + 4 * ka]), bf16x4_tr(&Kl[bf][c + 16 + te][16 * kb + 4 * ka]),
                                    dB[2 * p], dB[2 * p + 1], S[kb]);
       }
     }
-    lds_barrier();  // the next chunk overwrites q, k, W, P and the decays
+    // ---- o = e^g q^ S + P v_new (causal pairs of token tiles) ------------------------------------
+    Half4 vB[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) vB[j] = split4<SPLIT>(vnew[j]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v4f acc = oacc[i];
+#pragma unroll
+      for (int p = 0; p <= i / 2; ++p) {
+        // (no later tile's v_new beside a diagonal tile: an infinity there would reach these rows)
+        const Half4 v1 = 2 * p + 1 <= i ? vB[2 * p + 1] : kZero4;
+        const v8bf ph = op8(&Ph[16 * i + r16][32 * p + 8 * qd]), vh = op_hi(vB[2 * p], v1);
+        acc = mfma(ph, vh, acc);
+        if constexpr (SPLIT) {
+          acc = mfma(ph, op_lo(vB[2 * p], v1), acc);
+          acc = mfma(op8(&Po[16 * i + r16][32 * p + 8 * qd]), vh, acc);
+        }
+      }
+      store_o<OUT_F32, RAGGED>(a.o, of_tile + static_cast<uint32_t>(n * kC + 16 * i) * tok, tok, r16 & 3, acc,
+                               a.T - (n * kC + 16 * i + 4 * qd));
+    }
+    // ---- the next chunk's rows.  Unconditional (the last chunk stages and loads itself again,
+    // unused): behind a branch the compiler would lose count of the loads in flight and wait for every
+    // memory operation, the o stores included.
+    stage(n + 1);
+    load(min(n + 2, a.nchunks - 1));
+    lds_barrier();
   };
   // Chunk 0 runs on its own: then every path into the loop has the same memory operations in
-  // flight (the next chunk's loads, then this chunk's o stores), and the compiler's wait before
-  // the first use of the loads counts only them.
+  // flight, and the compiler's wait before the first use of the loads counts only them.
   chunk(0);
   for (int n = 1; n < a.nchunks; ++n) chunk(n);
 

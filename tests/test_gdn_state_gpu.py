@@ -350,3 +350,22 @@ def test_ragged_prefill_takes_strided_and_unaligned_inputs(gpu):
     strided = torch.stack((v, v), dim=-1)[..., 0]
     got = gdn_prefill(q, odd, strided, torch.stack((g, g), dim=-1)[..., 0], bt)
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("H", [2, 80], ids=["few_sequences", "many_sequences"])
+@pytest.mark.parametrize("token", [16, 47, 100])
+def test_state_infinity_stays_behind_its_tile(gpu, token, H, precision):
+    """An infinite U at one token reaches no output of an earlier 16-token tile (P is lower triangular)."""
+    import torch
+
+    from qcom_htp_amd.gdn import gdn_chunk_state, gdn_chunk_uw
+
+    q, k, v, bt, g = (to_dev(x, gpu) for x in seq_inputs(1, 128, H, seed=token))
+    w, u = gdn_chunk_uw(k, v, g, bt, 64, decay_w=True, out_dtype=torch.float32)
+    want, _ = gdn_chunk_state(q, k, g, w, u, None, precision)
+    u[:, token] = float("inf")
+    got, _ = gdn_chunk_state(q, k, g, w, u, None, precision)
+    first = token // 16 * 16
+    assert torch.equal(got[:, :first], want[:, :first])
+    assert not torch.isfinite(got[:, token]).all()
