@@ -338,6 +338,16 @@ qh_status qh_gdn_chunk_state(const uint16_t *q_dev, const uint16_t *k_dev, const
                              uint32_t tokens, uint32_t heads, uint32_t head_dim, uint32_t chunk, uint32_t flags,
                              uint32_t precision, void *stream);
 
+/* The same with a device workspace (16-byte aligned) of qh_gdn_chunk_state_workspace bytes, in which
+ * few sequences' chunk-local operands are formed for all chunks at once before the recurrence; NULL,
+ * or fewer bytes, leaves them to the recurrence.  The results are the same bit for bit.  The query
+ * returns 0 for shapes that use none. */
+size_t qh_gdn_chunk_state_workspace(uint32_t batch, uint32_t tokens, uint32_t heads, uint32_t precision);
+qh_status qh_gdn_chunk_state_ws(const uint16_t *q_dev, const uint16_t *k_dev, const float *g_dev, const void *w_dev,
+                                const void *u_dev, const float *s_in_dev, float *s_out_dev, void *o_dev, uint32_t batch,
+                                uint32_t tokens, uint32_t heads, uint32_t head_dim, uint32_t chunk, uint32_t flags,
+                                uint32_t precision, void *workspace_dev, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -81,6 +81,8 @@ EXPORTED = (
     "qh_gdn_chunk_uw",
     "qh_gdn_chunk_uw_ex",
     "qh_gdn_chunk_state",
+    "qh_gdn_chunk_state_workspace",
+    "qh_gdn_chunk_state_ws",
 )
 
 
@@ -177,6 +179,10 @@ def _declare(L: C.CDLL) -> None:
     L.qh_gdn_chunk_uw_ex.restype = st
     L.qh_gdn_chunk_state.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, u32, u32, u32, u32, u32, u32, u32, vp]
     L.qh_gdn_chunk_state.restype = st
+    L.qh_gdn_chunk_state_workspace.argtypes = [u32, u32, u32, u32]
+    L.qh_gdn_chunk_state_workspace.restype = C.c_size_t
+    L.qh_gdn_chunk_state_ws.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, u32, u32, u32, u32, u32, u32, u32, vp, C.c_size_t, vp]
+    L.qh_gdn_chunk_state_ws.restype = st
 
 
 def lib() -> C.CDLL:

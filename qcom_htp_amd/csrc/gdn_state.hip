@@ -33,14 +33,17 @@
 
 //
 // Few sequences (gdn_state_cols_kernel): the chunks of a sequence follow one another, so the launch
-// lasts as long as one sequence however few there are, and what counts is a chunk's latency.  A lone
-// wave issues one vector instruction every 5 ns or so whatever it is, so that latency is the
-// instructions of one wave: the work of a chunk is spread over 16 waves and, since v_new, o and S act
-// on value columns independently, over 128 / (16 CT) workgroups of CT column tiles each.  A column
-// tile's waves share its S by key blocks; S, v_new and the state update's operand go through LDS as
-// the records that the next products read as they are.  The next chunk's rows go into LDS behind the
-// state update (q and W are free after the products, k has two buffers), and their global loads are
-// issued a whole chunk ahead.
+// lasts as long as one sequence however few there are, and what counts is a chunk's latency.  The work
+// of a chunk is spread over 16 waves and, since v_new, o and S act on value columns independently, over
+// 128 / (16 CT) workgroups of CT column tiles each.  A column tile's waves share its S by key blocks; S,
+// v_new and the state update's operand go through LDS as the records that the next products read as
+// they are.  The next chunk's rows go into LDS behind the state update (q and W are free after the
+// products, k has two buffers), and their global loads are issued a whole chunk ahead.  With a
+// workspace, what a chunk needs besides the state (gdn_state_pre_kernel) is formed for all chunks first,
+// and the recurrence only copies it.  A chunk of 16 sequences then takes 1.6 / 2.2 us (bf16 / fp32)
+// against 3.1 / 3.8 us, and some 6 us before the first; its bounds are the LDS reads of a workgroup
+// (16 CT columns of S by 8 waves each) and the chain of products behind two barriers.
+// Stages A and B of T = 4096 x 16 sequences: bf16 212 -> 120 us, fp32 252 -> 158 us.
 
 #include <type_traits>
 
@@ -68,7 +71,12 @@ struct StateArgs {
   float *s_out;           // [B][H][D][D]
   void *o;                // [B][T][H][D] bf16 or fp32
   int B, T, H, nchunks;
+  // what gdn_state_pre_kernel formed of every (sequence, chunk), in order: P as [64][64] bf16 hi parts
+  // (then lo parts with SPLIT), and kPreF floats (the factors of q^ S's and v_new's rows, e^{g_last})
+  uint16_t *pre_p;
+  float *pre_f;
 };
+constexpr int kPreF = 2 * kC + 4;
 
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -97,7 +105,21 @@ __device__ __forceinline__ void unbf16x8(const uint4 v, float *f) {
   }
 }
 
-// The 10 lower 16 x 16 tiles of P (token tile i >= j), two for waves 0 and 1.
+// Sum of the squares of a row's 128 values, 16 in each of 8 adjacent lanes.
+__device__ __forceinline__ float row_square(const uint4 (&v)[2]) {
+  float f[16];
+  unbf16x8(v[0], f);
+  unbf16x8(v[1], f + 8);
+  float ss = 0.0f;
+#pragma unroll
+  for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
+  return sum8(ss);
+}
+// 1 / |q| / sqrt(D) and 1 / |k| of a sum of squares (eps 1e-6 inside the root).
+__device__ __forceinline__ float inv_k(float ss) { return 1.0f / sqrtf(ss + 1e-6f); }
+__device__ __forceinline__ float inv_q(float ss) { return inv_k(ss) * (1.0f / 11.313708498984761f); }
+
+// The 10 lower 16 x 16 tiles of P (token tile i >= j).
 __device__ __forceinline__ void p_tile(int idx, int &i, int &j) {
   i = idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3;
   j = idx - i * (i + 1) / 2;
@@ -234,21 +256,11 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
     *reinterpret_cast<uint2 *>(qd4 + 24) = make_uint2(iq[1].z, iq[1].w);
     *reinterpret_cast<uint4 *>(&Kl[bf][row][16 * seg]) = ik[0];
     *reinterpret_cast<uint4 *>(&Kl[bf][row][16 * seg + 8]) = ik[1];
-    float f[16];
-    unbf16x8(iq[0], f);
-    unbf16x8(iq[1], f + 8);
-    float ss = 0.0f;
-#pragma unroll
-    for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
-    ss = sum8(ss);
-    if (seg == 0) invq[bf][row] = (1.0f / sqrtf(ss + 1e-6f)) * (1.0f / 11.313708498984761f);  // then 1/sqrt(128)
-    unbf16x8(ik[0], f);
-    unbf16x8(ik[1], f + 8);
-    ss = 0.0f;
-#pragma unroll
-    for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
-    ss = sum8(ss);
-    if (seg == 0) invk[bf][row] = 1.0f / sqrtf(ss + 1e-6f);
+    const float sq = row_square(iq), sk = row_square(ik);
+    if (seg == 0) {
+      invq[bf][row] = inv_q(sq);
+      invk[bf][row] = inv_k(sk);
+    }
     // W: two lane quarters' 8 values, 4 of each 16-column block
     uint16_t *const wd = &Wh[row][kpos(wcol)];
     if constexpr (WU_F32) {
@@ -428,24 +440,31 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
   }
 }
 
-// One sequence's value columns 16 CT s .. 16 CT s + 16 CT - 1.  Waves: column tile wave / WPC; its WPC
-// waves own 8 / WPC key blocks of S each.  With WPC = 8 there are two waves per token tile, one for
-// W S (and v_new), the other for q S (and o); with WPC = 4 one wave does both.  The sums are formed in
-// the order of gdn_state_kernel, so the results are the same bit for bit.
+// One sequence's value columns 16 CT s .. 16 CT s + 16 CT - 1.  The 8 waves of a column tile own one key
+// block of S each, and are two per token tile: one for W S (and v_new), the other for q S (and o).  All
+// 16 waves stage; with one column tile the last 8 do nothing else.  The sums are formed in the order of
+// gdn_state_kernel, so the results are the same bit for bit.
 constexpr int kColThreads = 1024;
-template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED, int CT>
+// Fewest chunks for which gdn_state_pre_kernel runs: stages A and B of 16 sequences of 4 chunks take 22.8
+// us (fp32) with it and 26.4 without; at 3 chunks and 64 sequences both take as long.
+constexpr int kPreChunks = 3;
+//
+// PRE: P, the norms and the decays come from gdn_state_pre_kernel.
+template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED, int CT, bool PRE>
 __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a) {
-  constexpr int WPC = 16 / CT, KB = 8 / WPC;
-  constexpr bool kRoles = WPC == 8;        // W S and q S on different waves
+  static_assert(CT == 1 || CT == 2, "8 waves per column tile");
+  constexpr int kPB = PRE ? 2 : 1;         // buffers of P: formed and read in one chunk, or staged a chunk ahead
   constexpr bool kWlo = SPLIT && WU_F32;   // a bf16 W has no lo part
   constexpr int kPr = kC + 8;              // P row stride, bf16 (36 words: 8-byte reads conflict-free)
   using Rec = std::conditional_t<SPLIT, uint4, uint2>;  // 4 values as an operand: hi pairs (, lo pairs)
   __shared__ __attribute__((aligned(16))) uint16_t Ql[kC][kQs];
   __shared__ __attribute__((aligned(16))) uint16_t Kl[2][kC][kQs];
   __shared__ __attribute__((aligned(16))) uint16_t Wh[kC][kQs], Wo[kWlo ? kC : 1][kQs];
-  __shared__ __attribute__((aligned(16))) uint16_t Ph[kC][kPr], Po[SPLIT ? kC : 1][kPr];
+  __shared__ __attribute__((aligned(16))) uint16_t Ph[kPB][kC][kPr], Po[kPB][SPLIT ? kC : 1][kPr];
   __shared__ Rec Sr[CT][8][64], Vr[CT][4][64], Dr[CT][4][64];  // S, v_new, (e^{g_last - g} / |k|) v_new
-  __shared__ float invq[2][kC], invk[2][kC], gl[2][kC], egl[2][kC], decl[2][kC], eglast[2];
+  constexpr int kN = PRE ? 1 : kC;
+  __shared__ float invq[2][kN], invk[2][kN], gl[2][kN], egl[2][kN], decl[2][kN], eglast[2];
+  __shared__ __attribute__((aligned(16))) float pre[2][PRE ? kPreF : 4];
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int r16 = lane & 15, qd = lane >> 4;
@@ -454,9 +473,10 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
   const int k8 = blockIdx.x >> 3, slice = k8 % kSlices, seq = (blockIdx.x & 7) + 8 * (k8 / kSlices);
   if (seq >= a.B * a.H) return;  // uniform: before any barrier
   const int b = seq / a.H, h = seq % a.H;
-  const int ct = wave / WPC, wc = wave % WPC;
+  const bool owns = CT == 2 || wave < 8;  // has a key block and a token tile
+  const int ct = CT == 2 ? wave >> 3 : 0, wc = wave & 7;
   const int ti = wc & 3;                           // the wave's token tile
-  const bool do_w = !kRoles || wc < 4, do_q = !kRoles || wc >= 4;
+  const bool do_w = owns && wc < 4, do_q = owns && wc >= 4;
   const int gcol = 16 * (CT * slice + ct) + r16;   // value column
   auto put = [](Rec &r, const Half4 &x) __attribute__((always_inline)) {
     if constexpr (SPLIT) r = make_uint4(x.h01, x.h23, x.l01, x.l23);
@@ -467,14 +487,13 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
     else return exact4(r.x, r.y);
   };
 
-  v4f S[KB];  // key blocks KB wc .. : rows 16 kb + 4 qd + e, column gcol
-  const size_t sbase = static_cast<size_t>(seq) * kD * kD;
-#pragma unroll
-  for (int i = 0; i < KB; ++i) {
+  v4f S = {0.f, 0.f, 0.f, 0.f};  // key block wc: rows 16 wc + 4 qd + e, column gcol
+  const size_t sbase = static_cast<size_t>(seq) * kD * kD + static_cast<size_t>(16 * wc + 4 * qd) * kD + gcol;
+  if (owns) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      S[i][e] = a.s_in ? a.s_in[sbase + static_cast<size_t>(16 * (KB * wc + i) + 4 * qd + e) * kD + gcol] : 0.0f;
-    put(Sr[ct][KB * wc + i][lane], split4<SPLIT>(S[i]));
+      if (a.s_in) S[e] = a.s_in[sbase + static_cast<size_t>(e) * kD];
+    put(Sr[ct][wc][lane], split4<SPLIT>(S));
   }
   // element offsets of chunk 0 (a chunk adds 64 H D).  Waves 0..7 stage q, 8..15 k: 16 columns of a row
   // per thread; every wave W: 8 columns of a row per thread.
@@ -487,21 +506,30 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
   const uint32_t of_tile = head + (16 * ti + 4 * qd) * tok + gcol;
   const uint32_t of_g = static_cast<uint32_t>(b) * a.T * a.H + lane * a.H + h;
 
-  uint4 in[2], iw[WU_F32 ? 2 : 1];
-  float iu[4], igc;
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  v4u in0, in1;  // (vectors, not uint4: copied to LDS as they are, a struct goes through the stack)
+  uint4 iw[WU_F32 ? 2 : 1];
+  float iu[4], igc;  // igc: a token's log decay; PRE: one of the chunk's kPreF floats
+  v4u ip = {};       // PRE: 8 values of a row of P (waves 0..7 hi parts, 8..15 lo parts)
   auto load = [&](int n) __attribute__((always_inline)) {
     const uint32_t c0 = static_cast<uint32_t>(n) * kC * tok;
-    const uint4 *p = reinterpret_cast<const uint4 *>(qk + (of_row + c0 - past_end<RAGGED>(a, n, row) * tok));
-    in[0] = p[0];
-    in[1] = p[1];
+    const v4u *p = reinterpret_cast<const v4u *>(qk + (of_row + c0 - past_end<RAGGED>(a, n, row) * tok));
+    in0 = p[0];
+    in1 = p[1];
     const uint32_t wi = of_w + c0 - past_end<RAGGED>(a, n, wrow) * tok;
     const uint4 *wp = WU_F32 ? reinterpret_cast<const uint4 *>(static_cast<const float *>(a.w) + wi)
                              : reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.w) + wi);
     iw[0] = wp[0];
     if (WU_F32) iw[WU_F32 ? 1 : 0] = wp[1];
-    const uint32_t back = past_end<RAGGED>(a, n, lane);
-    igc = a.g[of_g + (static_cast<uint32_t>(n) * kC - back) * static_cast<uint32_t>(a.H)];
-    if (RAGGED && back) igc = 0.0f;
+    if constexpr (PRE) {
+      const size_t item = static_cast<size_t>(seq) * a.nchunks + n;
+      ip = *reinterpret_cast<const v4u *>(a.pre_p + (item * (SPLIT ? 2 : 1) + (SPLIT ? t >> 9 : 0)) * (kC * kC) + 8 * (t & 511));
+      igc = a.pre_f[item * kPreF + min(t, 2 * kC)];
+    } else {
+      const uint32_t back = past_end<RAGGED>(a, n, lane);
+      igc = a.g[of_g + (static_cast<uint32_t>(n) * kC - back) * static_cast<uint32_t>(a.H)];
+      if (RAGGED && back) igc = 0.0f;
+    }
   };
   auto load_u = [&](int n) __attribute__((always_inline)) {
     const uint32_t c0 = static_cast<uint32_t>(n) * kC * tok;
@@ -515,21 +543,16 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
   auto stage = [&](int n) __attribute__((always_inline)) {
     const int bf = n & 1;
     uint16_t *const d = is_q ? &Ql[row][16 * seg] : &Kl[bf][row][16 * seg];
-    *reinterpret_cast<uint4 *>(d) = in[0];
-    *reinterpret_cast<uint4 *>(d + 8) = in[1];
-    float f[16];
-    unbf16x8(in[0], f);
-    unbf16x8(in[1], f + 8);
-    float ss = 0.0f;
-#pragma unroll
-    for (int x = 0; x < 16; ++x) ss = fmaf(f[x], f[x], ss);
-    ss = sum8(ss);
-    if (seg == 0) {
-      const float r = 1.0f / sqrtf(ss + 1e-6f);
-      if (is_q)
-        invq[bf][row] = r * (1.0f / 11.313708498984761f);  // then 1/sqrt(128)
-      else
-        invk[bf][row] = r;
+    *reinterpret_cast<v4u *>(d) = in0;
+    *reinterpret_cast<v4u *>(d + 8) = in1;
+    if constexpr (!PRE) {
+      const float ss = row_square({__builtin_bit_cast(uint4, in0), __builtin_bit_cast(uint4, in1)});
+      if (seg == 0) {
+        if (is_q)
+          invq[bf][row] = inv_q(ss);
+        else
+          invk[bf][row] = inv_k(ss);
+      }
     }
     if constexpr (WU_F32) {
       const Half4 x = split4<SPLIT>(__uint_as_float(iw[0].x), __uint_as_float(iw[0].y), __uint_as_float(iw[0].z), __uint_as_float(iw[0].w));
@@ -540,7 +563,13 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
     } else {
       *reinterpret_cast<uint4 *>(&Wh[wrow][8 * wseg]) = iw[0];
     }
-    if (wave == 0) {  // (its token tile has no o to form)
+    if constexpr (PRE) {
+      if (SPLIT || wave < 8) {  // wave-uniform
+        const int pr = (t & 511) >> 3, pc = 8 * (t & 7);
+        *reinterpret_cast<v4u *>(SPLIT && wave >= 8 ? &Po[PRE ? bf : 0][SPLIT ? pr : 0][pc] : &Ph[PRE ? bf : 0][pr][pc]) = ip;
+      }
+      if (t <= 2 * kC) pre[bf][PRE ? t : 0] = igc;
+    } else if (wave == 0) {  // (its token tile has no o to form)
       const float g = scan64(igc);
       const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), 63));
       gl[bf][lane] = g;
@@ -557,10 +586,13 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
 
   auto chunk = [&](const int n) __attribute__((always_inline)) {
     const int bf = n & 1;
+    const int pb = PRE ? bf : 0;
     // ---- products: W S and q^ S of the wave's token tile, v_new; P tiles -------------------------
     Half4 sB[8];
+    if (owns) {
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb) sB[kb] = get(Sr[ct][kb][lane]);
+      for (int kb = 0; kb < 8; ++kb) sB[kb] = get(Sr[ct][kb][lane]);
+    }
     v4f oacc = {0.f, 0.f, 0.f, 0.f};
     if (do_w) {  // wave-uniform
       v4f ws = {0.f, 0.f, 0.f, 0.f};
@@ -579,7 +611,7 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
       for (int e = 0; e < 4; ++e) {
         const int rw = 16 * ti + 4 * qd + e;
         vn[e] = iu[e] - ws[e];
-        d[e] = vn[e] * (decl[bf][rw] * invk[bf][rw]);
+        d[e] = vn[e] * (PRE ? pre[bf][kC + rw] : decl[bf][rw] * invk[bf][rw]);
       }
       put(Vr[ct][ti][lane], split4<SPLIT>(vn));
       put(Dr[ct][ti][lane], split4<SPLIT>(d));
@@ -595,11 +627,13 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int rw = 16 * ti + 4 * qd + e;
-        oacc[e] = qs[e] * (invq[bf][rw] * egl[bf][rw]);
+        oacc[e] = qs[e] * (PRE ? pre[bf][rw] : invq[bf][rw] * egl[bf][rw]);
       }
     }
+    // (a load moved up across its registers' last use would have to be waited for and copied)
+    if constexpr (PRE) __builtin_amdgcn_sched_barrier(0);
     load_u(min(n + 1, a.nchunks - 1));
-    if (15 - wave < 10) {  // wave-uniform: one P tile on each of 10 waves
+    if (!PRE && 15 - wave < 10) {  // wave-uniform: one P tile on each of 10 waves
       int pi, pj;
       p_tile(15 - wave, pi, pj);
       v4f acc = {0.f, 0.f, 0.f, 0.f};
@@ -617,32 +651,26 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
         const int rw = 16 * pi + 4 * qd + e;
         const float pv = col <= rw ? acc[e] * (invq[bf][rw] * kf) * expf(gl[bf][rw] - gl[bf][col]) : 0.0f;
         const uint32_t w = hilo<SPLIT>(pv);
-        Ph[rw][col] = static_cast<uint16_t>(w);
-        if constexpr (SPLIT) Po[rw][col] = static_cast<uint16_t>(w >> 16);
+        Ph[pb][rw][col] = static_cast<uint16_t>(w);
+        if constexpr (SPLIT) Po[pb][rw][col] = static_cast<uint16_t>(w >> 16);
       }
     }
     lds_barrier();
 
-    // ---- S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new), the wave's key blocks --------------
-    const float el = eglast[bf];
+    // ---- S = e^{g_last} S + k^T ((e^{g_last - g} / |k|) v_new), the wave's key block ---------------
+    const float el = PRE ? pre[bf][2 * kC] : eglast[bf];
     const int te = r16 >> 2, ka = r16 & 3;
+    if (owns) {
 #pragma unroll
-    for (int i = 0; i < KB; ++i) {
+      for (int e = 0; e < 4; ++e) S[e] *= el;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[i][e] *= el;
-    }
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int c = 32 * p + 4 * qd;
-      const Half4 d0 = get(Dr[ct][2 * p][lane]), d1 = get(Dr[ct][2 * p + 1][lane]);
-#pragma unroll
-      for (int i = 0; i < KB; ++i) {
-        const int kc = 16 * (KB * wc + i) + 4 * ka;
-        S[i] = mma_exact_a<SPLIT>(bf16x4_tr(&Kl[bf][c + te][kc]), bf16x4_tr(&Kl[bf][c + 16 + te][kc]), d0, d1, S[i]);
+      for (int p = 0; p < 2; ++p) {
+        const int c = 32 * p + 4 * qd, kc = 16 * wc + 4 * ka;
+        S = mma_exact_a<SPLIT>(bf16x4_tr(&Kl[bf][c + te][kc]), bf16x4_tr(&Kl[bf][c + 16 + te][kc]), get(Dr[ct][2 * p][lane]),
+                               get(Dr[ct][2 * p + 1][lane]), S);
       }
+      put(Sr[ct][wc][lane], split4<SPLIT>(S));
     }
-#pragma unroll
-    for (int i = 0; i < KB; ++i) put(Sr[ct][KB * wc + i][lane], split4<SPLIT>(S[i]));
     // ---- o = e^g q^ S + P v_new ------------------------------------------------------------------
     if (do_q) {
       v4f acc = oacc;
@@ -651,13 +679,13 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
         if (p > ti / 2) continue;  // wave-uniform
         const bool two = 2 * p + 1 <= ti;
         const int c = 32 * p + 4 * qd;
-        Half4 p0 = bf16x4(&Ph[16 * ti + r16][c]), p1 = kZero4;
-        if (two) p1 = bf16x4(&Ph[16 * ti + r16][c + 16]);
+        Half4 p0 = bf16x4(&Ph[pb][16 * ti + r16][c]), p1 = kZero4;
+        if (two) p1 = bf16x4(&Ph[pb][16 * ti + r16][c + 16]);
         if constexpr (SPLIT) {
-          const Half4 l0 = bf16x4(&Po[16 * ti + r16][c]);
+          const Half4 l0 = bf16x4(&Po[pb][16 * ti + r16][c]);
           p0.l01 = l0.h01; p0.l23 = l0.h23;
           if (two) {
-            const Half4 l1 = bf16x4(&Po[16 * ti + r16][c + 16]);
+            const Half4 l1 = bf16x4(&Po[pb][16 * ti + r16][c + 16]);
             p1.l01 = l1.h01; p1.l23 = l1.h23;
           }
         }
@@ -667,23 +695,107 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
     }
     // ---- the next chunk's rows (the last chunk stages itself again, unused) -------------------------
     stage(n + 1);
+    if constexpr (PRE) __builtin_amdgcn_sched_barrier(0);
     load(min(n + 2, a.nchunks - 1));
     lds_barrier();
   };
-  for (int n = 0; n < a.nchunks; ++n) chunk(n);
+  if constexpr (PRE) chunk(0);  // on its own, for the wait counts (as in gdn_state_kernel)
+  for (int n = PRE ? 1 : 0; n < a.nchunks; ++n) chunk(n);
 
+  if (owns) {
 #pragma unroll
-  for (int i = 0; i < KB; ++i) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) a.s_out[sbase + static_cast<size_t>(16 * (KB * wc + i) + 4 * qd + e) * kD + gcol] = S[i][e];
+    for (int e = 0; e < 4; ++e) a.s_out[sbase + static_cast<size_t>(e) * kD] = S[e];
   }
+}
+
+// What a chunk needs besides the state, for every (sequence, chunk) at once: P, the row factors of q^ S
+// (e^g / |q| / sqrt(D)) and of v_new in the state update (e^{g_last - g} / |k|), e^{g_last}.  Left to
+// the recurrence, these are some 60 % of the instructions of a chunk of gdn_state_cols_kernel, repeated
+// by each of a sequence's workgroups, one chunk after another.
+template <bool SPLIT, bool RAGGED>
+__global__ __launch_bounds__(kThreads) void gdn_state_pre_kernel(StateArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t Ql[kC][kQs], Kl[kC][kQs];
+  __shared__ __attribute__((aligned(16))) float invq[kC], invk[kC], gl[kC];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int r16 = lane & 15, qd = lane >> 4;
+  const size_t item = blockIdx.x;
+  const int seq = blockIdx.x / a.nchunks, n = blockIdx.x % a.nchunks, b = seq / a.H, h = seq % a.H;
+  const uint32_t tok = static_cast<uint32_t>(a.H) * kD;
+  const int row = t >> 3, seg = t & 7;
+  const uint32_t at = (static_cast<uint32_t>(b) * a.T * a.H + h) * kD + 16 * seg +
+                      (static_cast<uint32_t>(n) * kC + row - past_end<RAGGED>(a, n, row)) * tok;
+  const uint4 *qp = reinterpret_cast<const uint4 *>(a.q + at), *kp = reinterpret_cast<const uint4 *>(a.k + at);
+  const uint4 iq[2] = {qp[0], qp[1]}, ik[2] = {kp[0], kp[1]};
+  float gc = 0.0f;
+  if (wave == 0) {
+    const uint32_t back = past_end<RAGGED>(a, n, lane);
+    gc = a.g[static_cast<uint32_t>(b) * a.T * a.H + h + (static_cast<uint32_t>(n) * kC + lane - back) * static_cast<uint32_t>(a.H)];
+    if (RAGGED && back) gc = 0.0f;
+  }
+  *reinterpret_cast<uint4 *>(&Ql[row][16 * seg]) = iq[0];
+  *reinterpret_cast<uint4 *>(&Ql[row][16 * seg + 8]) = iq[1];
+  *reinterpret_cast<uint4 *>(&Kl[row][16 * seg]) = ik[0];
+  *reinterpret_cast<uint4 *>(&Kl[row][16 * seg + 8]) = ik[1];
+  const float sq = row_square(iq), sk = row_square(ik);
+  if (seg == 0) {
+    invq[row] = inv_q(sq);
+    invk[row] = inv_k(sk);
+  }
+  const float g = scan64(gc);  // wave 0's counts
+  if (wave == 0) gl[lane] = g;
+  lds_barrier();
+  if (wave == 0) {
+    const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), 63));
+    float *const f = a.pre_f + item * kPreF;
+    f[lane] = invq[lane] * expf(g);
+    f[kC + lane] = (RAGGED && n * kC + lane >= a.T ? 0.0f : expf(glast - g)) * invk[lane];
+    if (lane == 0) f[2 * kC] = expf(glast);
+  }
+  uint16_t *const P = a.pre_p + item * (SPLIT ? 2 : 1) * (kC * kC);
+  for (int idx = kThreads / 64 - 1 - wave; idx < 10; idx += kThreads / 64) {  // wave-uniform
+    int ti, tj;
+    p_tile(idx, ti, tj);
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    const uint16_t *qrow = Ql[16 * ti + r16], *krow = Kl[16 * tj + r16];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int c = 32 * p + 4 * qd;
+      acc = mma<false>(bf16x4(qrow + c), bf16x4(qrow + c + 16), bf16x4(krow + c), bf16x4(krow + c + 16), acc);
+    }
+    const int col = 16 * tj + r16;
+    const float kf = invk[col];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int rw = 16 * ti + 4 * qd + e;
+      const uint32_t w = hilo<SPLIT>(col <= rw ? acc[e] * (invq[rw] * kf) * expf(gl[rw] - gl[col]) : 0.0f);
+      P[rw * kC + col] = static_cast<uint16_t>(w);
+      if constexpr (SPLIT) P[kC * kC + rw * kC + col] = static_cast<uint16_t>(w >> 16);
+    }
+  }
+}
+
+// Workgroups of the column-sliced kernel with CT column tiles each, or 0 where they would not all have a
+// compute unit of their own.  One tile where that fits (up to 32 sequences): 16 sequences of 4096 tokens
+// take 120 / 158 us (bf16 / fp32) with one tile, 153 / 191 with two.
+int cols_grid(int seqs, int ct) {
+  const int per8 = (seqs + 7) / 8 * 8, grid = per8 * (kD / (16 * ct));
+  return grid <= device_cu_count() ? grid : 0;
 }
 
 template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED>
 qh_status launch4(const StateArgs &a, hipStream_t stream) {
-  const int seqs = a.B * a.H, cus = device_cu_count(), per8 = (seqs + 7) / 8 * 8;
-  if (per8 * 4 <= cus)
-    hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, 2>), dim3(per8 * 4), dim3(kColThreads), 0, stream, a);
+  const int seqs = a.B * a.H, grid1 = cols_grid(seqs, 1), grid2 = cols_grid(seqs, 2);
+  if (grid2 && a.pre_p) {
+    hipLaunchKernelGGL((gdn_state_pre_kernel<SPLIT, RAGGED>), dim3(seqs * a.nchunks), dim3(kThreads), 0, stream, a);
+    hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return hip_fail(err, "gdn_state_pre_kernel launch");
+    if (grid1)
+      hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, 1, true>), dim3(grid1), dim3(kColThreads), 0, stream, a);
+    else
+      hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, 2, true>), dim3(grid2), dim3(kColThreads), 0, stream, a);
+  } else if (grid2)
+    hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, 2, false>), dim3(grid2), dim3(kColThreads), 0, stream, a);
   else
     hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32, RAGGED>), dim3(seqs), dim3(kThreads), 0, stream, a);
   hipError_t err = hipGetLastError();
@@ -704,10 +816,25 @@ qh_status launch2(const StateArgs &a, bool wu_f32, bool out_f32, hipStream_t str
 
 }  // namespace
 
+// Bytes that gdn_state_pre_kernel writes: P, then the factors (both multiples of 16).
+static size_t pre_p_bytes(size_t items, int precision) { return items * (precision == QH_GDN_BF16 ? 2 : 4) * kC * kC; }
+
+size_t gdn_chunk_state_workspace(int B, int T, int H, int precision) {
+  const int nchunks = (T + kC - 1) / kC;
+  if (nchunks < kPreChunks || cols_grid(B * H, 2) == 0) return 0;
+  const size_t items = static_cast<size_t>(B) * H * nchunks;
+  return pre_p_bytes(items, precision) + items * kPreF * sizeof(float);
+}
+
 qh_status launch_gdn_chunk_state(const uint16_t *q, const uint16_t *k, const float *g, const void *w, const void *u,
                                  const float *s_in, float *s_out, void *o, int B, int T, int H, int precision,
-                                 bool wu_f32, bool out_f32, hipStream_t stream) {
-  StateArgs a{q, k, g, w, u, s_in, s_out, o, B, T, H, (T + kC - 1) / kC};
+                                 bool wu_f32, bool out_f32, void *ws, size_t ws_bytes, hipStream_t stream) {
+  StateArgs a{q, k, g, w, u, s_in, s_out, o, B, T, H, (T + kC - 1) / kC, nullptr, nullptr};
+  const size_t need = ws ? gdn_chunk_state_workspace(B, T, H, precision) : 0;
+  if (need && ws_bytes >= need) {
+    a.pre_p = static_cast<uint16_t *>(ws);
+    a.pre_f = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + pre_p_bytes(static_cast<size_t>(B) * H * a.nchunks, precision));
+  }
   return precision == QH_GDN_BF16 ? launch2<false>(a, wu_f32, out_f32, stream)
                                   : launch2<true>(a, wu_f32, out_f32, stream);
 }

@@ -224,5 +224,6 @@ qh_status launch_gdn_chunk_uw(const uint16_t *k, const uint16_t *v, const float 
                               void *u, int B, int T, int H, int C, int flags, int max_wg, hipStream_t stream);
 qh_status launch_gdn_chunk_state(const uint16_t *q, const uint16_t *k, const float *g, const void *w, const void *u,
                                  const float *s_in, float *s_out, void *o, int B, int T, int H, int precision,
-                                 bool wu_f32, bool out_f32, hipStream_t stream);
+                                 bool wu_f32, bool out_f32, void *ws, size_t ws_bytes, hipStream_t stream);
+size_t gdn_chunk_state_workspace(int B, int T, int H, int precision);
 }  // namespace qh

@@ -147,11 +147,14 @@ def _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, mor
     with _on(stream):
         o = torch.empty((B, T, H, D), dtype=out_dtype, device=q.device)
         s_out = torch.empty((B, H, D, D), dtype=torch.float32, device=q.device)
+        ws_bytes = _lib.lib().qh_gdn_chunk_state_workspace(B, T, H, precision)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     flags = more_flags | (_lib.QH_GDN_WU_F32 if w.dtype == torch.float32 else 0) | (
         _lib.QH_GDN_OUT_F32 if out_dtype == torch.float32 else 0)
-    st = _lib.lib().qh_gdn_chunk_state(q.data_ptr(), k.data_ptr(), g.data_ptr(), w.data_ptr(), u.data_ptr(),
+    st = _lib.lib().qh_gdn_chunk_state_ws(q.data_ptr(), k.data_ptr(), g.data_ptr(), w.data_ptr(), u.data_ptr(),
                                        0 if initial_state is None else initial_state.data_ptr(), s_out.data_ptr(),
-                                       o.data_ptr(), B, T, H, D, STATE_CHUNK, flags, precision, _stream(stream))
+                                       o.data_ptr(), B, T, H, D, STATE_CHUNK, flags, precision,
+                                       0 if ws is None else ws.data_ptr(), ws_bytes, _stream(stream))
     _lib.check(st, "qh_gdn_chunk_state")
     return o, s_out
 

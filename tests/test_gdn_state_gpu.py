@@ -369,3 +369,32 @@ def test_state_infinity_stays_behind_its_tile(gpu, token, H, precision):
     first = token // 16 * 16
     assert torch.equal(got[:, :first], want[:, :first])
     assert not torch.isfinite(got[:, token]).all()
+
+
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("wu", ["f32", "bf16"], ids=["wu_f32", "wu_bf16"])
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("T", [192, 193, 250, 320])
+def test_operands_formed_ahead_equal_in_recurrence(gpu, T, precision, wu, out):
+    """Few sequences' chunk operands formed in a workspace before the recurrence (one and two column tiles
+    per workgroup, partial last chunks) give the bits of the one-workgroup kernel."""
+    import torch
+
+    from qcom_htp_amd import _lib
+    from qcom_htp_amd.gdn import _chunk_state, _chunk_uw
+
+    H = 130
+    q, k, v, bt, g = (to_dev(x, gpu) for x in seq_inputs(1, T, H, seed=T))
+    s0 = torch.randn((1, H, 128, 128), generator=torch.Generator(device=gpu).manual_seed(3), device=gpu)
+    flags = _lib.QH_GDN_RAGGED if T % 64 else 0
+    odt = torch.float32 if out == "f32" else torch.bfloat16
+    w, u = _chunk_uw(k, v, g, bt, 64, True, torch.float32 if wu == "f32" else torch.bfloat16, None, 0, flags)
+    run = lambda sl: _chunk_state(*(x[:, :, sl].contiguous() for x in (q, k, g, w, u)), s0[:, sl].contiguous(), precision, odt,
+                                  None, flags)
+    assert _lib.lib().qh_gdn_chunk_state_workspace(1, T, H, precision) == 0
+    o_all, s_all = run(slice(0, H))
+    for lo, n in ((0, 1), (1, 9), (10, 32), (50, 33), (60, 64)):
+        assert _lib.lib().qh_gdn_chunk_state_workspace(1, T, n, precision) > 0
+        o, s = run(slice(lo, lo + n))
+        assert torch.equal(o, o_all[:, :, lo:lo + n]), f"{n} sequences: o differs"
+        assert torch.equal(s, s_all[:, lo:lo + n]), f"{n} sequences: S differs"
