@@ -348,6 +348,18 @@ qh_status qh_gdn_chunk_state_ws(const uint16_t *q_dev, const uint16_t *k_dev, co
                                 uint32_t tokens, uint32_t heads, uint32_t head_dim, uint32_t chunk, uint32_t flags,
                                 uint32_t precision, void *workspace_dev, size_t workspace_bytes, void *stream);
 
+/* The whole prefill (both halves, scripts/gdn_ref_kernel.py:104-131) of many sequences without W and U:
+ * T = (I - A)^-1 of every chunk into the workspace, then the recurrence with
+ *   v_new = T (beta v - beta e^g k^ S).
+ * Operands as in qh_gdn_chunk_uw and qh_gdn_chunk_state; tokens need not be a multiple of 64 (the last
+ * chunk's missing tokens count as zeros).  flags: QH_GDN_OUT_F32 (o as float32).  The query returns the
+ * workspace's bytes, or 0 for shapes that qh_gdn_chunk_uw and qh_gdn_chunk_state_ws serve better. */
+size_t qh_gdn_prefill_workspace(uint32_t batch, uint32_t tokens, uint32_t heads, uint32_t precision);
+qh_status qh_gdn_prefill(const uint16_t *q_dev, const uint16_t *k_dev, const uint16_t *v_dev, const float *g_dev,
+                         const float *beta_dev, const float *s_in_dev, float *s_out_dev, void *o_dev, uint32_t batch,
+                         uint32_t tokens, uint32_t heads, uint32_t head_dim, uint32_t flags, uint32_t precision,
+                         void *workspace_dev, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

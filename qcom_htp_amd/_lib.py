@@ -83,6 +83,8 @@ EXPORTED = (
     "qh_gdn_chunk_state",
     "qh_gdn_chunk_state_workspace",
     "qh_gdn_chunk_state_ws",
+    "qh_gdn_prefill",
+    "qh_gdn_prefill_workspace",
 )
 
 
@@ -183,6 +185,10 @@ def _declare(L: C.CDLL) -> None:
     L.qh_gdn_chunk_state_workspace.restype = C.c_size_t
     L.qh_gdn_chunk_state_ws.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, u32, u32, u32, u32, u32, u32, u32, vp, C.c_size_t, vp]
     L.qh_gdn_chunk_state_ws.restype = st
+    L.qh_gdn_prefill_workspace.argtypes = [u32, u32, u32, u32]
+    L.qh_gdn_prefill_workspace.restype = C.c_size_t
+    L.qh_gdn_prefill.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, u32, u32, u32, u32, u32, u32, vp, C.c_size_t, vp]
+    L.qh_gdn_prefill.restype = st
 
 
 def lib() -> C.CDLL:

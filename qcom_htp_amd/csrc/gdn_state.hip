@@ -27,10 +27,19 @@
 // issue and wait for; with W and P as hi | lo words (two reads and eight byte permutes an operand)
 // and a staging phase of its own between two more barriers it took 523 / 398 us (fp32 / bf16), now 505 / 387
 // (B = 8, T = 4096, H = 32; the bytes it moves take 365 / 257 us at the 5.2 TB/s of a large copy).
+//
+// Prefill of many sequences (FROM_T) needs no W and U: they are T (beta e^g k^) and T (beta v), so
+//     v_new = T (beta v - beta e^g k^ S),
+// where k^ S takes k from the rows that are in LDS anyway (exact, one operand half instead of W's two)
+// and T times the result is one more lower triangular product of a wave's own columns.  gdn_t_kernel
+// forms T (16 KB a chunk as hi / lo parts) from k, g and beta alone.  Stage A is bound by the 64 KB of W
+// and U that it writes per chunk in float32 (1.6 GB, 312 us), which stage B then reads again: B = 8,
+// T = 4096, H = 32 takes 130 + 538 us with T against 311 + 523 us (bf16: 117 + 411 against 229 + 392),
+// shortest launches; the prefill 822 -> 626 us.
+//
 // Precision: QH_GDN_FP32 carries W, S, P and v_new as bf16 hi/lo splits (hi*hi + hi*lo + lo*hi,
 // fp32 accumulation; products with the exact q, k take two terms); QH_GDN_BF16 uses the hi
-// parts only.  Norms, decays and the prefix sum are fp32.
-
+// parts only; T's own products are split in both.  Norms, decays and the prefix sum are fp32.
 //
 // Few sequences (gdn_state_cols_kernel): the chunks of a sequence follow one another, so the launch
 // lasts as long as one sequence however few there are, and what counts is a chunk's latency.  The work
@@ -75,6 +84,10 @@ struct StateArgs {
   // (then lo parts with SPLIT), and kPreF floats (the factors of q^ S's and v_new's rows, e^{g_last})
   uint16_t *pre_p;
   float *pre_f;
+  // FROM_T: T = (I - A)^-1 of every (sequence, chunk), [64][64] bf16 hi parts in operand order (then lo
+  // parts with SPLIT), and beta; u holds v
+  uint16_t *t;
+  const float *beta;
 };
 constexpr int kPreF = 2 * kC + 4;
 
@@ -147,6 +160,22 @@ __device__ __forceinline__ v4f mfma(const v8bf a, const v8bf b, const v4f c) {
 // A operand half of one 32-deep step in operand order.
 __device__ __forceinline__ v8bf op8(const uint16_t *p) { return __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4 *>(p)); }
 
+// Of four bf16 rows x 4 adjacent columns in a quad of lanes (P0 = rows 0, 1 and P1 = rows 2, 3 of the
+// lane's column): row q's 4 columns in lane q of the quad, by DPP quad broadcasts.
+__device__ __forceinline__ uint2 quad_rows(uint32_t P0, uint32_t P1, int qq) {
+  const uint32_t a0 = __builtin_amdgcn_mov_dpp(P0, 0x00, 0xF, 0xF, false);
+  const uint32_t a1 = __builtin_amdgcn_mov_dpp(P0, 0x55, 0xF, 0xF, false);
+  const uint32_t a2 = __builtin_amdgcn_mov_dpp(P0, 0xAA, 0xF, 0xF, false);
+  const uint32_t a3 = __builtin_amdgcn_mov_dpp(P0, 0xFF, 0xF, 0xF, false);
+  const uint32_t b0 = __builtin_amdgcn_mov_dpp(P1, 0x00, 0xF, 0xF, false);
+  const uint32_t b1 = __builtin_amdgcn_mov_dpp(P1, 0x55, 0xF, 0xF, false);
+  const uint32_t b2 = __builtin_amdgcn_mov_dpp(P1, 0xAA, 0xF, 0xF, false);
+  const uint32_t b3 = __builtin_amdgcn_mov_dpp(P1, 0xFF, 0xF, 0xF, false);
+  const uint32_t sel = (qq & 1) ? 0x07060302u : 0x05040100u;
+  return qq < 2 ? make_uint2(__builtin_amdgcn_perm(a1, a0, sel), __builtin_amdgcn_perm(a3, a2, sel))
+                : make_uint2(__builtin_amdgcn_perm(b1, b0, sel), __builtin_amdgcn_perm(b3, b2, sel));
+}
+
 // One 16 x 16 result tile of o: `at` is the element offset of the lane's column in row 4 qd of the
 // tile, tok the elements per token, qq the lane's place in its quad; rows: how many of the lane's 4
 // rows exist (RAGGED).
@@ -157,41 +186,55 @@ __device__ __forceinline__ void store_o(void *o, uint32_t at, uint32_t tok, int 
     for (int e = 0; e < 4; ++e)
       if (!RAGGED || e < rows) static_cast<float *>(o)[at + static_cast<uint32_t>(e) * tok] = acc[e];
   } else {
-    // the quad's 4 rows x 4 adjacent columns, transposed with DPP quad broadcasts so that lane
-    // q of the quad stores row 4 qd + q, the quad's 4 columns, in one 8-byte store
-    const uint32_t P0 = pack_bf16(acc[0], acc[1]), P1 = pack_bf16(acc[2], acc[3]);
-    const uint32_t a0 = __builtin_amdgcn_mov_dpp(P0, 0x00, 0xF, 0xF, false);
-    const uint32_t a1 = __builtin_amdgcn_mov_dpp(P0, 0x55, 0xF, 0xF, false);
-    const uint32_t a2 = __builtin_amdgcn_mov_dpp(P0, 0xAA, 0xF, 0xF, false);
-    const uint32_t a3 = __builtin_amdgcn_mov_dpp(P0, 0xFF, 0xF, 0xF, false);
-    const uint32_t b0 = __builtin_amdgcn_mov_dpp(P1, 0x00, 0xF, 0xF, false);
-    const uint32_t b1 = __builtin_amdgcn_mov_dpp(P1, 0x55, 0xF, 0xF, false);
-    const uint32_t b2 = __builtin_amdgcn_mov_dpp(P1, 0xAA, 0xF, 0xF, false);
-    const uint32_t b3 = __builtin_amdgcn_mov_dpp(P1, 0xFF, 0xF, 0xF, false);
-    const uint32_t sel = (qq & 1) ? 0x07060302u : 0x05040100u;
-    const uint2 w = qq < 2 ? make_uint2(__builtin_amdgcn_perm(a1, a0, sel), __builtin_amdgcn_perm(a3, a2, sel))
-                           : make_uint2(__builtin_amdgcn_perm(b1, b0, sel), __builtin_amdgcn_perm(b3, b2, sel));
+    // lane q of the quad stores row 4 qd + q, the quad's 4 columns, in one 8-byte store
+    const uint2 w = quad_rows(pack_bf16(acc[0], acc[1]), pack_bf16(acc[2], acc[3]), qq);
     if (!RAGGED || qq < rows)
       *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(o) + (at - static_cast<uint32_t>(qq) + static_cast<uint32_t>(qq) * tok)) = w;
   }
 }
 
-template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED>
+// acc[i] (or zero, with `fresh`) += sum over the token tiles j <= i of L_ij X_j, L lower triangular in
+// LDS in operand order (lo parts with SPLIT).
+template <bool SPLIT, int NL>
+__device__ __forceinline__ void lower_product(const uint16_t (&hi)[kC][kPs], const uint16_t (&lo)[NL][kPs], int r16, int qd,
+                                              const Half4 (&x)[4], v4f (&acc)[4], bool fresh) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v4f s = fresh ? v4f{0.f, 0.f, 0.f, 0.f} : acc[i];
+#pragma unroll
+    for (int p = 0; p <= i / 2; ++p) {
+      // (no later tile beside a diagonal one: an infinity there would reach these rows)
+      const Half4 x1 = 2 * p + 1 <= i ? x[2 * p + 1] : kZero4;
+      const v8bf l = op8(&hi[16 * i + r16][32 * p + 8 * qd]), xh = op_hi(x[2 * p], x1);
+      s = mfma(l, xh, s);
+      if constexpr (SPLIT) {
+        s = mfma(l, op_lo(x[2 * p], x1), s);
+        s = mfma(op8(&lo[16 * i + r16][32 * p + 8 * qd]), xh, s);
+      }
+    }
+    acc[i] = s;
+  }
+}
+
+// FROM_T: v_new = T (beta v - beta e^g K^ S) from gdn_t_kernel's T instead of U - W S.
+template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED, bool FROM_T>
 __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
+  static_assert(!(FROM_T && WU_F32), "v is bf16");
   constexpr bool kWlo = SPLIT && WU_F32;  // a bf16 W has no lo part
   // q, k rows as given (bf16, exact MFMA operands) with their l2norm factors; W and the lower
   // tiles of P as bf16 hi parts (and lo parts with SPLIT); g, e^g, e^{g_last - g}
   __shared__ __attribute__((aligned(16))) uint16_t Ql[kC][kWs];
   __shared__ __attribute__((aligned(16))) uint16_t Kl[2][kC][kQs];
-  __shared__ __attribute__((aligned(16))) uint16_t Wh[kC][kWs], Wo[kWlo ? kC : 1][kWs];
+  __shared__ __attribute__((aligned(16))) uint16_t Wh[FROM_T ? 1 : kC][kWs], Wo[kWlo ? kC : 1][kWs];
+  __shared__ __attribute__((aligned(16))) uint16_t Th[FROM_T ? kC : 1][kPs], Tl[FROM_T && SPLIT ? kC : 1][kPs];
   __shared__ __attribute__((aligned(16))) uint16_t Ph[kC][kPs], Po[SPLIT ? kC : 1][kPs];
   // 1 / |q| / sqrt(D), 1 / |k| (eps 1e-6 inside the root); g, e^g, e^{g_last - g}
-  __shared__ __attribute__((aligned(16))) float invq[2][kC], invk[2][kC], gl[2][kC], egl[2][kC], decl[2][kC];
+  __shared__ __attribute__((aligned(16))) float invq[2][kC], invk[2][kC], gl[2][kC], egl[2][kC], decl[2][kC], bet[2][kC];
   __shared__ float eglast[2];
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int r16 = lane & 15, qd = lane >> 4;
-  const int b = blockIdx.x / a.H, h = blockIdx.x % a.H;
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / a.H), h = blockIdx.x - b * a.H;
 
   // S: tile kb holds rows (keys) 16 kb + 4 qd + e, column (value) 16 wave + r16
   v4f S[8];
@@ -203,46 +246,68 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
       S[kb][e] = a.s_in ? a.s_in[sbase + static_cast<size_t>(16 * kb + 4 * qd + e) * kD + 16 * wave + r16] : 0.0f;
   }
 
-  // Element offsets of chunk 0 (a chunk adds 64 H D).  A thread stages 16 columns of one row: of q and
-  // k columns 16 seg .., of W the 8 columns 32 (seg / 2) + 8 (seg % 2) .. and the 8 that are 16 further
-  // on, which are adjacent in operand order.
+  // A thread stages 16 columns of one row: of q and k columns 16 seg .., of W the 8 columns
+  // 32 (seg / 2) + 8 (seg % 2) .. and the 8 that are 16 further on, which are adjacent in operand order.
+  // Addresses are a chunk's uniform base and a lane's 32-bit offset in the chunk, so that the bases are
+  // scalar and few registers hold offsets (RAGGED: the row is at most the last one that exists).  The
+  // offsets are opaque in every chunk: left alone, the compiler keeps a 64-bit address for each of the
+  // 30 accesses across the loop, and spills.
   const uint32_t tok = static_cast<uint32_t>(a.H) * kD;
   const uint32_t head = (static_cast<uint32_t>(b) * a.T * a.H + h) * kD;
   const int row = t >> 3, seg = t & 7, wcol = 32 * (seg >> 1) + 8 * (seg & 1);
-  const uint32_t of_row = head + row * tok + 16 * seg, of_w = head + row * tok + wcol;
-  const uint32_t of_tile = head + 4 * qd * tok + 16 * wave + r16;
+  auto chunk_at = [&](int n) __attribute__((always_inline)) { return static_cast<size_t>(head + static_cast<uint32_t>(n) * kC * tok); };
+  auto row_at = [&](int n, int r) __attribute__((always_inline)) {
+    return static_cast<uint32_t>(RAGGED ? min(r, a.T - 1 - n * kC) : r) * tok;
+  };
+  const uint32_t col = 16 * wave + r16;
   const uint32_t of_g = static_cast<uint32_t>(b) * a.T * a.H + lane * a.H + h;
 
   uint4 iq[2], ik[2], iw[2][WU_F32 ? 2 : 1];
-  float iu[4][4], igc;
+  float iu[4][4], igc, ibeta = 0.0f;
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  v4u it[2] = {};
   auto load = [&](int n) __attribute__((always_inline)) {
-    const uint32_t c0 = static_cast<uint32_t>(n) * kC * tok, back = past_end<RAGGED>(a, n, row) * tok;
-    const uint4 *qp = reinterpret_cast<const uint4 *>(a.q + (of_row + c0 - back));
-    const uint4 *kp = reinterpret_cast<const uint4 *>(a.k + (of_row + c0 - back));
+    const size_t c0 = chunk_at(n);
+    uint32_t ro = row_at(n, row);
+    asm volatile("" : "+v"(ro));
+    const uint4 *qp = reinterpret_cast<const uint4 *>(a.q + c0 + (ro + 16 * seg));
+    const uint4 *kp = reinterpret_cast<const uint4 *>(a.k + c0 + (ro + 16 * seg));
     iq[0] = qp[0];
     iq[1] = qp[1];
     ik[0] = kp[0];
     ik[1] = kp[1];
+    if constexpr (FROM_T) {
+      const v4u *tp = reinterpret_cast<const v4u *>(a.t + (static_cast<size_t>(blockIdx.x) * a.nchunks + n) * (SPLIT ? 2 : 1) * (kC * kC)) + t;
+      it[0] = tp[0];
+      if constexpr (SPLIT) it[1] = tp[kC * kC / 8];
+    } else {
 #pragma unroll
-    for (int x = 0; x < 2; ++x) {
-      const uint32_t wi = of_w + c0 - back + 16 * x;
-      const uint4 *wp = WU_F32 ? reinterpret_cast<const uint4 *>(static_cast<const float *>(a.w) + wi)
-                               : reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.w) + wi);
-      iw[x][0] = wp[0];
-      if constexpr (WU_F32) iw[x][1] = wp[1];
+      for (int x = 0; x < 2; ++x) {
+        const uint32_t wi = ro + wcol + 16 * x;
+        const uint4 *wp = WU_F32 ? reinterpret_cast<const uint4 *>(static_cast<const float *>(a.w) + c0 + wi)
+                                 : reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.w) + c0 + wi);
+        iw[x][0] = wp[0];
+        if constexpr (WU_F32) iw[x][1] = wp[1];
+      }
     }
     const uint32_t gb = past_end<RAGGED>(a, n, lane);
-    igc = a.g[of_g + (static_cast<uint32_t>(n) * kC - gb) * static_cast<uint32_t>(a.H)];
-    if (RAGGED && gb) igc = 0.0f;
+    const uint32_t gi = of_g + (static_cast<uint32_t>(n) * kC - gb) * static_cast<uint32_t>(a.H);
+    igc = a.g[gi];
+    if constexpr (FROM_T) ibeta = a.beta[gi];
+    if (RAGGED && gb) igc = ibeta = 0.0f;
   };
   auto load_u = [&](int n) __attribute__((always_inline)) {
-    const uint32_t ti = of_tile + static_cast<uint32_t>(n) * kC * tok;
+    const size_t c0 = chunk_at(n);
+    uint32_t lo = 4 * qd * tok + col;
+    asm volatile("" : "+v"(lo));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint32_t ui = ti + static_cast<uint32_t>(16 * i + e) * tok - past_end<RAGGED>(a, n, 16 * i + 4 * qd + e) * tok;
-        iu[i][e] = WU_F32 ? static_cast<const float *>(a.u)[ui] : bf16f(static_cast<const uint16_t *>(a.u)[ui]);
+        // the lane's row is 4 qd + (16 i + e): the second part in the base unless rows are clamped
+        const size_t base = RAGGED ? c0 : c0 + static_cast<size_t>(static_cast<uint32_t>(16 * i + e) * tok);
+        const uint32_t ui = RAGGED ? row_at(n, 16 * i + 4 * qd + e) + col : lo;
+        iu[i][e] = WU_F32 ? (static_cast<const float *>(a.u) + base)[ui] : bf16f((static_cast<const uint16_t *>(a.u) + base)[ui]);
       }
     }
   };
@@ -262,8 +327,11 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
       invk[bf][row] = inv_k(sk);
     }
     // W: two lane quarters' 8 values, 4 of each 16-column block
-    uint16_t *const wd = &Wh[row][kpos(wcol)];
-    if constexpr (WU_F32) {
+    uint16_t *const wd = &Wh[FROM_T ? 0 : row][kpos(wcol)];
+    if constexpr (FROM_T) {
+      *reinterpret_cast<v4u *>(&Th[FROM_T ? row : 0][8 * seg]) = it[0];
+      if constexpr (SPLIT) *reinterpret_cast<v4u *>(&Tl[FROM_T && SPLIT ? row : 0][8 * seg]) = it[1];
+    } else if constexpr (WU_F32) {
       Half4 x[2][2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -290,6 +358,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
       egl[bf][lane] = expf(g);
       decl[bf][lane] = RAGGED && n * kC + lane >= a.T ? 0.0f : expf(glast - g);
       if (lane == 0) eglast[bf] = expf(glast);
+      if constexpr (FROM_T) bet[bf][lane] = ibeta;
     }
   };
 
@@ -307,41 +376,51 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
   auto chunk = [&](const int n) __attribute__((always_inline)) {
     const int bf = n & 1;
     // ---- M: W S, q^ S, v_new; P tiles ----------------------------------------------------------
-    v8bf sh[4], sl[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const Half4 s0 = split4<SPLIT>(S[2 * p]), s1 = split4<SPLIT>(S[2 * p + 1]);
-      sh[p] = op_hi(s0, s1);
-      sl[p] = op_lo(s0, s1);
-    }
     v4f ws[4], qs[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) ws[i] = qs[i] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int p = 0; p < 4; ++p) {  // key blocks 2p, 2p + 1: 8 independent accumulations
       const int c = 32 * p + 8 * qd;
+      const Half4 s0 = split4<SPLIT>(S[2 * p]), s1 = split4<SPLIT>(S[2 * p + 1]);
+      const v8bf sh = op_hi(s0, s1), sl = op_lo(s0, s1);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const v8bf w = op8(&Wh[16 * i + r16][c]), q = op8(&Ql[16 * i + r16][c]);
-        ws[i] = mfma(w, sh[p], ws[i]);
-        qs[i] = mfma(q, sh[p], qs[i]);
+        const uint16_t *const krow = &Kl[bf][16 * i + r16][32 * p + 4 * qd];
+        const v8bf w = FROM_T ? op_hi(bf16x4(krow), bf16x4(krow + 16)) : op8(&Wh[FROM_T ? 0 : 16 * i + r16][c]);
+        const v8bf q = op8(&Ql[16 * i + r16][c]);
+        ws[i] = mfma(w, sh, ws[i]);
+        qs[i] = mfma(q, sh, qs[i]);
         if constexpr (SPLIT) {
-          ws[i] = mfma(w, sl[p], ws[i]);
-          qs[i] = mfma(q, sl[p], qs[i]);
+          ws[i] = mfma(w, sl, ws[i]);
+          qs[i] = mfma(q, sl, qs[i]);
         }
-        if constexpr (kWlo) ws[i] = mfma(op8(&Wo[16 * i + r16][c]), sh[p], ws[i]);
+        if constexpr (kWlo) ws[i] = mfma(op8(&Wo[16 * i + r16][c]), sh, ws[i]);
       }
+      if constexpr (FROM_T) __builtin_amdgcn_sched_barrier(0);  // (reads of a later step moved up here spill)
     }
     v4f vnew[4], oacc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const v4f iq4 = *reinterpret_cast<const v4f *>(&invq[bf][16 * i + 4 * qd]);
       const v4f eg4 = *reinterpret_cast<const v4f *>(&egl[bf][16 * i + 4 * qd]);
+      const v4f be4 = *reinterpret_cast<const v4f *>(&bet[bf][16 * i + 4 * qd]);
+      const v4f ik4 = *reinterpret_cast<const v4f *>(&invk[bf][16 * i + 4 * qd]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        vnew[i][e] = iu[i][e] - ws[i][e];
+        vnew[i][e] = FROM_T ? be4[e] * (iu[i][e] - (eg4[e] * ik4[e]) * ws[i][e]) : iu[i][e] - ws[i][e];
         oacc[i][e] = qs[i][e] * (iq4[e] * eg4[e]);
       }
+    }
+    if constexpr (FROM_T) {  // v_new = T R, R's tiles from the accumulators as they are
+      __builtin_amdgcn_sched_barrier(0);
+      Half4 rB[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) rB[j] = split4<SPLIT>(vnew[j]);
+      lower_product<SPLIT>(Th, Tl, r16, qd, rB, vnew, true);
+      // (formed here: moved behind the P loop, its 12 operand reads would stay in registers across it)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(vnew[i]));
     }
     load_u(min(n + 1, a.nchunks - 1));
     for (int idx = kThreads / 64 - 1 - wave; idx < 10; idx += kThreads / 64) {  // wave-uniform
@@ -354,15 +433,15 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
         const int c = 32 * p + 4 * qd;
         acc = mfma(op8(&Ql[16 * ti + r16][32 * p + 8 * qd]), op_hi(bf16x4(krow + c), bf16x4(krow + c + 16)), acc);
       }
-      const int col = 16 * tj + r16;
-      const float kf = invk[bf][col], gc = gl[bf][col];
+      const int pcol = 16 * tj + r16;
+      const float kf = invk[bf][pcol], gc = gl[bf][pcol];
       const v4f iq4 = *reinterpret_cast<const v4f *>(&invq[bf][16 * ti + 4 * qd]);
       const v4f gr4 = *reinterpret_cast<const v4f *>(&gl[bf][16 * ti + 4 * qd]);
-      const int pc = kpos(col);
+      const int pc = kpos(pcol);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int rw = 16 * ti + 4 * qd + e;
-        const uint32_t pv = hilo<SPLIT>(col <= rw ? acc[e] * (iq4[e] * kf) * expf(gr4[e] - gc) : 0.0f);
+        const uint32_t pv = hilo<SPLIT>(pcol <= rw ? acc[e] * (iq4[e] * kf) * expf(gr4[e] - gc) : 0.0f);
         Ph[rw][pc] = static_cast<uint16_t>(pv);
         if constexpr (SPLIT) Po[rw][pc] = static_cast<uint16_t>(pv >> 16);
       }
@@ -399,27 +478,19 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
                                    dB[2 * p], dB[2 * p + 1], S[kb]);
       }
     }
+    if constexpr (FROM_T) __builtin_amdgcn_sched_barrier(0);
     // ---- o = e^g q^ S + P v_new (causal pairs of token tiles) ------------------------------------
     Half4 vB[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) vB[j] = split4<SPLIT>(vnew[j]);
+    lower_product<SPLIT>(Ph, Po, r16, qd, vB, oacc, false);
+    if constexpr (FROM_T) __builtin_amdgcn_sched_barrier(0);
+    uint32_t oo = 4 * qd * tok + col;
+    asm volatile("" : "+v"(oo));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v4f acc = oacc[i];
-#pragma unroll
-      for (int p = 0; p <= i / 2; ++p) {
-        // (no later tile's v_new beside a diagonal tile: an infinity there would reach these rows)
-        const Half4 v1 = 2 * p + 1 <= i ? vB[2 * p + 1] : kZero4;
-        const v8bf ph = op8(&Ph[16 * i + r16][32 * p + 8 * qd]), vh = op_hi(vB[2 * p], v1);
-        acc = mfma(ph, vh, acc);
-        if constexpr (SPLIT) {
-          acc = mfma(ph, op_lo(vB[2 * p], v1), acc);
-          acc = mfma(op8(&Po[16 * i + r16][32 * p + 8 * qd]), vh, acc);
-        }
-      }
-      store_o<OUT_F32, RAGGED>(a.o, of_tile + static_cast<uint32_t>(n * kC + 16 * i) * tok, tok, r16 & 3, acc,
-                               a.T - (n * kC + 16 * i + 4 * qd));
-    }
+    for (int i = 0; i < 4; ++i)
+      store_o<OUT_F32, RAGGED>(static_cast<char *>(a.o) + (chunk_at(n) + static_cast<uint32_t>(16 * i) * tok) * (OUT_F32 ? 4 : 2),
+                               oo, tok, r16 & 3, oacc[i], a.T - (n * kC + 16 * i + 4 * qd));
     // ---- the next chunk's rows.  Unconditional (the last chunk stages and loads itself again,
     // unused): behind a branch the compiler would lose count of the loads in flight and wait for every
     // memory operation, the o stores included.
@@ -708,6 +779,119 @@ __global__ __launch_bounds__(kColThreads) void gdn_state_cols_kernel(StateArgs a
   }
 }
 
+// T = (I - A)^-1 of every chunk of 64 tokens, A_ij = -beta_i (k^_i . k^_j) e^{g_i - g_j} for i > j, as
+// gdn_state_kernel reads it (FROM_T).  One workgroup (4 waves) per (sequence, chunk): the 10 lower tiles
+// of K K^T over the waves; T's diagonal blocks by forward substitution, one lane per column; then wave j
+// the strip of block column j, its solved blocks in registers as the next products' B operands.
+constexpr int kTThreads = 256;
+constexpr int kTd = 260;  // floats per diagonal block (padded: four blocks are read at once)
+constexpr int kTr = 20;   // row stride of a lower block, floats
+template <bool SPLIT, bool RAGGED>
+__global__ __launch_bounds__(kTThreads) void gdn_t_kernel(StateArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t Kl[kC][kQs];
+  __shared__ __attribute__((aligned(16))) float diag[4 * kTd], low[6][16][kTr], invk[kC], gl[kC], bet[kC];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int r16 = lane & 15, qd = lane >> 4;
+  const int seq = blockIdx.x / a.nchunks, n = blockIdx.x % a.nchunks, b = seq / a.H, h = seq % a.H;
+  const uint32_t tok = static_cast<uint32_t>(a.H) * kD;
+  const uint32_t head = (static_cast<uint32_t>(b) * a.T * a.H + h) * kD;
+  uint4 ik[2][2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int row = 32 * r + (t >> 3);
+    const uint4 *kp = reinterpret_cast<const uint4 *>(a.k + (head + 16 * (t & 7) + (static_cast<uint32_t>(n) * kC + row - past_end<RAGGED>(a, n, row)) * tok));
+    ik[r][0] = kp[0];
+    ik[r][1] = kp[1];
+  }
+  if (wave == 0) {
+    const uint32_t back = past_end<RAGGED>(a, n, lane);
+    const uint32_t gi = static_cast<uint32_t>(b) * a.T * a.H + h + (static_cast<uint32_t>(n) * kC + lane - back) * static_cast<uint32_t>(a.H);
+    const bool past = RAGGED && back;
+    gl[lane] = scan64(past ? 0.0f : a.g[gi]);
+    bet[lane] = past ? 0.0f : a.beta[gi];
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int row = 32 * r + (t >> 3), seg = t & 7;
+    *reinterpret_cast<uint4 *>(&Kl[row][16 * seg]) = ik[r][0];
+    *reinterpret_cast<uint4 *>(&Kl[row][16 * seg + 8]) = ik[r][1];
+    const float ss = row_square(ik[r]);
+    if (seg == 0) invk[row] = inv_k(ss);
+  }
+  lds_barrier();
+  for (int idx = wave; idx < 10; idx += kTThreads / 64) {  // wave-uniform
+    int ti, tj;
+    p_tile(idx, ti, tj);
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    const uint16_t *irow = Kl[16 * ti + r16], *jrow = Kl[16 * tj + r16];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int c = 32 * p + 4 * qd;
+      acc = mma<false>(bf16x4(irow + c), bf16x4(irow + c + 16), bf16x4(jrow + c), bf16x4(jrow + c + 16), acc);
+    }
+    const int col = 16 * tj + r16;
+    const float kf = invk[col], gc = gl[col];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 4 * qd + e, rw = 16 * ti + r;
+      const float av = col < rw ? -bet[rw] * acc[e] * (invk[rw] * kf) * expf(gl[rw] - gc) : 0.0f;
+      if (ti > tj)
+        low[ti * (ti - 1) / 2 + tj][r][r16] = av;
+      else
+        diag[ti * kTd + r16 * 16 + r] = av;  // by columns
+    }
+  }
+  lds_barrier();
+  if (wave == 0) {  // T_II, lane: block lane / 16, column lane % 16; in place, by rows
+    float *const d = diag + qd * kTd;
+    float x[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float s = r == r16 ? 1.0f : 0.0f;
+#pragma unroll
+      for (int c = 0; c < r; ++c) s = fmaf(d[c * 16 + r], x[c], s);
+      x[r] = s;
+    }
+    asm volatile("" ::: "memory");  // every read of A is before the first store of T
+#pragma unroll
+    for (int r = 0; r < 16; ++r) d[r * 16 + r16] = x[r];
+  }
+  lds_barrier();
+  uint16_t *const T = a.t + static_cast<size_t>(blockIdx.x) * (SPLIT ? 2 : 1) * (kC * kC);
+  const int j = wave, qq = r16 & 3;
+  auto store = [&](int i, const Half4 &x) __attribute__((always_inline)) {
+    uint16_t *const d = T + (16 * i + 4 * qd + qq) * kC + kpos(16 * j + (r16 & ~3));
+    *reinterpret_cast<uint2 *>(d) = quad_rows(x.h01, x.h23, qq);
+    if constexpr (SPLIT) *reinterpret_cast<uint2 *>(d + kC * kC) = quad_rows(x.l01, x.l23, qq);
+  };
+  auto f4 = [](const float *p) __attribute__((always_inline)) { return split4<true>(*reinterpret_cast<const float4 *>(p)); };
+  if (j & 1) store(j - 1, kZero4);  // read beside the diagonal tile
+  Half4 xs[4];
+  {
+    const float *const d = diag + j * kTd + 64 * qd + r16;
+    xs[0] = split4<true>(d[0], d[16], d[32], d[48]);
+    store(j, xs[0]);
+  }
+#pragma unroll
+  for (int s = 1; s < 4; ++s) {
+    const int i = j + s;
+    if (i < 4) {  // wave-uniform
+      v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < s; u += 2) {
+        const int blk = i * (i - 1) / 2 + j + u;
+        const bool two = u + 1 < s;
+        acc = mma<true>(f4(&low[blk][r16][4 * qd]), two ? f4(&low[two ? blk + 1 : blk][r16][4 * qd]) : kZero4, xs[u],
+                        two ? xs[u + 1] : kZero4, acc);
+      }
+      const v4f x = mma<true>(f4(diag + i * kTd + 16 * r16 + 4 * qd), kZero4, split4<true>(acc), kZero4, v4f{0.f, 0.f, 0.f, 0.f});
+      xs[s] = split4<true>(x);
+      store(i, xs[s]);
+    }
+  }
+}
+
 // What a chunk needs besides the state, for every (sequence, chunk) at once: P, the row factors of q^ S
 // (e^g / |q| / sqrt(D)) and of v_new in the state update (e^{g_last - g} / |k|), e^{g_last}.  Left to
 // the recurrence, these are some 60 % of the instructions of a chunk of gdn_state_cols_kernel, repeated
@@ -797,7 +981,7 @@ qh_status launch4(const StateArgs &a, hipStream_t stream) {
   } else if (grid2)
     hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, 2, false>), dim3(grid2), dim3(kColThreads), 0, stream, a);
   else
-    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32, RAGGED>), dim3(seqs), dim3(kThreads), 0, stream, a);
+    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, false>), dim3(seqs), dim3(kThreads), 0, stream, a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return hip_fail(err, "gdn_state_kernel launch");
   return QH_STATUS_OK;
@@ -806,6 +990,22 @@ qh_status launch4(const StateArgs &a, hipStream_t stream) {
 template <bool SPLIT, bool WU_F32, bool OUT_F32>
 qh_status launch3(const StateArgs &a, hipStream_t stream) {
   return a.T % kC ? launch4<SPLIT, WU_F32, OUT_F32, true>(a, stream) : launch4<SPLIT, WU_F32, OUT_F32, false>(a, stream);
+}
+
+// Prefill of many sequences: T, then the recurrence from T and v.
+template <bool SPLIT, bool RAGGED>
+qh_status launch_prefill2(const StateArgs &a, bool out_f32, hipStream_t stream) {
+  const int seqs = a.B * a.H;
+  hipLaunchKernelGGL((gdn_t_kernel<SPLIT, RAGGED>), dim3(seqs * a.nchunks), dim3(kTThreads), 0, stream, a);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return hip_fail(err, "gdn_t_kernel launch");
+  if (out_f32)
+    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, false, true, RAGGED, true>), dim3(seqs), dim3(kThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, false, false, RAGGED, true>), dim3(seqs), dim3(kThreads), 0, stream, a);
+  err = hipGetLastError();
+  if (err != hipSuccess) return hip_fail(err, "gdn_state_kernel launch");
+  return QH_STATUS_OK;
 }
 
 template <bool SPLIT>
@@ -829,7 +1029,7 @@ size_t gdn_chunk_state_workspace(int B, int T, int H, int precision) {
 qh_status launch_gdn_chunk_state(const uint16_t *q, const uint16_t *k, const float *g, const void *w, const void *u,
                                  const float *s_in, float *s_out, void *o, int B, int T, int H, int precision,
                                  bool wu_f32, bool out_f32, void *ws, size_t ws_bytes, hipStream_t stream) {
-  StateArgs a{q, k, g, w, u, s_in, s_out, o, B, T, H, (T + kC - 1) / kC, nullptr, nullptr};
+  StateArgs a{q, k, g, w, u, s_in, s_out, o, B, T, H, (T + kC - 1) / kC, nullptr, nullptr, nullptr, nullptr};
   const size_t need = ws ? gdn_chunk_state_workspace(B, T, H, precision) : 0;
   if (need && ws_bytes >= need) {
     a.pre_p = static_cast<uint16_t *>(ws);
@@ -837,6 +1037,22 @@ qh_status launch_gdn_chunk_state(const uint16_t *q, const uint16_t *k, const flo
   }
   return precision == QH_GDN_BF16 ? launch2<false>(a, wu_f32, out_f32, stream)
                                   : launch2<true>(a, wu_f32, out_f32, stream);
+}
+
+// Few sequences take the column-sliced recurrence, which reads W and U.
+size_t gdn_prefill_workspace(int B, int T, int H, int precision) {
+  if (cols_grid(B * H, 2) != 0) return 0;
+  return pre_p_bytes(static_cast<size_t>(B) * H * ((T + kC - 1) / kC), precision);  // T is P's size
+}
+
+qh_status launch_gdn_prefill(const uint16_t *q, const uint16_t *k, const uint16_t *v, const float *g, const float *beta,
+                             const float *s_in, float *s_out, void *o, int B, int T, int H, int precision, bool out_f32,
+                             void *ws, hipStream_t stream) {
+  StateArgs a{q, k, g, nullptr, v, s_in, s_out, o, B, T, H, (T + kC - 1) / kC, nullptr, nullptr, static_cast<uint16_t *>(ws), beta};
+  const bool ragged = T % kC != 0;
+  if (precision == QH_GDN_BF16)
+    return ragged ? launch_prefill2<false, true>(a, out_f32, stream) : launch_prefill2<false, false>(a, out_f32, stream);
+  return ragged ? launch_prefill2<true, true>(a, out_f32, stream) : launch_prefill2<true, false>(a, out_f32, stream);
 }
 
 }  // namespace qh

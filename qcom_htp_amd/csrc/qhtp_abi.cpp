@@ -334,4 +334,36 @@ qh_status qh_gdn_chunk_state_ws(const uint16_t *q_dev, const uint16_t *k_dev, co
                                 static_cast<hipStream_t>(stream));
 }
 
+size_t qh_gdn_prefill_workspace(uint32_t batch, uint32_t tokens, uint32_t heads, uint32_t precision) {
+  if (batch == 0 || heads == 0 || tokens == 0 || static_cast<uint64_t>(batch) * tokens * heads > (1ull << 31) / 128) return 0;
+  return gdn_prefill_workspace(static_cast<int>(batch), static_cast<int>(tokens), static_cast<int>(heads),
+                               static_cast<int>(precision));
+}
+
+qh_status qh_gdn_prefill(const uint16_t *q_dev, const uint16_t *k_dev, const uint16_t *v_dev, const float *g_dev,
+                         const float *beta_dev, const float *s_in_dev, float *s_out_dev, void *o_dev, uint32_t batch,
+                         uint32_t tokens, uint32_t heads, uint32_t head_dim, uint32_t flags, uint32_t precision,
+                         void *workspace_dev, size_t workspace_bytes, void *stream) {
+  if (!q_dev || !k_dev || !v_dev || !g_dev || !beta_dev || !s_out_dev || !o_dev || !workspace_dev)
+    return fail(QH_STATUS_INVALID_ARGUMENT, "qh_gdn_prefill: NULL buffer");
+  if (head_dim != 128) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_prefill: head_dim=%u (need 128)", head_dim);
+  if (flags & ~static_cast<uint32_t>(QH_GDN_OUT_F32)) return fail(QH_STATUS_UNSUPPORTED, "qh_gdn_prefill: unknown flags 0x%x", flags);
+  if (precision > QH_GDN_BF16) return fail(QH_STATUS_UNSUPPORTED, "qh_gdn_prefill: unknown precision %u", precision);
+  const size_t need = qh_gdn_prefill_workspace(batch, tokens, heads, precision);
+  if (need == 0)
+    return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_prefill: batch=%u tokens=%u heads=%u has no workspace (few sequences: stages A and B)",
+                batch, tokens, heads);
+  if (workspace_bytes < need) return fail(QH_STATUS_INVALID_ARGUMENT, "qh_gdn_prefill: workspace too small");
+  if (s_in_dev != nullptr && s_in_dev == s_out_dev)
+    return fail(QH_STATUS_INVALID_ARGUMENT, "qh_gdn_prefill: s_out_dev aliases s_in_dev");
+  const uintptr_t al = reinterpret_cast<uintptr_t>(q_dev) | reinterpret_cast<uintptr_t>(k_dev) |
+                       reinterpret_cast<uintptr_t>(v_dev) | reinterpret_cast<uintptr_t>(o_dev) |
+                       reinterpret_cast<uintptr_t>(s_out_dev) | reinterpret_cast<uintptr_t>(s_in_dev) |
+                       reinterpret_cast<uintptr_t>(workspace_dev);
+  if (al % 16) return fail(QH_STATUS_INVALID_ARGUMENT, "qh_gdn_prefill: buffers must be 16-byte aligned");
+  return launch_gdn_prefill(q_dev, k_dev, v_dev, g_dev, beta_dev, s_in_dev, s_out_dev, o_dev, static_cast<int>(batch),
+                            static_cast<int>(tokens), static_cast<int>(heads), static_cast<int>(precision),
+                            (flags & QH_GDN_OUT_F32) != 0, workspace_dev, static_cast<hipStream_t>(stream));
+}
+
 }  // extern "C"

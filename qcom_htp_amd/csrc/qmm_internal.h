@@ -226,4 +226,8 @@ qh_status launch_gdn_chunk_state(const uint16_t *q, const uint16_t *k, const flo
                                  const float *s_in, float *s_out, void *o, int B, int T, int H, int precision,
                                  bool wu_f32, bool out_f32, void *ws, size_t ws_bytes, hipStream_t stream);
 size_t gdn_chunk_state_workspace(int B, int T, int H, int precision);
+qh_status launch_gdn_prefill(const uint16_t *q, const uint16_t *k, const uint16_t *v, const float *g, const float *beta,
+                             const float *s_in, float *s_out, void *o, int B, int T, int H, int precision, bool out_f32,
+                             void *ws, hipStream_t stream);
+size_t gdn_prefill_workspace(int B, int T, int H, int precision);
 }  // namespace qh

@@ -89,7 +89,7 @@ def gdn_chunk_uw(k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, beta: torch.
     return _chunk_uw(k, v, g, beta, chunk, decay_w, out_dtype, stream, max_workgroups, 0)
 
 
-def _chunk_uw(k, v, g, beta, chunk, decay_w, out_dtype, stream, max_workgroups, more_flags):
+def _check_uw(k, v, g, beta, out_dtype):
     for name, x, dt in (("k", k, torch.bfloat16), ("v", v, torch.bfloat16), ("g", g, torch.float32),
                         ("beta", beta, torch.float32)):
         if x.device.type != "cuda" or x.dtype != dt or not x.is_contiguous():
@@ -99,6 +99,10 @@ def _chunk_uw(k, v, g, beta, chunk, decay_w, out_dtype, stream, max_workgroups, 
     if out_dtype not in (torch.bfloat16, torch.float32):
         raise TypeError("out_dtype must be bfloat16 or float32")
     _same_device(k.device, v=v, g=g, beta=beta)
+
+
+def _chunk_uw(k, v, g, beta, chunk, decay_w, out_dtype, stream, max_workgroups, more_flags):
+    _check_uw(k, v, g, beta, out_dtype)
     B, T, H, D = k.shape
     with _on(stream):
         w = torch.empty((B, T, H, D), dtype=out_dtype, device=k.device)
@@ -123,7 +127,7 @@ def gdn_chunk_state(q: torch.Tensor, k: torch.Tensor, g: torch.Tensor, w: torch.
     return _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, 0)
 
 
-def _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, more_flags):
+def _check_state(q, k, g, w, u, initial_state, out_dtype):
     for name, x in (("q", q), ("k", k)):
         if x.device.type != "cuda" or x.dtype != torch.bfloat16 or not x.is_contiguous():
             raise TypeError(f"{name} must be a contiguous bfloat16 CUDA tensor")
@@ -144,6 +148,11 @@ def _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, mor
             raise TypeError("initial_state must be a contiguous float32 [B, H, D, D] tensor")
     # every operand on q's device: a host tensor's address would be dereferenced by the kernel
     _same_device(q.device, k=k, g=g, w=w, u=u, initial_state=initial_state)
+
+
+def _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, more_flags):
+    _check_state(q, k, g, w, u, initial_state, out_dtype)
+    B, T, H, D = q.shape
     with _on(stream):
         o = torch.empty((B, T, H, D), dtype=out_dtype, device=q.device)
         s_out = torch.empty((B, H, D, D), dtype=torch.float32, device=q.device)
@@ -165,8 +174,9 @@ def gdn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tens
     """The chunked gated-delta-rule prefill, the reference's ``gdn_kernel``
     (scripts/gdn_ref_kernel.py:104-131): q, k, v bf16 [B, T, H, 128], g (per-token log decay) and
     beta float32 [B, T, H] -> (o [B, T, H, 128], S [B, H, 128, 128] float32).  The missing tokens
-    of a last partial chunk of 64 count as zeros, which leaves o and S unchanged.  Stage A runs
-    with float32 W, U for ``FP32`` and bf16 for ``BF16``."""
+    of a last partial chunk of 64 count as zeros, which leaves o and S unchanged.  Few sequences
+    run stages A (float32 W, U for ``FP32``, bf16 for ``BF16``) and B; many take the recurrence
+    from T = (I - A)^-1, without W and U."""
     B, T, H, D = q.shape
     _same_device(q.device, k=k, v=v, g=g, beta=beta, initial_state=initial_state)
     ragged = _lib.QH_GDN_RAGGED if T % STATE_CHUNK else 0
@@ -178,5 +188,18 @@ def gdn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tens
             # a partial last chunk takes inputs of any strides and alignment; whole chunks are checked
             g, beta = g.contiguous(), beta.contiguous()
             q, k, v = (x if x.data_ptr() % 16 == 0 else x.clone() for x in (q.contiguous(), k.contiguous(), v.contiguous()))
+        ws_bytes = _lib.lib().qh_gdn_prefill_workspace(B, T, H, precision) if D == 128 and precision in (FP32, BF16) else 0
+        if ws_bytes:
+            _check_uw(k, v, g, beta, wu_dtype)
+            _check_state(q, k, g, v, v, initial_state, out_dtype)
+            o = torch.empty((B, T, H, D), dtype=out_dtype, device=q.device)
+            s_out = torch.empty((B, H, D, D), dtype=torch.float32, device=q.device)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+            st = _lib.lib().qh_gdn_prefill(q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(),
+                                           0 if initial_state is None else initial_state.data_ptr(), s_out.data_ptr(),
+                                           o.data_ptr(), B, T, H, D, _lib.QH_GDN_OUT_F32 if out_dtype == torch.float32 else 0,
+                                           precision, ws.data_ptr(), ws_bytes, _stream(stream))
+            _lib.check(st, "qh_gdn_prefill")
+            return o, s_out
         w, u = _chunk_uw(k, v, g, beta, STATE_CHUNK, True, wu_dtype, stream, 0, ragged)
         return _chunk_state(q, k, g, w, u, initial_state, precision, out_dtype, stream, ragged)

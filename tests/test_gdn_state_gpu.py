@@ -398,3 +398,35 @@ def test_operands_formed_ahead_equal_in_recurrence(gpu, T, precision, wu, out):
         o, s = run(slice(lo, lo + n))
         assert torch.equal(o, o_all[:, :, lo:lo + n]), f"{n} sequences: o differs"
         assert torch.equal(s, s_all[:, lo:lo + n]), f"{n} sequences: S differs"
+
+
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("T", [1, 17, 64, 127, 193])
+def test_prefill_from_t_matches_fp64(gpu, T, precision, out):
+    """Many sequences take the recurrence from T = (I - A)^-1: o and S against the float64 recurrence, with the
+    bound of stage A's bf16 products (1.05e-2), which the route through W and U meets as well."""
+    import torch
+
+    from qcom_htp_amd import _lib
+    from qcom_htp_amd.gdn import gdn_prefill
+
+    B, H = 2, 40
+    qb, kb, vb, beta, gc = seq_inputs(B, T, H, seed=31 + T)
+    q, k, v, bt, g = (to_dev(x, gpu) for x in (qb, kb, vb, beta, gc))
+    s0 = 0.1 * torch.randn((B, H, 128, 128), generator=torch.Generator(device=gpu).manual_seed(3), device=gpu)
+    assert _lib.lib().qh_gdn_prefill_workspace(B, T, H, precision) > 0
+    o, S = gdn_prefill(q, k, v, g, bt, s0, precision, torch.float32 if out == "f32" else torch.bfloat16)
+    x = lambda a: a.double().cpu().transpose(1, 2).contiguous()  # noqa: E731  [B, H, T, ...]
+    qd, kd, vd, bd, gd, St = x(q), x(k), x(v), x(bt), x(g), s0.double().cpu().clone()
+    qd = qd / torch.sqrt((qd * qd).sum(-1, keepdim=True) + 1e-6) / 128 ** 0.5
+    kd = kd / torch.sqrt((kd * kd).sum(-1, keepdim=True) + 1e-6)
+    want = torch.empty_like(vd)
+    for t in range(T):  # token by token
+        St = St * torch.exp(gd[:, :, t])[..., None, None]
+        kt = kd[:, :, t]
+        d = bd[:, :, t, None] * (vd[:, :, t] - (St * kt[..., None]).sum(-2))
+        St = St + kt[..., None] * d[..., None, :]
+        want[:, :, t] = (St * qd[:, :, t, :, None]).sum(-2)
+    rel = lambda a, b: float((a - b).norm() / b.norm())  # noqa: E731
+    assert rel(x(o), want) <= 1.05e-2 and rel(S.double().cpu(), St) <= 1.05e-2
