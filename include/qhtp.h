@@ -353,7 +353,9 @@ qh_status qh_gdn_chunk_state_ws(const uint16_t *q_dev, const uint16_t *k_dev, co
  *   v_new = T (beta v - beta e^g k^ S).
  * Operands as in qh_gdn_chunk_uw and qh_gdn_chunk_state; tokens need not be a multiple of 64 (the last
  * chunk's missing tokens count as zeros).  flags: QH_GDN_OUT_F32 (o as float32).  The query returns the
- * workspace's bytes, or 0 for shapes that qh_gdn_chunk_uw and qh_gdn_chunk_state_ws serve better. */
+ * workspace's bytes, or 0 for shapes that qh_gdn_chunk_uw and qh_gdn_chunk_state_ws serve better.  The
+ * results round differently from those of the two calls, and are nearer to float64: no product of
+ * QH_GDN_FP32 is a single bf16 one, as stage A's are, and QH_GDN_BF16 rounds v_new once. */
 size_t qh_gdn_prefill_workspace(uint32_t batch, uint32_t tokens, uint32_t heads, uint32_t precision);
 qh_status qh_gdn_prefill(const uint16_t *q_dev, const uint16_t *k_dev, const uint16_t *v_dev, const float *g_dev,
                          const float *beta_dev, const float *s_in_dev, float *s_out_dev, void *o_dev, uint32_t batch,

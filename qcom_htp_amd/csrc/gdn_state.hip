@@ -25,8 +25,9 @@
 // W, q and P lie in LDS in operand order (kpos): each half of a 32-deep product step's A operand is
 // one 16-byte read, with nothing to repack.  The kernel is bound by what its two waves per SIMD
 // issue and wait for; with W and P as hi | lo words (two reads and eight byte permutes an operand)
-// and a staging phase of its own between two more barriers it took 523 / 398 us (fp32 / bf16), now 505 / 387
-// (B = 8, T = 4096, H = 32; the bytes it moves take 365 / 257 us at the 5.2 TB/s of a large copy).
+// and a staging phase of its own between two more barriers the median launch took 529 / 367 us (fp32 /
+// bf16), now 524 / 363 (B = 8, T = 4096, H = 32; the bytes it moves take 365 / 257 us at the 5.2 TB/s of
+// a large copy).
 //
 // Prefill of many sequences (FROM_T) needs no W and U: they are T (beta e^g k^) and T (beta v), so
 //     v_new = T (beta v - beta e^g k^ S),
@@ -34,12 +35,15 @@
 // and T times the result is one more lower triangular product of a wave's own columns.  gdn_t_kernel
 // forms T (16 KB a chunk as hi / lo parts) from k, g and beta alone.  Stage A is bound by the 64 KB of W
 // and U that it writes per chunk in float32 (1.6 GB, 312 us), which stage B then reads again: B = 8,
-// T = 4096, H = 32 takes 130 + 538 us with T against 311 + 523 us (bf16: 117 + 411 against 229 + 392),
-// shortest launches; the prefill 822 -> 626 us.
+// T = 4096, H = 32 takes 136 + 560 us with T against 314 + 524 us (bf16: 111 + 399 against 228 + 363),
+// median launches of 30 in a row.
 //
 // Precision: QH_GDN_FP32 carries W, S, P and v_new as bf16 hi/lo splits (hi*hi + hi*lo + lo*hi,
 // fp32 accumulation; products with the exact q, k take two terms); QH_GDN_BF16 uses the hi
-// parts only; T's own products are split in both.  Norms, decays and the prefix sum are fp32.
+// parts only; T's own products and its right-hand side's parts are split in both.  Norms, decays and
+// the prefix sum are fp32.  (With the right-hand side rounded to bf16 as well, BF16's o from T was further
+// from 64 bits than from W and U, which round v_new once: 2.92e-3 against 2.54e-3 .. 2.90e-3; now 2.41e-3,
+// for 7 us of the 399 above.  FP32 is at 5.1e-6 from T, 3.4e-4 from stage A's bf16 products.)
 //
 // Few sequences (gdn_state_cols_kernel): the chunks of a sequence follow one another, so the launch
 // lasts as long as one sequence however few there are, and what counts is a chunk's latency.  The work
@@ -194,8 +198,8 @@ __device__ __forceinline__ void store_o(void *o, uint32_t at, uint32_t tok, int 
 }
 
 // acc[i] (or zero, with `fresh`) += sum over the token tiles j <= i of L_ij X_j, L lower triangular in
-// LDS in operand order (lo parts with SPLIT).
-template <bool SPLIT, int NL>
+// LDS in operand order (lo parts with SPLIT); XLO: with X's lo parts.
+template <bool SPLIT, bool XLO, int NL>
 __device__ __forceinline__ void lower_product(const uint16_t (&hi)[kC][kPs], const uint16_t (&lo)[NL][kPs], int r16, int qd,
                                               const Half4 (&x)[4], v4f (&acc)[4], bool fresh) {
 #pragma unroll
@@ -207,10 +211,8 @@ __device__ __forceinline__ void lower_product(const uint16_t (&hi)[kC][kPs], con
       const Half4 x1 = 2 * p + 1 <= i ? x[2 * p + 1] : kZero4;
       const v8bf l = op8(&hi[16 * i + r16][32 * p + 8 * qd]), xh = op_hi(x[2 * p], x1);
       s = mfma(l, xh, s);
-      if constexpr (SPLIT) {
-        s = mfma(l, op_lo(x[2 * p], x1), s);
-        s = mfma(op8(&lo[16 * i + r16][32 * p + 8 * qd]), xh, s);
-      }
+      if constexpr (XLO) s = mfma(l, op_lo(x[2 * p], x1), s);
+      if constexpr (SPLIT) s = mfma(op8(&lo[16 * i + r16][32 * p + 8 * qd]), xh, s);
     }
     acc[i] = s;
   }
@@ -416,8 +418,8 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       Half4 rB[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) rB[j] = split4<SPLIT>(vnew[j]);
-      lower_product<SPLIT>(Th, Tl, r16, qd, rB, vnew, true);
+      for (int j = 0; j < 4; ++j) rB[j] = split4<true>(vnew[j]);  // (with lo parts in both precisions)
+      lower_product<SPLIT, true>(Th, Tl, r16, qd, rB, vnew, true);
       // (formed here: moved behind the P loop, its 12 operand reads would stay in registers across it)
 #pragma unroll
       for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(vnew[i]));
@@ -483,7 +485,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
     Half4 vB[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) vB[j] = split4<SPLIT>(vnew[j]);
-    lower_product<SPLIT>(Ph, Po, r16, qd, vB, oacc, false);
+    lower_product<SPLIT, SPLIT>(Ph, Po, r16, qd, vB, oacc, false);
     if constexpr (FROM_T) __builtin_amdgcn_sched_barrier(0);
     uint32_t oo = 4 * qd * tok + col;
     asm volatile("" : "+v"(oo));

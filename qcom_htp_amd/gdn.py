@@ -175,8 +175,11 @@ def gdn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tens
     (scripts/gdn_ref_kernel.py:104-131): q, k, v bf16 [B, T, H, 128], g (per-token log decay) and
     beta float32 [B, T, H] -> (o [B, T, H, 128], S [B, H, 128, 128] float32).  The missing tokens
     of a last partial chunk of 64 count as zeros, which leaves o and S unchanged.  Few sequences
-    run stages A (float32 W, U for ``FP32``, bf16 for ``BF16``) and B; many take the recurrence
-    from T = (I - A)^-1, without W and U."""
+    (B * H <= 64 on 256 compute units) run stages A (float32 W, U for ``FP32``, bf16 for ``BF16``)
+    and B; many take the recurrence from T = (I - A)^-1, without W and U.  The two round
+    differently: a sequence's bits may differ between a call of few and one of many sequences,
+    by less than stage A's bf16 products are from float64 (3.4e-4 of o in ``FP32``; o from T is
+    within 5.1e-6).  Within one of the two they do not depend on the other sequences."""
     B, T, H, D = q.shape
     _same_device(q.device, k=k, v=v, g=g, beta=beta, initial_state=initial_state)
     ragged = _lib.QH_GDN_RAGGED if T % STATE_CHUNK else 0
