@@ -512,8 +512,10 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
     return D;
   };
   if constexpr (C::kRound) {
-    // rint by adding 1.5 * 2^52 after a clamp to [-1, qmax + 1] (outside, both candidate roundings
-    // clip to the same output)
+    // rint by adding 1.5 * 2^52 after a clamp to [-1, qmax + 1].  An output that is not certain is
+    // listed unless it clips to the same end over the whole error bound 0.5 - th, which can be any
+    // number of steps: below t = th (above qmax - th) it does, and from 2 th - 1 on also with the
+    // rounding of t itself.
     constexpr double kMagic = 6755399441055744.0;
     const double qmaxd = static_cast<double>(g.out_qmax);
     double al[4], be[4], th[4];
@@ -524,21 +526,22 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
       th[e] = ctab[2 * TC + c4 + e];
     }
     outputs([&](int r, int (&o)[4]) __attribute__((always_inline)) {
-      int oi[4];
+      double u[4];
       bool sure[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const double tv = fmin(fmax(fma(static_cast<double>(sums[r * TC + c4 + e]), al[e], be[e]), -1.0), qmaxd + 1.0);
+        u[e] = fma(static_cast<double>(sums[r * TC + c4 + e]), al[e], be[e]);
+        const double tv = fmin(fmax(u[e], -1.0), qmaxd + 1.0);
         const double y = tv + kMagic;
-        oi[e] = __double2loint(y);
         sure[e] = fabs(tv - (y - kMagic)) <= th[e];  // (a threshold that is not a number lists the output)
-        o[e] = min(max(oi[e], 0), g.out_qmax);
+        o[e] = min(max(__double2loint(y), 0), g.out_qmax);
       }
       if (!(sure[0] & sure[1] & sure[2] & sure[3])) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (!sure[e] && static_cast<uint32_t>(oi[e]) <= static_cast<uint32_t>(g.out_qmax))
-            list[atomicAdd(&fix_cnt, 1)] = static_cast<uint16_t>(r * TC + c4 + e);
+        for (int e = 0; e < 4; ++e) {
+          const double end = 2.0 * th[e] - 1.0;
+          if (!sure[e] && !(u[e] < end) && !(u[e] > qmaxd - end)) list[atomicAdd(&fix_cnt, 1)] = static_cast<uint16_t>(r * TC + c4 + e);
+        }
       }
     });
   } else if constexpr (MODE == kAccumulate) {

@@ -81,6 +81,42 @@ def test_per_group(gpu, fam, mkng, span):
     assert np.array_equal(got, want.astype(got.dtype)), f"{(got != want).sum()} of {got.size} differ"
 
 
+@pytest.mark.parametrize("ob", [8, 16], ids=["o8", "o16"])
+@pytest.mark.parametrize("zp", ["low", "mid", "high"])
+@pytest.mark.parametrize("ab,span", [(8, 20), (8, 25), (8, 28), (16, 14), (16, 17), (16, 20)], ids=lambda v: str(v))
+def test_per_group_outputs_far_below_a_group_of_large_scale(gpu, ab, span, zp, ob):
+    """Group scales 2^14 to 2^28 apart (the widest that prepare accepts), where the int32 multipliers round the small ones away, with the large
+    group's activations at the zero point: the sums that the kernel forms are then off by many steps of
+    the output, and each output whose error bound reaches the output range has to be recomputed, however
+    far outside that range its sum lies."""
+    import torch
+
+    from qcom_htp_amd import _lib
+    from qcom_htp_amd.qmm import QuantMatmul
+
+    m, k, n = 70, 192, 96
+    rng = np.random.default_rng(span + ab)
+    azp = {"low": 0, "mid": 1 << (ab - 1), "high": (1 << ab) - 1}[zp]
+    x = np.full((m, k), azp, dtype=np.int64)
+    x[:, 64:128] = np.clip(azp + rng.integers(-30, 31, size=(m, 64)), 0, (1 << ab) - 1)
+    w = rng.integers(-7, 8, size=(n, k)).astype(np.int8)
+    w[: n // 2, :64] = 0
+    w[: n // 2, 0] = 1  # one code in the large group; the other channels have 64 codes in one 2^-9 as large
+    s = np.float32(rng.uniform(4e-3, 7e-3, size=(n, 3))) * np.float32([2.0 ** span, 1.0, 1.0])
+    s[n // 2 :, 0] *= np.float32(2.0 ** -9)
+    deq = w.astype(np.float32) * np.repeat(s, 64, axis=1)
+    t = ((x - azp) * 0.02) @ deq.astype(np.float64).T
+    q = (1 << ob) - 1
+    so = float(np.abs(t).max()) / q * 1.5  # some outputs clip at either end
+    ozp = q // 3
+    want = np.clip(np.rint(t / so + ozp), 0, q)
+    op = QuantMatmul(w, s, np.zeros(n, np.int32), act_bits=ab, out_bits=ob, act_scale=0.02, out_scale=so, act_zp=azp, out_zp=ozp,
+                     weight_format=_lib.QH_WEIGHT_I4_GROUP, bias_float=np.zeros(n, np.float32), device=gpu)
+    got = op(torch.from_numpy(x.astype(np.uint16 if ab == 16 else np.uint8)).to(gpu)).cpu().numpy()
+    op.close()
+    assert np.array_equal(got, want.astype(got.dtype)), f"{(got != want).sum()} of {got.size} differ"
+
+
 @pytest.mark.parametrize("tie", [False, True], ids=["random", "ties"])
 @pytest.mark.parametrize("mkn", [(17, 32, 32), (33, 160, 96), (65, 1184, 1088), (130, 4096, 480), (700, 288, 2080)],
                          ids=lambda s: "x".join(map(str, s)))
