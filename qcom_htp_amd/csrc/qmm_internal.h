@@ -107,7 +107,8 @@ struct QmmDevice {
   int32_t *bias_q;  // [Np] the descriptor's int32 bias (integer contracts)
   int64_t *corr_int; // [Np] activation-shift term of the exact integer dot product sum (a - zp) w_int
   // Per-group weights (qmm_tile.hip): the group scales as int32 multiples of one unit per channel
-  // (16-bit acts: a second plane for 256 times the high byte's residue sum) [planes][G][Np], and per
+  // (a second plane for the residue sums: 256 times the high byte's for 16-bit acts; for 8-bit acts
+  // with group_resid) [planes][G][Np], and per
   // channel the largest |t - rint(t)| that certifies the rounding; alpha_e is output LSB per unit and
   // beta includes the activation shift's term.  The float32 group scales serve the float64
   // recomputation.
@@ -137,6 +138,7 @@ struct QmmShape {
   long long int_mult[2];
   int int_ones;
   int groups, group_shift;
+  int group_resid;    // per-group, 8-bit acts: the tile kernel forms the residue products too
 };
 
 // Arguments of the one-launch chains (qmm_exact.hip).

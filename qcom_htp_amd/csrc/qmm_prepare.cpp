@@ -128,7 +128,7 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
   std::vector<int64_t> corr_int(Np, 0);
   std::vector<int32_t> biasv(Np, 0);
   std::vector<int32_t> mult;
-  std::vector<double> alpha_e(Np, 0.0), beta(Np, 0.0), thr(Np, 0.0), bdeq(Np, 0.0);
+  std::vector<double> alpha_e(Np, 0.0), beta(Np, 0.0), thr(Np, 0.0), thr_r(Np, 0.0), bdeq(Np, 0.0);
   std::vector<float> s32g;
   for (int n = 0; n < N; ++n) biasv[n] = d->bias_q ? d->bias_q[n] : 0;
   if (!group) {
@@ -152,7 +152,8 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
     sh.int_mult[0] = 1;
     sh.int_mult[1] = 0;
     sh.int_ones = 0;
-    mult.assign(static_cast<size_t>(a16 ? 2 : 1) * G * Np, 0);
+    mult.assign(static_cast<size_t>(2) * G * Np, 0);
+    double uncertain = 0.0;  // 8-bit acts: expected outputs per row that the left-out residues make uncertain
     s32g.assign(static_cast<size_t>(N) * G, 1.0f);
     const double sA = d->act_scale, sO = d->out_scale;
     std::vector<int64_t> Mg(G), m0s(G), m1s(G);
@@ -231,27 +232,38 @@ qh_status prepare_exact(const qh_qmm_desc *d, qh_qmm_prepared **out) {
       double rounded = 0.0;  // bound of what the rounded multipliers change, units of 2^E_min
       for (int g = 0; g < G; ++g) {
         mult[static_cast<size_t>(g) * Np + n] = static_cast<int32_t>(std::rint(static_cast<double>(m0s[g]) / unit));
-        if (a16) mult[(static_cast<size_t>(G) + g) * Np + n] = static_cast<int32_t>(std::rint(256.0 * static_cast<double>(m1s[g]) / unit));
+        mult[(static_cast<size_t>(G) + g) * Np + n] = static_cast<int32_t>(std::rint((a16 ? 256.0 : 1.0) * static_cast<double>(m1s[g]) / unit));
         double aq = 0.0, ar = 0.0;
         for (int k = g * gsz; k < (g + 1) * gsz && u > 0; ++k) {
           aq += std::abs(static_cast<int>(d->weight_nk[static_cast<size_t>(n) * K + k]));
           ar += 127.0;
         }
-        rounded += half * (a16 ? 33024.0 * aq + 128.0 * ar : 128.0 * aq);
+        rounded += half * (a16 ? 33024.0 * aq + 128.0 * ar : 128.0 * (aq + ar));
       }
       alpha_e[n] = ae * unit;
       // The kernel's t = alpha_e sum_g S_g mult_g + beta leaves out the residue products of the
-      // shifted activations (8 bits: |a - 128| <= 128; 16 bits: of the low byte, |lo'| <= 128), rounds
-      // the multipliers to their unit and makes a few float64 roundings; the oracle's own float64
-      // noise is K roundings of terms bounded by amax 2^E_min sum_abs / K.  rint(t) is certain while
-      // |t - rint(t)| stays below this threshold.
-      const double left_out = (128.0 * sum_r + rounded) * ae;
+      // shifted activations (8 bits without group_resid: |a - 128| <= 128; 16 bits: of the low byte,
+      // |lo'| <= 128), rounds the multipliers to their unit and makes a few float64 roundings; the
+      // oracle's own float64 noise is K roundings of terms bounded by amax 2^E_min sum_abs / K.
+      // rint(t) is certain while |t - rint(t)| stays below this threshold.
+      const double left_out = 128.0 * sum_r * ae;
       const double noise = (K + 8.0) * std::ldexp(1.0, -52) * amax * sum_abs * ae;
       const double size = (a16 ? 33024.0 : 128.0) * (sum_abs + sum_r) * ae + std::fabs(shift) + 2.0 * std::fabs(off) +
                           2.0 * d->out_zp + ((1 << d->out_bits) + 2.0);
       const double own = 16.0 * std::ldexp(1.0, -52) * size + std::ldexp(1.0, -48) * (std::fabs(off) + (1 << d->out_bits));
-      thr[n] = 0.5 - (left_out + noise + own) * kSafety;
+      thr[n] = 0.5 - (left_out + rounded * ae + noise + own) * kSafety;
+      thr_r[n] = 0.5 - (rounded * ae + noise + own) * kSafety;
+      uncertain += std::min(1.0, 2.0 * left_out);
     }
+    // Forming the residues too costs about half as much again as the code products; without them an
+    // output within left_out of a rounding boundary is recomputed in float64 by a whole wave.  u8 to u16,
+    // 500 x 4096 x 4096, at 0.04 / 0.15 / 0.3 / 0.6 / 1.2 / 9 % of the outputs expected uncertain (the last
+    // with an output scale that fits the range): 22 / 27 / 32 / 42 / 62 / 272 us without, 31 to 34 us with;
+    // 2000 x 2048 x 2048: 25 / 29 / 33 / 40 / 59 / 232 against 35 to 37.  8-bit outputs whose left_out is
+    // that large clip, all but a few: 23 us at most.
+    sh.group_resid = !a16 && d->out_bits == 16 && uncertain > N / 256.0;
+    if (sh.group_resid) thr = thr_r;
+    if (!a16 && !sh.group_resid) mult.resize(static_cast<size_t>(G) * Np);
   }
   auto *p = new qh_qmm_prepared();
   p->shape = sh;

@@ -30,8 +30,9 @@
 // channel's scales span too far), and every 64 k the exact int32 S_g goes into an int64 sum by one
 // 32 x 32 + 64-bit multiply-add per output: the loop is bound by those (at two waves per SIMD an
 // instruction issues every 2.4 to 2.7 ns; a float64 sum took two, an int64 multiplier about ten).
-// 8-bit activations leave R_g out and bound it; 16-bit ones form the high byte's part as a third
-// product and bound the low byte's.  An output closer to a rounding boundary than that bound and
+// 8-bit activations leave R_g out and bound it while few outputs are uncertain for it, and else form it
+// as a second product (prepare_exact's rule); 16-bit ones form the high byte's part as a third product
+// and bound the low byte's.  An output closer to a rounding boundary than that bound and
 // the roundings is listed and recomputed as the oracle forms its dot product (float64 products of
 // fl64((a - zp) sA) and fl32(q s_g)).
 // Per-channel requantisation is the same with one group: 8-bit activations keep the code products
@@ -368,6 +369,11 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
             if constexpr (!A16) {
               dacc[0][j] += acc[0][0][j] * c0;
               dacc[kGB - 1][j] += acc[1][0][j] * c0;
+              if constexpr (PL2) {
+                const long long c1 = r.c[s >> 1][C::kPlanes - 1];
+                dacc[0][j] += acc[0][NT - 1][j] * c1;
+                dacc[kGB - 1][j] += acc[1][NT - 1][j] * c1;
+              }
             } else {
               // c1 carries the residue plane's multiplier times 256 (the high byte's weight)
               const long long c1 = r.c[s >> 1][C::kPlanes - 1];
@@ -618,7 +624,10 @@ long long tile_count(int m, int n, bool a16, int cols, int ks) {
 template <bool A16, int NT, bool PL2, int MODE>
 qh_status pick_split(const TileArgs &g, hipStream_t stream) {
   const int cus = device_cu_count(), cols = PL2 ? 32 : 32 * NT;
-  if (g.KT >= 8 && tile_count(g.M, g.N, A16, cols, 8) <= cus) return launch<A16, NT, PL2, MODE, 8>(g, stream);
+  // (8-bit activations with both planes' group sums: eight groups spill 60 registers)
+  if constexpr (!(!A16 && PL2 && MODE == kGroup)) {
+    if (g.KT >= 8 && tile_count(g.M, g.N, A16, cols, 8) <= cus) return launch<A16, NT, PL2, MODE, 8>(g, stream);
+  }
   if (tile_count(g.M, g.N, A16, cols, 4) <= cus) return launch<A16, NT, PL2, MODE, 4>(g, stream);
   return launch<A16, NT, PL2, MODE, 2>(g, stream);
 }
@@ -688,7 +697,10 @@ qh_status launch_qmm_tile(const qh_qmm_prepared *p, int m, const void *act, void
   }
   const bool a16 = sh.act_bits == 16, w16 = sh.int_planes == 2;
   if (mode == kTileRequant) return a16 ? pick_split<true, 2, true, kRequant>(g, stream) : pick_split<false, 2, false, kRequant>(g, stream);
-  if (mode == kTileGroup) return a16 ? pick_split<true, 2, true, kGroup>(g, stream) : pick_split<false, 1, false, kGroup>(g, stream);
+  if (mode == kTileGroup) {
+    if (a16) return pick_split<true, 2, true, kGroup>(g, stream);
+    return sh.group_resid ? pick_split<false, 2, true, kGroup>(g, stream) : pick_split<false, 1, false, kGroup>(g, stream);
+  }
   if (mode == kTileAccumulate) {
     if (w16) return a16 ? pick_split<true, 2, true, kAccumulate>(g, stream) : pick_split<false, 2, true, kAccumulate>(g, stream);
     return a16 ? pick_split<true, 2, false, kAccumulate>(g, stream) : pick_split<false, 2, false, kAccumulate>(g, stream);

@@ -81,6 +81,77 @@ def test_per_group(gpu, fam, mkng, span):
     assert np.array_equal(got, want.astype(got.dtype)), f"{(got != want).sum()} of {got.size} differ"
 
 
+def per_group_8_to_16(m, k, n, gsz, span, coarse, tie, rng):
+    """Operands of u8 activations, per-group int4 weights and u16 outputs; coarse: an output scale that
+    uses a 2^-8 of the range; tie: odd dot products of the first rows on half-integers."""
+    x = np.clip(np.rint(rng.normal(128.0, 40.0, size=(m, k))), 0, 255).astype(np.uint8)
+    w = rng.integers(-7, 8, size=(n, k)).astype(np.int8)
+    s = (rng.uniform(1e-3, 1e-2, size=(n, k // gsz)) * 2.0 ** rng.integers(-span, 1, size=(n, k // gsz))).astype(np.float32)
+    sa, bias = 0.02, rng.uniform(-0.5, 0.5, size=n).astype(np.float32)
+    if tie:
+        sa, s = 2.0 ** -7, np.full_like(s, 2.0 ** -8)
+        bias = (rng.integers(-8, 8, size=n) * (sa * 2.0 ** -8)).astype(np.float32)
+        for r in range(min(m, 40)):
+            x[r] = 128
+            x[r, rng.choice(k, size=5, replace=False)] = 128 + rng.integers(-3, 4, size=5)
+    t = ((x.astype(np.float64) - 128.0) * sa) @ (w.astype(np.float32) * np.repeat(s, gsz, axis=1)).astype(np.float64).T + bias
+    so = 2.0 * sa * 2.0 ** -8 if tie else float(np.abs(t).max()) / 32767.0 * (256.0 if coarse else 1.0)
+    return x, w, s, sa, bias, so, np.clip(np.rint(t / so + 32768.0), 0, 65535).astype(np.uint16)
+
+
+def per_group_8_to_16_op(gpu, n, w, s, sa, bias, so, ob=16):
+    from qcom_htp_amd import _lib
+    from qcom_htp_amd.qmm import QuantMatmul
+
+    return QuantMatmul(w, s, np.zeros(n, np.int32), act_bits=8, out_bits=ob, act_scale=sa, out_scale=so, act_zp=128,
+                       out_zp=1 << (ob - 1), weight_format=_lib.QH_WEIGHT_I4_GROUP, bias_float=bias, device=gpu)
+
+
+@pytest.mark.parametrize("span,coarse,tie", [(0, False, False), (10, False, False), (0, True, False), (0, False, True)],
+                         ids=["fitted", "wide_scales", "coarse", "ties"])
+@pytest.mark.parametrize("mkng", [(1, 256, 32, 128), (33, 192, 96, 64), (65, 2048, 352, 1024), (130, 4096, 480, 256),
+                                  (700, 320, 2080, 64)], ids=lambda s: "x".join(map(str, s)))
+def test_per_group_8_bit_to_16_bit(gpu, mkng, span, coarse, tie):
+    """8-bit activations and 16-bit outputs, with the residue products (where many outputs would be
+    uncertain without them) and without (a coarse output scale), at each number of K groups."""
+    import torch
+
+    m, k, n, gsz = mkng
+    x, w, s, sa, bias, so, want = per_group_8_to_16(m, k, n, gsz, span, coarse, tie, np.random.default_rng(m + k))
+    op = per_group_8_to_16_op(gpu, n, w, s, sa, bias, so)
+    got = op(torch.from_numpy(x).to(gpu), out=unaligned(gpu, m, n, op.out_dtype)).cpu().numpy()
+    op.close()
+    assert np.array_equal(got, want), f"{(got != want).sum()} of {got.size} differ"
+
+
+def test_per_group_16_bit_outputs_cost_little_more_than_8_bit_ones(gpu):
+    """The time does not depend on how fine the output scale is: 12 against 10 us where recomputing every
+    output that the left-out residues make uncertain took 65."""
+    import torch
+
+    m, k, n = 500, 2048, 2048
+    x, w, s, sa, bias, so, _ = per_group_8_to_16(m, k, n, 64, 0, False, False, np.random.default_rng(1))
+    act = torch.from_numpy(x).to(gpu)
+
+    def best(ob):
+        op = per_group_8_to_16_op(gpu, n, w, s, sa, bias, so * 2.0 ** (16 - ob), ob)
+        times = []
+        for _ in range(6):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(50):
+                op(act)
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1) * 20.0)
+        op.close()
+        return min(times)
+
+    t8, t16 = best(8), best(16)
+    print(f"[tile] per-group {m}x{k}x{n}: u8 outputs {t8:.1f} us, u16 outputs {t16:.1f} us", flush=True)
+    assert t16 <= 3.0 * t8
+
+
 @pytest.mark.parametrize("ob", [8, 16], ids=["o8", "o16"])
 @pytest.mark.parametrize("zp", ["low", "mid", "high"])
 @pytest.mark.parametrize("ab,span", [(8, 20), (8, 25), (8, 28), (16, 14), (16, 17), (16, 20)], ids=lambda v: str(v))
