@@ -219,7 +219,10 @@ __device__ __forceinline__ void lower_product(const uint16_t (&hi)[kC][kPs], con
 }
 
 // FROM_T: v_new = T (beta v - beta e^g K^ S) from gdn_t_kernel's T instead of U - W S.
-template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED, bool FROM_T>
+// ONE: the sequence is one whole chunk, and nothing is loaded or staged for a next one (a uniform branch
+// around that in the same kernel spills 20 to 100 registers).  Sequences past the compute units run in
+// rounds of one workgroup per unit: 1280 of them 56 us against 66 (fp32) and 44 against 51 (bf16).
+template <bool SPLIT, bool WU_F32, bool OUT_F32, bool RAGGED, bool FROM_T, bool ONE = false>
 __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
   static_assert(!(FROM_T && WU_F32), "v is bf16");
   constexpr bool kWlo = SPLIT && WU_F32;  // a bf16 W has no lo part
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
     if constexpr (SPLIT) reinterpret_cast<uint32_t *>(Po)[x] = 0u;
   }
   stage(0);
-  load(min(1, a.nchunks - 1));
+  if constexpr (!ONE) load(min(1, a.nchunks - 1));
   lds_barrier();
 
   auto chunk = [&](const int n) __attribute__((always_inline)) {
@@ -424,7 +427,7 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(vnew[i]));
     }
-    load_u(min(n + 1, a.nchunks - 1));
+    if constexpr (!ONE) load_u(min(n + 1, a.nchunks - 1));
     for (int idx = kThreads / 64 - 1 - wave; idx < 10; idx += kThreads / 64) {  // wave-uniform
       int ti, tj;
       p_tile(idx, ti, tj);
@@ -496,14 +499,18 @@ __global__ __launch_bounds__(kThreads) void gdn_state_kernel(StateArgs a) {
     // ---- the next chunk's rows.  Unconditional (the last chunk stages and loads itself again,
     // unused): behind a branch the compiler would lose count of the loads in flight and wait for every
     // memory operation, the o stores included.
-    stage(n + 1);
-    load(min(n + 2, a.nchunks - 1));
-    lds_barrier();
+    if constexpr (!ONE) {
+      stage(n + 1);
+      load(min(n + 2, a.nchunks - 1));
+      lds_barrier();
+    }
   };
   // Chunk 0 runs on its own: then every path into the loop has the same memory operations in
   // flight, and the compiler's wait before the first use of the loads counts only them.
   chunk(0);
-  for (int n = 1; n < a.nchunks; ++n) chunk(n);
+  if constexpr (!ONE) {
+    for (int n = 1; n < a.nchunks; ++n) chunk(n);
+  }
 
 #pragma unroll
   for (int kb = 0; kb < 8; ++kb) {
@@ -982,6 +989,8 @@ qh_status launch4(const StateArgs &a, hipStream_t stream) {
       hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, 2, true>), dim3(grid2), dim3(kColThreads), 0, stream, a);
   } else if (grid2)
     hipLaunchKernelGGL((gdn_state_cols_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, 2, false>), dim3(grid2), dim3(kColThreads), 0, stream, a);
+  else if (!RAGGED && a.nchunks == 1)
+    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32, false, false, true>), dim3(seqs), dim3(kThreads), 0, stream, a);
   else
     hipLaunchKernelGGL((gdn_state_kernel<SPLIT, WU_F32, OUT_F32, RAGGED, false>), dim3(seqs), dim3(kThreads), 0, stream, a);
   hipError_t err = hipGetLastError();
@@ -1001,10 +1010,18 @@ qh_status launch_prefill2(const StateArgs &a, bool out_f32, hipStream_t stream) 
   hipLaunchKernelGGL((gdn_t_kernel<SPLIT, RAGGED>), dim3(seqs * a.nchunks), dim3(kTThreads), 0, stream, a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return hip_fail(err, "gdn_t_kernel launch");
-  if (out_f32)
-    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, false, true, RAGGED, true>), dim3(seqs), dim3(kThreads), 0, stream, a);
-  else
-    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, false, false, RAGGED, true>), dim3(seqs), dim3(kThreads), 0, stream, a);
+  auto recurrence = [&](auto out32, auto one) {
+    hipLaunchKernelGGL((gdn_state_kernel<SPLIT, false, decltype(out32)::value, RAGGED, true, decltype(one)::value>), dim3(seqs),
+                       dim3(kThreads), 0, stream, a);
+  };
+  auto by_chunks = [&](auto out32) {
+    if constexpr (!RAGGED) {
+      if (a.nchunks == 1) return recurrence(out32, std::true_type{});
+    }
+    recurrence(out32, std::false_type{});
+  };
+  if (out_f32) by_chunks(std::true_type{});
+  else by_chunks(std::false_type{});
   err = hipGetLastError();
   if (err != hipSuccess) return hip_fail(err, "gdn_state_kernel launch");
   return QH_STATUS_OK;

@@ -337,6 +337,31 @@ def test_ragged_prefill_equals_zero_padded(gpu, T, H, precision, out):
     assert torch.equal(o, o_ref[:, :T]) and torch.equal(s, s_ref)
 
 
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("route", ["wu_f32", "wu_bf16", "from_t"])
+def test_one_chunk_of_many_sequences(gpu, route, precision, out):
+    """The kernels without a next chunk give the bits of the looping ones: the first chunk of two, and S
+    handed over after it."""
+    import torch
+
+    from qcom_htp_amd.gdn import gdn_chunk_state, gdn_chunk_uw, gdn_prefill
+
+    B, T, H = 1, 128, 70
+    q, k, v, bt, g = (to_dev(x, gpu) for x in seq_inputs(B, T, H, seed=19))
+    s0 = torch.randn((B, H, 128, 128), generator=torch.Generator(device=gpu).manual_seed(3), device=gpu)
+    odt = torch.float32 if out == "f32" else torch.bfloat16
+    if route == "from_t":
+        args, run = (q, k, v, g, bt), lambda a, s: gdn_prefill(*a, s, precision, odt)
+    else:
+        w, u = gdn_chunk_uw(k, v, g, bt, 64, decay_w=True, out_dtype=torch.float32 if route == "wu_f32" else torch.bfloat16)
+        args, run = (q, k, g, w, u), lambda a, s: gdn_chunk_state(*a, s, precision, odt)
+    o, S = run(args, s0)
+    o1, S1 = run([x[:, :64].contiguous() for x in args], s0)
+    o2, S2 = run([x[:, 64:].contiguous() for x in args], S1)
+    assert torch.equal(o1, o[:, :64]) and torch.equal(o2, o[:, 64:]) and torch.equal(S2, S)
+
+
 def test_ragged_prefill_takes_strided_and_unaligned_inputs(gpu):
     import torch
 
