@@ -40,6 +40,7 @@
 // output first gets its missing residue sum exactly (a dot product over the residue plane or
 // column), then the float64 recomputation if it still lies within the oracle's own noise.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "qmm_contract.h"
@@ -594,17 +595,27 @@ __global__ __launch_bounds__(kTlThreads, 1) void qmm_tile_kernel(const TileArgs 
   }
 }
 
+// Most workgroups of one launch: its threads are counted in 32 bits (a larger grid is cut short without
+// an error), in whole rounds over the XCDs.
+constexpr long long kMaxBlocks = 0xFFFFFFFFLL / kTlThreads / 8 * 8;
+
 template <bool A16, int NT, bool PL2, int MODE, int KS>
-qh_status launch(TileArgs g, hipStream_t stream) {
+qh_status launch(const TileArgs &whole, hipStream_t stream) {
   using C = TileCfg<A16, NT, PL2, MODE, KS>;
-  const long long tm = (static_cast<long long>(g.M) + C::RB - 1) / C::RB, tn = (g.N + C::TC - 1) / C::TC;
-  const long long blocks = (tm * tn + 7) / 8 * 8;  // whole rounds over the XCDs
-  if (blocks > 0x7FFFFFFFLL) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "M=%d too large for one launch", g.M);
-  g.TM = static_cast<int>(tm);
-  g.TN = static_cast<int>(tn);
-  hipLaunchKernelGGL((qmm_tile_kernel<A16, NT, PL2, MODE, KS>), dim3(static_cast<unsigned>(blocks)), dim3(kTlThreads), 0, stream, g);
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return hip_fail(err, "qmm_tile_kernel launch");
+  const long long tn = (whole.N + C::TC - 1) / C::TC, rows = kMaxBlocks / tn * C::RB;  // rows of one launch
+  const size_t out_row = static_cast<size_t>(whole.N) * (MODE == kAccumulate ? 8 : whole.out16 ? 2 : 1);
+  for (long long m0 = 0; m0 < whole.M; m0 += rows) {
+    TileArgs g = whole;
+    g.M = static_cast<int>(std::min(rows, whole.M - m0));
+    g.act += static_cast<size_t>(m0) * whole.K * (A16 ? 2 : 1);
+    g.out = static_cast<uint8_t *>(whole.out) + static_cast<size_t>(m0) * out_row;
+    g.TM = (g.M + C::RB - 1) / C::RB;
+    g.TN = static_cast<int>(tn);
+    const long long blocks = (static_cast<long long>(g.TM) * tn + 7) / 8 * 8;  // whole rounds over the XCDs
+    hipLaunchKernelGGL((qmm_tile_kernel<A16, NT, PL2, MODE, KS>), dim3(static_cast<unsigned>(blocks)), dim3(kTlThreads), 0, stream, g);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return hip_fail(err, "qmm_tile_kernel launch");
+  }
   return QH_STATUS_OK;
 }
 

@@ -217,3 +217,30 @@ def test_requantised_few_tiles(gpu, fam, mkn, tie):
     op.close()
     want = oq.expected_output_case(c)
     assert np.array_equal(got, want), f"{(got != want).sum()} of {got.size} differ"
+
+
+def test_more_tiles_than_one_launch_holds(gpu):
+    """2^35 outputs: their 32 x 128 tiles of 512 threads are more than the 2^32 threads of a launch, so the
+    rows are shared out over two.  The activations repeat every 64 rows, and so must the outputs."""
+    import torch
+
+    from qcom_htp_amd import _lib
+    from qcom_htp_amd.qmm import QuantMatmul
+
+    m, k, n, per = 65535 * 64, 32, 8224, 64
+    if torch.cuda.mem_get_info(gpu)[0] < 2 * m * n * 3 // 2:
+        pytest.skip("needs 104 GB of device memory")
+    rng = np.random.default_rng(1)
+    w = rng.integers(-32768, 32768, size=(n, k)).astype(np.int16)
+    x = rng.integers(0, 65536, size=(per, k)).astype(np.uint16)
+    op = QuantMatmul(w, np.ones(n, np.float32), np.zeros(n, np.int32), act_bits=16, out_bits=16, act_scale=1.0, out_scale=1.0,
+                     act_zp=32768, out_zp=32768, weight_format=_lib.QH_WEIGHT_I16, device=gpu)
+    act = torch.from_numpy(x.view(np.int16)).to(gpu).repeat(m // per, 1).view(torch.uint16)
+    out = op.run_contract(act, "div_rint", 1 << 18).view(torch.int16).view(m // per, per * n)
+    differ = sum(int((out[i:i + 4096] != out[0]).any(dim=1).sum()) for i in range(0, m // per, 4096))
+    first = out[0].cpu().numpy().view(np.uint16).reshape(per, n)
+    op.close()
+    del out, act
+    torch.cuda.empty_cache()
+    assert np.array_equal(first, oq.contract_output(oq.int_accumulator(x, w, 32768), "div_rint", 1 << 18, None, 32768, 16))
+    assert differ == 0, f"{differ} of {m // per} blocks of rows differ"
