@@ -107,6 +107,47 @@ def test_run_rejects_null_and_bad_shapes(qhtp_lib):
     assert L.qh_gdn_solve_u16(8, 16, 1, 64, 0, 0, 1.0, 1.0, 0, None) == _lib.QH_STATUS_INVALID_ARGUMENT
 
 
+def test_gdn_prefill_rejects_bad_arguments(qhtp_lib):
+    """Every refusal comes before a launch (the buffers are made-up addresses)."""
+    L, INV, UNS, SHP = qhtp_lib, _lib.QH_STATUS_INVALID_ARGUMENT, _lib.QH_STATUS_UNSUPPORTED, _lib.QH_STATUS_SHAPE_UNSUPPORTED
+    B, T, H = 4, 100, 32  # more sequences than any device runs on the route of few
+    need = L.qh_gdn_prefill_workspace(B, T, H, _lib.QH_GDN_FP32)
+    assert need == B * H * 2 * 2 * 64 * 64 * 2  # two chunks' T, hi and lo parts
+    assert L.qh_gdn_prefill_workspace(B, T, H, _lib.QH_GDN_BF16) == need // 2
+    names = ("q", "k", "v", "g", "beta", "s_in", "s_out", "o", "batch", "tokens", "heads", "head_dim", "flags", "precision", "ws",
+             "ws_bytes", "stream")
+    good = dict(zip(names, (4096, 4096, 4096, 4096, 4096, 0, 8192, 4096, B, T, H, 128, 0, 0, 16384, need, None)))
+    bad = [(dict([(p, None)]), INV) for p in ("q", "k", "v", "g", "beta", "s_out", "o", "ws")]
+    bad += [(dict([(p, 4104)]), INV) for p in ("q", "k", "v", "s_in", "s_out", "o", "ws")]
+    bad += [({"s_in": 8192}, INV), ({"ws_bytes": need - 1}, INV), ({"ws_bytes": 0}, INV), ({"head_dim": 64}, SHP),
+            ({"flags": _lib.QH_GDN_RAGGED}, UNS), ({"flags": _lib.QH_GDN_WU_F32}, UNS), ({"flags": 1 << 31}, UNS),
+            ({"precision": _lib.QH_GDN_OP_MODEL}, UNS), ({"batch": 0}, SHP), ({"tokens": 0}, SHP), ({"heads": 0}, SHP),
+            ({"tokens": 1 << 24}, SHP), ({"batch": 1 << 31, "heads": 1 << 31}, SHP)]
+    for change, status in bad:
+        args = {**good, **change}
+        assert L.qh_gdn_prefill(*(args[n] for n in names)) == status, change
+        assert L.qh_last_error().decode().startswith("qh_gdn_prefill")
+
+
+def test_gdn_chunk_rejects_bad_ragged_and_workspace_arguments(qhtp_lib):
+    L, INV, UNS, SHP = qhtp_lib, _lib.QH_STATUS_INVALID_ARGUMENT, _lib.QH_STATUS_UNSUPPORTED, _lib.QH_STATUS_SHAPE_UNSUPPORTED
+    uw = lambda T, chunk, flags: L.qh_gdn_chunk_uw(4096, 4096, 4096, 4096, 4096, 4096, 1, T, 1, 128, chunk, flags, None)  # noqa: E731
+    assert uw(100, 64, 0) == SHP
+    assert uw(0, 64, _lib.QH_GDN_RAGGED) == SHP
+    assert uw(100, 128, _lib.QH_GDN_RAGGED) == UNS and uw(256, 256, _lib.QH_GDN_RAGGED) == UNS
+
+    def state(T=64, flags=0, s_in=0, ws=0, ws_bytes=0, chunk=64):
+        return L.qh_gdn_chunk_state_ws(4096, 4096, 4096, 4096, 4096, s_in, 8192, 4096, 1, T, 1, 128, chunk, flags, 0, ws, ws_bytes, None)
+
+    assert state(T=100) == SHP and state(T=0, flags=_lib.QH_GDN_RAGGED) == SHP
+    assert state(T=100, flags=_lib.QH_GDN_RAGGED, chunk=128) == SHP
+    assert state(s_in=8192) == INV and state(ws=4104, ws_bytes=1 << 20) == INV
+    assert state(flags=_lib.QH_GDN_W_DECAY) == UNS
+    for query in (L.qh_gdn_chunk_state_workspace, L.qh_gdn_prefill_workspace):
+        assert query(0, 64, 1, 0) == 0 and query(1, 0, 1, 0) == 0 and query(1, 64, 0, 0) == 0
+        assert query(1 << 12, 1 << 12, 2, 0) == 0  # batch * tokens * heads over 2^24
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "libqhtp.so")
     monkeypatch.setattr(_lib, "_lib", None)

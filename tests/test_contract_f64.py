@@ -1,8 +1,9 @@
-"""The one-launch contract chain computes the dividing contracts in float64 without a division
-(a reciprocal product; only quotients near a half-integer take the exact integer remainder that
-picks the rounding neighbour).  This
+"""The contract kernels (one matmul, and the one-launch chain) compute the dividing contracts in
+float64 without a division (a reciprocal product; only quotients near a half-integer take the exact
+integer remainder that picks the rounding neighbour).  This
 restates that algorithm with numpy and checks it against the oracle's contracts over random
-accumulators, exact ties, near-ties and the extremes of the divisor range (CPU only).  numpy has
+accumulators, exact ties, near-ties and the extremes of the divisor range, up to the 2^50 that the
+kernels' proof assumes and past the 2^47 that K = 65536 of 16-bit operands reaches (CPU only).  numpy has
 no fused multiply-add: the reciprocal product and the sum round separately here, which the error
 bound of the kernel's comment covers as well."""
 
@@ -41,18 +42,22 @@ def chain_round_div(D, d, zp, qmax):
 
 
 def accumulators(d, rng):
-    """Random |D| < 2^40, exact ties (D = (2n + 1) d / 2), their integer neighbours, and values
-    that divide to just inside and outside the output range."""
-    base = rng.integers(-(1 << 40), 1 << 40, size=4000, dtype=np.int64)
+    """Random |D| < 2^40 and < 2^50, exact ties (D = (2n + 1) d / 2) up to 2^50, their integer
+    neighbours, and values that divide to just inside and outside the output range."""
+    base = np.concatenate([rng.integers(-(1 << b), 1 << b, size=4000, dtype=np.int64) for b in (40, 47, 50)])
     mid = rng.integers(-(1 << 20), 1 << 20, size=4000, dtype=np.int64) * d + rng.integers(-d, d + 1, size=4000)
     ties = []
     if d % 2 == 0:
         n = rng.integers(-(1 << 17), 1 << 17, size=2000, dtype=np.int64)
         t = (2 * n + 1) * (d // 2)
+        n = rng.integers(-((1 << 50) // d) + 1, (1 << 50) // d - 1, size=2000, dtype=np.int64)
+        t = np.concatenate([t, (2 * n + 1) * (d // 2)])
         ties = [t, t - 1, t + 1]
     edge = np.arange(-3 * d, 3 * d + 1, max(1, d // 7), dtype=np.int64)
     edge2 = edge + 65535 * d
-    return np.concatenate([base, mid, edge, edge2] + ties)
+    ends = np.arange(-8, 1, dtype=np.int64) + (1 << 50) - 1
+    D = np.concatenate([base, mid, edge, edge2, ends, -ends] + ties)
+    return D[np.abs(D) < 1 << 50]
 
 
 @pytest.mark.parametrize("d", [1, 2, 7, 127, 256, 1000, 32767, 65536, (1 << 30) - 1, 1 << 30])

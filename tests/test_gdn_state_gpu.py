@@ -202,6 +202,42 @@ def test_chunk_state_rejects_bad_arguments(gpu):
     assert L.qh_gdn_chunk_state(*args(T, 64, 128, s.data_ptr())) == _lib.QH_STATUS_INVALID_ARGUMENT  # alias
 
 
+def test_prefill_of_few_sequences_has_no_workspace(gpu):
+    """qh_gdn_prefill refuses the sequences that stages A and B serve better."""
+    import torch
+
+    from qcom_htp_amd import _lib
+
+    L, x = _lib.lib(), torch.zeros(1 << 16, device=gpu)
+    assert L.qh_gdn_prefill_workspace(1, 64, 64, 0) == 0 and L.qh_gdn_prefill_workspace(1, 64, 65, 0) > 0
+    p = x.data_ptr()
+    assert L.qh_gdn_prefill(p, p, p, p, p, 0, p, p, 1, 64, 1, 128, 0, 0, p, x.numel() * 4, 0) == _lib.QH_STATUS_SHAPE_UNSUPPORTED
+
+
+def test_chunk_state_with_a_short_workspace_leaves_it_alone(gpu):
+    """A workspace one byte short is not written, and the results are those of a sufficient one."""
+    import torch
+
+    from qcom_htp_amd import _lib
+    from qcom_htp_amd.gdn import gdn_chunk_state, gdn_chunk_uw
+
+    B, T, H = 1, 256, 3
+    q, k, v, bt, g = (to_dev(x, gpu) for x in seq_inputs(B, T, H, seed=91))
+    w, u = gdn_chunk_uw(k, v, g, bt, 64, decay_w=True, out_dtype=torch.float32)
+    want, s_want = gdn_chunk_state(q, k, g, w, u, out_dtype=torch.float32)
+    L = _lib.lib()
+    need = L.qh_gdn_chunk_state_workspace(B, T, H, 0)
+    assert need > 0
+    for size in (need - 1, 0):
+        ws = torch.full((need,), 0x5A, dtype=torch.uint8, device=gpu)
+        o, s = torch.empty_like(want), torch.empty_like(s_want)
+        st = L.qh_gdn_chunk_state_ws(q.data_ptr(), k.data_ptr(), g.data_ptr(), w.data_ptr(), u.data_ptr(), 0, s.data_ptr(),
+                                     o.data_ptr(), B, T, H, 128, 64, _lib.QH_GDN_OUT_F32 | _lib.QH_GDN_WU_F32, 0, ws.data_ptr(),
+                                     size, torch.cuda.current_stream().cuda_stream)
+        assert st == _lib.QH_STATUS_OK
+        assert torch.equal(o, want) and torch.equal(s, s_want) and bool((ws == 0x5A).all())
+
+
 def test_prefill_full_config5_every_sequence(gpu):
     """Config 5 at full size (B=8, T=4096, H=32, D=128; 64 chunks per sequence): the GPU prefill
     against the float64 oracle on all 256 (batch, head) sequences, o and the final state, one

@@ -14,8 +14,33 @@ from qcom_htp_amd import cases as C
 pytestmark = pytest.mark.gpu
 
 # (M, K, N): one output block; row and column remainders with a K tail; 8 K groups with a tail; a
-# row past a tile at many columns; a grid of wide tiles
-SHAPES = [(1, 32, 32), (33, 160, 96), (64, 1056, 1088), (65, 2048, 352), (700, 288, 2080)]
+# row past a tile at many columns; a grid of wide tiles, for every width but 8 x 8 bits and for those
+SHAPES = [(1, 32, 32), (33, 160, 96), (64, 1056, 1088), (65, 2048, 352), (700, 288, 2080), (700, 288, 4160)]
+# ... requantised: the last four are the two K groups of the widest tiles and the GEMM just past them,
+# for 16-bit and for 8-bit activations
+REQUANT_SHAPES = [(17, 32, 32), (33, 160, 96), (65, 1184, 1088), (130, 4096, 480), (700, 288, 2080),
+                  (330, 288, 2080), (500, 288, 2080), (700, 288, 4160), (1100, 288, 4160)]
+
+
+def k_groups(cus, m, k, n, ab, cols, requant):
+    """K groups of the kernel's workgroups (qmm_tile.hip, pick_split), cols channels per wave; 0: the
+    GEMM's product (tile_pays)."""
+    rows = 32 if ab == 16 else 64
+    tiles = lambda ks: -(-m // rows) * -(-n // (cols * 8 // ks))  # noqa: E731
+    if requant and tiles(2) > cus:
+        return 0
+    return 8 if -(-k // 128) >= 8 and tiles(8) <= cus else 4 if tiles(4) <= cus else 2
+
+
+def test_shapes_reach_every_number_of_k_groups(gpu):
+    import torch
+
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    for ab in (8, 16):
+        for wb in (8, 16):
+            assert {k_groups(cus, *s, ab, 32 if wb == 16 else 64, False) for s in SHAPES} == {2, 4, 8}, (ab, wb)
+        groups = [k_groups(cus, *s, ab, 32 if ab == 16 else 64, True) for s in REQUANT_SHAPES]
+        assert set(groups) == {0, 2, 4, 8}, (ab, groups)
 
 
 def unaligned(gpu, m, n, dtype):
@@ -189,8 +214,7 @@ def test_per_group_outputs_far_below_a_group_of_large_scale(gpu, ab, span, zp, o
 
 
 @pytest.mark.parametrize("tie", [False, True], ids=["random", "ties"])
-@pytest.mark.parametrize("mkn", [(17, 32, 32), (33, 160, 96), (65, 1184, 1088), (130, 4096, 480), (700, 288, 2080)],
-                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("mkn", REQUANT_SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("fam", C.GATED_FAMILIES)
 def test_requantised_few_tiles(gpu, fam, mkn, tie):
     """Per-channel and LPBQ weights on the automatic path; with ties, power-of-two scales put odd
