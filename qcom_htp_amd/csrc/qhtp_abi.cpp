@@ -253,6 +253,17 @@ qh_status qh_gdn_solve_u16(const uint16_t *A_dev, uint16_t *T_dev, uint32_t head
 }
 
 
+namespace {
+
+// batch * tokens * heads <= 2^24 rows (32-bit element offsets); the product itself may pass 2^64.
+bool gdn_rows_fit(uint32_t batch, uint32_t tokens, uint32_t heads) {
+  constexpr uint64_t kMost = (1ull << 31) / 128;
+  const uint64_t bt = static_cast<uint64_t>(batch) * tokens;
+  return bt <= kMost && bt * heads <= kMost;
+}
+
+}  // namespace
+
 qh_status qh_gdn_chunk_uw_ex(const uint16_t *k_dev, const uint16_t *v_dev, const float *g_dev, const float *beta_dev,
                              void *w_dev, void *u_dev, uint32_t batch, uint32_t tokens, uint32_t heads,
                              uint32_t head_dim, uint32_t chunk, uint32_t flags, uint32_t max_workgroups,
@@ -267,7 +278,7 @@ qh_status qh_gdn_chunk_uw_ex(const uint16_t *k_dev, const uint16_t *v_dev, const
   if (batch == 0 || heads == 0 || tokens == 0 || (!ragged && tokens % chunk))
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_uw: batch=%u tokens=%u heads=%u (tokens %% chunk == 0)",
                 batch, tokens, heads);
-  if (static_cast<uint64_t>(batch) * tokens * heads > (1ull << 31) / 128)
+  if (!gdn_rows_fit(batch, tokens, heads))
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_uw: batch * tokens * heads too large");
   if (flags & ~static_cast<uint32_t>(QH_GDN_W_DECAY | QH_GDN_OUT_F32 | QH_GDN_RAGGED))
     return fail(QH_STATUS_UNSUPPORTED, "qh_gdn_chunk_uw: unknown flags 0x%x", flags);
@@ -291,7 +302,7 @@ qh_status qh_gdn_chunk_uw(const uint16_t *k_dev, const uint16_t *v_dev, const fl
 }
 
 size_t qh_gdn_chunk_state_workspace(uint32_t batch, uint32_t tokens, uint32_t heads, uint32_t precision) {
-  if (batch == 0 || heads == 0 || tokens == 0 || static_cast<uint64_t>(batch) * tokens * heads > (1ull << 31) / 128) return 0;
+  if (batch == 0 || heads == 0 || tokens == 0 || !gdn_rows_fit(batch, tokens, heads)) return 0;
   return gdn_chunk_state_workspace(static_cast<int>(batch), static_cast<int>(tokens), static_cast<int>(heads),
                                    static_cast<int>(precision));
 }
@@ -315,8 +326,7 @@ qh_status qh_gdn_chunk_state_ws(const uint16_t *q_dev, const uint16_t *k_dev, co
   if (batch == 0 || heads == 0 || tokens == 0 || (!(flags & QH_GDN_RAGGED) && tokens % 64))
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_state: batch=%u tokens=%u heads=%u (tokens %% 64 == 0)",
                 batch, tokens, heads);
-  if (static_cast<uint64_t>(batch) * tokens * heads > (1ull << 31) / 128 ||
-      static_cast<uint64_t>(batch) * heads > (1u << 24))
+  if (!gdn_rows_fit(batch, tokens, heads))
     return fail(QH_STATUS_SHAPE_UNSUPPORTED, "qh_gdn_chunk_state: batch * tokens * heads too large");
   if (flags & ~static_cast<uint32_t>(QH_GDN_OUT_F32 | QH_GDN_WU_F32 | QH_GDN_RAGGED))
     return fail(QH_STATUS_UNSUPPORTED, "qh_gdn_chunk_state: unknown flags 0x%x", flags);
@@ -335,7 +345,7 @@ qh_status qh_gdn_chunk_state_ws(const uint16_t *q_dev, const uint16_t *k_dev, co
 }
 
 size_t qh_gdn_prefill_workspace(uint32_t batch, uint32_t tokens, uint32_t heads, uint32_t precision) {
-  if (batch == 0 || heads == 0 || tokens == 0 || static_cast<uint64_t>(batch) * tokens * heads > (1ull << 31) / 128) return 0;
+  if (batch == 0 || heads == 0 || tokens == 0 || !gdn_rows_fit(batch, tokens, heads)) return 0;
   return gdn_prefill_workspace(static_cast<int>(batch), static_cast<int>(tokens), static_cast<int>(heads),
                                static_cast<int>(precision));
 }

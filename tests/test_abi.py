@@ -148,6 +148,19 @@ def test_gdn_chunk_rejects_bad_ragged_and_workspace_arguments(qhtp_lib):
         assert query(1 << 12, 1 << 12, 2, 0) == 0  # batch * tokens * heads over 2^24
 
 
+def test_gdn_sizes_whose_product_wraps_are_refused(qhtp_lib):
+    """batch * tokens * heads of these is 2^64 + 10 and 2^64."""
+    L, SHP = qhtp_lib, _lib.QH_STATUS_SHAPE_UNSUPPORTED
+    for B, T, H in ((21398, 289529, 2977518503), (289529, 2977518503, 21398), (1 << 24, 1 << 16, 1 << 24)):
+        for precision in (0, 1):
+            assert L.qh_gdn_prefill_workspace(B, T, H, precision) == 0
+            assert L.qh_gdn_chunk_state_workspace(B, T, H, precision) == 0
+        p = 4096
+        assert L.qh_gdn_prefill(p, p, p, p, p, 0, 8192, p, B, T, H, 128, 0, 0, p, 1 << 62, None) == SHP
+        assert L.qh_gdn_chunk_uw(p, p, p, p, p, p, B, T, H, 128, 64, _lib.QH_GDN_RAGGED, None) == SHP
+        assert L.qh_gdn_chunk_state(p, p, p, p, p, 0, 8192, p, B, T, H, 128, 64, _lib.QH_GDN_RAGGED, 0, None) == SHP
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "libqhtp.so")
     monkeypatch.setattr(_lib, "_lib", None)
