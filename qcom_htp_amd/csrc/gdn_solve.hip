@@ -32,6 +32,8 @@
 // The u16 variant applies the GdnSolve op's code contract on load / store
 // (A = (code - zpA) * sA; T_code = clip(rint(T / sT) + zpT, 0, 65535)).
 
+#include <algorithm>
+
 #include "bf16_split.h"
 #include "qmm_internal.h"
 
@@ -385,10 +387,8 @@ GdnArgs make_args(const void *A, void *T, int heads, int C, int zpA, int zpT, fl
 }
 
 template <bool U16, bool SPLIT>
-qh_status launch_fs(const GdnArgs &g, int heads, hipStream_t stream) {
-  const long long blocks = static_cast<long long>((heads + 7) / 8) * 8 * g.groups;
-  if (blocks > 0x7FFFFFFFLL) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "gdn: %d heads exceed one launch", heads);
-  const dim3 grid(static_cast<unsigned>(blocks));
+qh_status launch_part(const GdnArgs &g, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>((g.heads + 7) / 8 * 8 * g.groups));
   const int nb = g.C / 16;
   if (nb <= 1)
     hipLaunchKernelGGL((gdn_fs_kernel<U16, SPLIT, 1>), grid, dim3(fs_threads<1>()), 0, stream, g);
@@ -405,17 +405,31 @@ qh_status launch_fs(const GdnArgs &g, int heads, hipStream_t stream) {
   return QH_STATUS_OK;
 }
 
+template <bool U16, bool SPLIT>
+qh_status launch_fs(const GdnArgs &whole, hipStream_t stream) {
+  const size_t head = static_cast<size_t>(whole.C) * whole.C * (U16 ? 2 : 4);
+  for (int h0 = 0; h0 < whole.heads; h0 += kSolveHeads) {
+    GdnArgs g = whole;
+    g.A = static_cast<const uint8_t *>(whole.A) + h0 * head;
+    g.T = static_cast<uint8_t *>(whole.T) + h0 * head;
+    g.heads = std::min(kSolveHeads, whole.heads - h0);
+    const qh_status st = launch_part<U16, SPLIT>(g, stream);
+    if (st != QH_STATUS_OK) return st;
+  }
+  return QH_STATUS_OK;
+}
+
 }  // namespace
 
 qh_status launch_gdn_solve_f32(const float *A, float *T, int heads, int C, int precision, hipStream_t stream) {
   const GdnArgs g = make_args(A, T, heads, C, 0, 0, 1.0f, 1.0f);
-  return precision == QH_GDN_BF16 ? launch_fs<false, false>(g, heads, stream) : launch_fs<false, true>(g, heads, stream);
+  return precision == QH_GDN_BF16 ? launch_fs<false, false>(g, stream) : launch_fs<false, true>(g, stream);
 }
 
 qh_status launch_gdn_solve_u16(const uint16_t *A, uint16_t *T, int heads, int C, int zpA, int zpT, float sA, float sT,
                                int precision, hipStream_t stream) {
   const GdnArgs g = make_args(A, T, heads, C, zpA, zpT, sA, sT);
-  return precision == QH_GDN_BF16 ? launch_fs<true, false>(g, heads, stream) : launch_fs<true, true>(g, heads, stream);
+  return precision == QH_GDN_BF16 ? launch_fs<true, false>(g, stream) : launch_fs<true, true>(g, stream);
 }
 
 }  // namespace qh

@@ -16,6 +16,8 @@
 
 #pragma clang fp contract(off)
 
+#include <algorithm>
+
 #include "qmm_internal.h"
 
 namespace qh {
@@ -110,10 +112,14 @@ __global__ __launch_bounds__(kOpThreads) void gdn_op_model_kernel(OpArgs g) {
 qh_status launch_gdn_solve_op_model(const uint16_t *A, uint16_t *T, int heads, int C, int zpA, int zpT, float sA,
                                     float sT, hipStream_t stream) {
   if (C > kOpMaxC) return fail(QH_STATUS_SHAPE_UNSUPPORTED, "gdn op model: C=%d (the op supports C <= 64)", C);
-  OpArgs g{A, T, C, heads, zpA, zpT, sA, sT};
-  hipLaunchKernelGGL(gdn_op_model_kernel, dim3(heads), dim3(kOpThreads), 0, stream, g);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return hip_fail(err, "gdn_op_model_kernel launch");
+  for (int h0 = 0; h0 < heads; h0 += kSolveHeads) {
+    const size_t at = static_cast<size_t>(h0) * C * C;
+    const int n = std::min(kSolveHeads, heads - h0);
+    OpArgs g{A + at, T + at, C, n, zpA, zpT, sA, sT};
+    hipLaunchKernelGGL(gdn_op_model_kernel, dim3(n), dim3(kOpThreads), 0, stream, g);
+    hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return hip_fail(err, "gdn_op_model_kernel launch");
+  }
   return QH_STATUS_OK;
 }
 

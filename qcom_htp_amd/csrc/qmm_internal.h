@@ -215,6 +215,9 @@ qh_status launch_qmm_tile(const qh_qmm_prepared *p, int m, const void *act, void
 bool chain_fusable(const qh_qmm_prepared *p);
 qh_status launch_qmm_chain(const qh_qmm_prepared *p, int m, int chain, const void *act, void *out, int contract,
                            int divisor, hipStream_t stream);
+// Most heads of one launch of the GDN solves (at most two workgroups of 512 threads each): a launch counts
+// its threads in 32 bits, and a larger grid is cut short without an error.
+constexpr int kSolveHeads = 1 << 21;
 qh_status launch_gdn_solve_f32(const float *A, float *T, int heads, int C, int precision, hipStream_t stream);
 qh_status launch_gdn_solve_u16(const uint16_t *A, uint16_t *T, int heads, int C, int zpA, int zpT, float sA,
                                float sT, int precision, hipStream_t stream);

@@ -248,3 +248,29 @@ def test_every_block_count_bound(gpu, C, heads):
     ref = og.inverse_fp64((codes.astype(np.int64) - 32768) * float(sA))
     assert np.abs(np.clip(Td - ref, -1, 1)).max() <= 0.51 * float(sT) + 1e-4 * np.abs(ref).max()
     assert (got[np.broadcast_to(np.triu(np.ones((C, C), bool), 1), got.shape)] == 32768).all()
+
+
+@pytest.mark.parametrize("heads", [(1 << 21) + 9, 1 << 24])
+@pytest.mark.parametrize("kind", ["f32", "u16", "op_model"])
+def test_more_heads_than_one_launch(gpu, kind, heads):
+    """The heads are shared out over launches of 2^21 (a launch's threads are counted in 32 bits; 2^24 heads
+    of 256 threads are 2^32).  The operands repeat every 24 heads, and so must T."""
+    import torch
+
+    from qcom_htp_amd.gdn import FP32, OP_MODEL, GdnSolve, gdn_solve
+
+    C, per = 16, 24
+    k, beta, gc = og.config4_inputs(heads=per, C=C, seed=3)
+    A = torch.from_numpy(og.build_A(k, beta, gc).astype(np.float32)).to(gpu)
+    zp, sA, sT = 32768, float(A.abs().max() / 32767.0), 2.0 / 32767.0
+    if kind == "f32":
+        solve = gdn_solve
+    else:
+        A = (torch.round(A / sA) + zp).clamp(0, 65535).to(torch.int32).to(torch.uint16)
+        solve = lambda a: GdnSolve(a, zp, sA, zp, sT, precision=OP_MODEL if kind == "op_model" else FP32)  # noqa: E731
+    bits = lambda t: t.view(torch.int32 if kind == "f32" else torch.int16)  # noqa: E731
+    want = bits(solve(A)).view(per, -1)
+    many = bits(A).repeat(heads // per + 1, 1, 1)[:heads].contiguous().view(A.dtype)
+    got = bits(solve(many)).view(heads, -1)
+    whole = heads // per * per
+    assert bool((got[:whole].view(-1, per, C * C) == want).all()) and bool((got[whole:] == want[:heads - whole]).all())
