@@ -20,7 +20,7 @@
 // head of up to 4 blocks is one wave per strip with the LDS and registers of that size, so that a
 // compute unit holds several heads (up to 10 of C = 64) and their latencies overlap, where the
 // 16-block workgroup (512 threads, 157 KB of LDS) has the unit to itself.  With the 16-block kernel
-// for every C against this: u16 C = 64 x 2048 heads 43.3 -> 15.1 us, C = 16 x 8192 101 -> 8.4, C = 128 x
+// for every C against this: u16 C = 64 x 2048 heads 41.7 -> 13.6 us, C = 16 x 8192 101 -> 8.4, C = 128 x
 // 1024 35.1 -> 22.5; 8 heads of C = 64 6.2 -> 5.3.  The G workgroups of a head get block indexes of one residue mod 8,
 // which places them on one XCD and one L2.
 // The products run on v_mfma_f32_16x16x32_bf16: a 32-deep k step takes rows 4q .. 4q+3 of two

@@ -177,9 +177,10 @@ def gdn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tens
     of a last partial chunk of 64 count as zeros, which leaves o and S unchanged.  Few sequences
     (B * H <= 64 on 256 compute units) run stages A (float32 W, U for ``FP32``, bf16 for ``BF16``)
     and B; many take the recurrence from T = (I - A)^-1, without W and U.  The two round
-    differently: a sequence's bits may differ between a call of few and one of many sequences,
-    by less than stage A's bf16 products are from float64 (3.4e-4 of o in ``FP32``; o from T is
-    within 5.1e-6).  Within one of the two they do not depend on the other sequences."""
+    differently, so a sequence's bits differ between a call of few and one of many sequences: o
+    is 3.4e-4 from float64 with stage A and 5.1e-6 from T in ``FP32``, 2.9e-3 and 2.4e-3 in
+    ``BF16``, before its rounding to ``out_dtype``.  Within one of the two they do not depend on
+    the other sequences."""
     B, T, H, D = q.shape
     _same_device(q.device, k=k, v=v, g=g, beta=beta, initial_state=initial_state)
     ragged = _lib.QH_GDN_RAGGED if T % STATE_CHUNK else 0

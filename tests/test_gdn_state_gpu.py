@@ -8,8 +8,8 @@ Bounds:
   stage B alone, W and U exact (float64 -> float32):
     QH_GDN_FP32  <= 1e-4   (hi/lo split products; the solve's fp32 bound)
     QH_GDN_BF16  <= 1.05e-2 (the bf16 bound of tests/qnn_kernel_e2e/correctness/test_gdn_solve_e2e.sh:18)
-  prefill (stage A + B): stage A is bf16-MFMA (qh_gdn_chunk_uw, bound 1.05e-2), so the whole
-  path is held to 1.05e-2.
+  prefill of few sequences (stage A + B): stage A is bf16-MFMA (qh_gdn_chunk_uw, bound 1.05e-2), so
+  the whole path is held to 1.05e-2; of many (from T, no bf16 product in FP32): stage B's bounds.
 """
 
 import numpy as np
